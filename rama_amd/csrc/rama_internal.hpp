@@ -186,6 +186,32 @@ DCoo mp_reparametrized(Ctx& ctx, MPState& S);
 double dual_solver(Ctx& ctx, DCoo& A, int max_cycle_length, int num_iter, float tri_memory_factor, int num_outer,
                    float tol_ratio, bool want_lb = true);
 
+// ---- small.hip
+// Matching-contraction rounds of a small graph, run by one workgroup that
+// holds it in LDS.
+constexpr int kSmallMaxEdges = 4096;
+constexpr int kSmallMaxNodes = 4096;
+constexpr int kSmallBitWords = 20480;  // 32-bit words of the attractive adjacency's bit matrix
+enum SmallReason : int {
+    kSmallMore = 0,    // the launch's rounds are used up
+    kSmallCycles = 1,  // the next round's cycle search finds something: its dual pass is due
+    kSmallDone = 2,    // nothing (left) to contract
+    kSmallBad = 3,     // a negative self-loop was contracted
+    kSmallForest = 4,  // the next round contracts by the spanning forest
+};
+struct SmallState {
+    int reason;
+    int iter;  // the driver's round number after the rounds done
+    int nnz, rows, cols, max_node;
+};
+// Whether A (the result of a contraction: no repeated pair, no self-loop)
+// can go to small_rounds under these options.
+bool small_rounds_fit(const DCoo& A, const Options& o);
+// Runs rounds from number `iter` on while matching picks the contractions and
+// no round's cycle search finds anything; A becomes the graph they leave and
+// labels (num_labels of them) are mapped along.
+SmallState small_rounds(Ctx& ctx, DCoo& A, const Options& o, int iter, int* labels, i64 num_labels);
+
 // ---- forest.hip
 void connected_components(Ctx& ctx, const int* off, const int* adj, int n, int* labels);
 // Forest edge indices (into the given edge list) of the maximum spanning

@@ -85,10 +85,34 @@ void solve_rounds(Ctx& ctx, DCoo& A, SolveResult& out, const Options& o, int sta
     if (start_iter > 0) ctx.last_cycles_empty = false;  // resumed on another context: no hint
     const auto t0 = out.t0;  // the time budget counts from the start of the solve
     const i64 N = out.num_labels;
+    const bool duals = o.max_cycle_length_primal >= 3 && o.num_dual_itr_primal != 0;
+    const bool observed = o.verbose || o.dump_timeline || o.max_time_sec >= 0;
     for (int iter = start_iter; A.nnz > 0; ++iter) {
         const auto r0 = std::chrono::steady_clock::now();
         const int64_t l0 = launch_count(), s0 = ctx.syncs;
         const i64 e0 = A.nnz;
+        // a contracted graph that fits one workgroup: its rounds run in one
+        // launch up to the next dual pass or the forest.  Not where a round
+        // is observed (printing, snapshots, the time budget), nor while the
+        // rounds' cycle searches still find something.
+        if (use_mm && iter > 0 && (!duals || ctx.last_cycles_empty) && !observed && small_rounds_fit(A, o)) {
+            st.begin(ctx);
+            const SmallState ss = small_rounds(ctx, A, o, iter, out.labels.get(), N);
+            st.end(ctx, "small_rounds");
+            if (ss.reason == kSmallBad) throw Error(RAMA_ERR_BAD_CONTRACTION, "Found bad contractions");
+            if (st.on)
+                std::fprintf(stderr, "rounds %d..%d: %lld edges, small, reason %d, %.3f ms\n", iter, ss.iter - 1,
+                             (long long)e0, ss.reason,
+                             std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - r0).count());
+            if (ss.iter > iter) out.iterations = ss.iter;
+            if (ss.reason == kSmallDone) break;
+            iter = ss.iter;
+            if (ss.reason == kSmallForest) use_mm = false;
+            if (ss.reason == kSmallMore) {
+                --iter;  // the loop's increment
+                continue;
+            }
+        }
         st.begin(ctx);
         if (iter > 0)
             dual_solver(ctx, A, o.max_cycle_length_primal, o.num_dual_itr_primal, 1.0f, 1, 1e-4f, false);

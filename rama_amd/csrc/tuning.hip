@@ -39,6 +39,7 @@ const Spec& spec(int k) {
         {"match_blocks", 64, 65536, {{-1, 1024}}},
         {"mp_fused_max_blocks", 0, 65536, {{-1, 256}}},
         {"cycle_chunk_pct", 100, 1000, {{-1, 125}}},
+        {"small_rounds", 0, 1, {{kSmallMaxEdges, 1}, {-1, 0}}},
     };
     return specs[k];
 }

@@ -39,6 +39,9 @@ enum Knob : int {
     // size = expansions; chunked 4/5-cycle counts size the next chunk as this
     // percentage of the blocks the rate so far expects to reach the budget
     CycleChunkPct,
+    // size = edges; 1 = matching rounds of a small graph run in one launch
+    // (small.hip; at most kSmallMaxEdges edges), 0 = stage by stage
+    SmallRounds,
     KnobCount
 };
 

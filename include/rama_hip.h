@@ -312,7 +312,8 @@ void rama_profile_only(const char* name);
  * mp_fused_max_blocks (message-passing edges -> largest edge grid that sums
  * its own lower bound), cycle_chunk_pct (expansions -> growth of the chunked
  * 4/5-cycle counts), small_rounds (edges -> 1 matching rounds of a small
- * graph in one launch, 0 stage by stage).  None of them changes a result.  The table is read on
+ * graph in one launch, 0 stage by stage), mid_rounds (edges -> 1 matching
+ * rounds queued without read-backs).  None of them changes a result.  The table is read on
  * first use from RAMA_TUNING_TABLE, else tuning/gfx950.table beside the
  * library; "none" or no file keeps the built-in defaults.
  * ------------------------------------------------------------------------ */

@@ -212,6 +212,28 @@ bool small_rounds_fit(const DCoo& A, const Options& o);
 // labels (num_labels of them) are mapped along.
 SmallState small_rounds(Ctx& ctx, DCoo& A, const Options& o, int iter, int* labels, i64 num_labels);
 
+// ---- mid.hip
+// Matching-contraction rounds queued without a read-back, for graphs of up
+// to 2^18 edges whose symmetric CSR the contraction left (A.sym).
+constexpr int kMidMaxEdges = 1 << 18;
+constexpr int kMidMaxNodes = 1 << 18;
+enum MidReason : int {  // besides SmallReason's; 0: rounds still go on
+    kMidMatching = 5,   // this round's matching takes more rounds than are queued
+    kMidSkew = 6,       // a row bucket of the contraction does not fit in LDS
+    kMidSmall = 7,      // small enough for small_rounds
+};
+struct MidState {
+    int stop;
+    int iter;  // the driver's round number after the rounds done
+    int nf, n, rows, cols, max_node;
+    int found, any, matched, kb;
+    int rounds;  // done since entry
+    float thr, minw;
+};
+bool mid_rounds_fit(const DCoo& A, const Options& o);
+// As small_rounds; `first` rounds are queued before the first host wait.
+MidState mid_rounds(Ctx& ctx, DCoo& A, const Options& o, int iter, int first, int* labels, i64 num_labels);
+
 // ---- forest.hip
 void connected_components(Ctx& ctx, const int* off, const int* adj, int n, int* labels);
 // Forest edge indices (into the given edge list) of the maximum spanning

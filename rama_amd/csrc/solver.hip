@@ -86,29 +86,45 @@ void solve_rounds(Ctx& ctx, DCoo& A, SolveResult& out, const Options& o, int sta
     const auto t0 = out.t0;  // the time budget counts from the start of the solve
     const i64 N = out.num_labels;
     const bool duals = o.max_cycle_length_primal >= 3 && o.num_dual_itr_primal != 0;
+    i64 mid_max = kMidMaxEdges;  // largest graph given to mid_rounds
+    int mid_first = 2;           // rounds it queues before its first wait
     const bool observed = o.verbose || o.dump_timeline || o.max_time_sec >= 0;
     for (int iter = start_iter; A.nnz > 0; ++iter) {
         const auto r0 = std::chrono::steady_clock::now();
         const int64_t l0 = launch_count(), s0 = ctx.syncs;
         const i64 e0 = A.nnz;
-        // a contracted graph that fits one workgroup: its rounds run in one
-        // launch up to the next dual pass or the forest.  Not where a round
+        // A contracted graph of up to a few thousand edges: its rounds run in
+        // one launch; of up to 2^18, they are queued without read-backs.
+        // Both stop at the next dual pass or the forest.  Not where a round
         // is observed (printing, snapshots, the time budget), nor while the
         // rounds' cycle searches still find something.
-        if (use_mm && iter > 0 && (!duals || ctx.last_cycles_empty) && !observed && small_rounds_fit(A, o)) {
+        if (use_mm && iter > 0 && (!duals || ctx.last_cycles_empty) && !observed) {
+            const bool small = small_rounds_fit(A, o), mid = !small && A.nnz <= mid_max && mid_rounds_fit(A, o);
+            int reason = kSmallCycles, next = iter;
             st.begin(ctx);
-            const SmallState ss = small_rounds(ctx, A, o, iter, out.labels.get(), N);
-            st.end(ctx, "small_rounds");
-            if (ss.reason == kSmallBad) throw Error(RAMA_ERR_BAD_CONTRACTION, "Found bad contractions");
-            if (st.on)
-                std::fprintf(stderr, "rounds %d..%d: %lld edges, small, reason %d, %.3f ms\n", iter, ss.iter - 1,
-                             (long long)e0, ss.reason,
+            if (small) {
+                const SmallState ss = small_rounds(ctx, A, o, iter, out.labels.get(), N);
+                reason = ss.reason;
+                next = ss.iter;
+            } else if (mid) {
+                const MidState ms = mid_rounds(ctx, A, o, iter, mid_first, out.labels.get(), N);
+                reason = ms.stop;
+                next = ms.iter;
+                mid_first = next > iter ? 4 : 1;
+                // a row too long for its bucket: wait until the graph is half as large
+                if (reason == kMidSkew) mid_max = ms.nf / 2;
+            }
+            st.end(ctx, small ? "small_rounds" : "mid_rounds");
+            if (st.on && (small || mid))
+                std::fprintf(stderr, "rounds %d..%d: %lld edges, %s, reason %d, %.3f ms\n", iter, next - 1,
+                             (long long)e0, small ? "small" : "mid", reason,
                              std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - r0).count());
-            if (ss.iter > iter) out.iterations = ss.iter;
-            if (ss.reason == kSmallDone) break;
-            iter = ss.iter;
-            if (ss.reason == kSmallForest) use_mm = false;
-            if (ss.reason == kSmallMore) {
+            if (reason == kSmallBad) throw Error(RAMA_ERR_BAD_CONTRACTION, "Found bad contractions");
+            if (next > iter) out.iterations = next;
+            if (reason == kSmallDone) break;
+            iter = next;
+            if (reason == kSmallForest) use_mm = false;
+            if (reason == kSmallMore || reason == kMidSmall) {
                 --iter;  // the loop's increment
                 continue;
             }

@@ -40,6 +40,7 @@ const Spec& spec(int k) {
         {"mp_fused_max_blocks", 0, 65536, {{-1, 256}}},
         {"cycle_chunk_pct", 100, 1000, {{-1, 125}}},
         {"small_rounds", 0, 1, {{kSmallMaxEdges, 1}, {-1, 0}}},
+        {"mid_rounds", 0, 1, {{kMidMaxEdges, 1}, {-1, 0}}},
     };
     return specs[k];
 }

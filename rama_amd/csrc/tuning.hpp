@@ -42,6 +42,9 @@ enum Knob : int {
     // size = edges; 1 = matching rounds of a small graph run in one launch
     // (small.hip; at most kSmallMaxEdges edges), 0 = stage by stage
     SmallRounds,
+    // size = edges; 1 = matching rounds queued without read-backs (mid.hip; at
+    // most kMidMaxEdges edges), 0 = stage by stage
+    MidRounds,
     KnobCount
 };
 

@@ -8,8 +8,8 @@
 // (tuning table): three launches per pass (per-tile histograms, their scan,
 // the scatter), or one histogram launch for every pass and then one
 // "onesweep" launch per pass with decoupled look-back for each digit's
-// global offset, or a top-digit onesweep pass followed by one block per
-// bucket.  Arrays of at most 8192 pairs are sorted by one block.
+// global offset, or a top-digit pass (two launches) followed by one block per
+// bucket.  Short arrays are sorted by one block.
 #include <cstdlib>
 
 #include "prims.cuh"
@@ -199,6 +199,153 @@ __global__ __launch_bounds__(NT) void k_radix_scatter(const K* __restrict__ kin,
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < (kRsTile + kScThreads - 1) / kScThreads; ++q) {
+        const int p = tid + q * kScThreads;
+        if (p < nvalid) vout[outp[q]] = sv[p];
+    }
+}
+
+// The top-digit pass of the bucket path: k_radix_scatter without an offset
+// scan before it.  The tiles' counts lie tile-major (hist[tile * 256 + d]);
+// every block adds up the columns itself, NT / 256 threads per digit with 16
+// loads in flight each, and block 0 leaves the bucket sizes in `sizes`.  Up to
+// a few hundred tiles this is cheaper than an order between blocks.  Whole
+// sorts of 35-bit u64 keys, with the buckets' items counted (tile_items),
+// against a onesweep pass behind a histogram that one block combines: 16k
+// pairs 39.5 -> 23.0 us, 260k 52.4 -> 28.6, 1M 79.8 -> 48.3; bound by the three
+// launches' load chains up to about 200k pairs, by the LDS passes above.
+template <class K, int NT>
+__global__ __launch_bounds__(NT) void k_split_hist(const K* __restrict__ keys, i64 n, int shift, int* hist) {
+    RAMA_SC_SHAPE(NT)
+    __shared__ int h[256];
+    if (threadIdx.x < 256) h[threadIdx.x] = 0;
+    __syncthreads();
+    const i64 base = (i64)blockIdx.x * kRsTile;
+    K key[kScItems];
+#pragma unroll
+    for (int k = 0; k < kScItems; ++k) {
+        const i64 i = base + (i64)k * kScThreads + threadIdx.x;
+        key[k] = i < n ? keys[i] : K(0);
+    }
+#pragma unroll
+    for (int k = 0; k < kScItems; ++k) {
+        const i64 i = base + (i64)k * kScThreads + threadIdx.x;
+        wave_count(h, (u32)(key[k] >> shift) & 255u, i < n);
+    }
+    __syncthreads();
+    if (threadIdx.x < 256) hist[(i64)blockIdx.x * 256 + threadIdx.x] = h[threadIdx.x];
+}
+
+template <class K, int NT>
+__global__ __launch_bounds__(NT) void k_split_scatter(const K* __restrict__ kin, const u32* __restrict__ vin,
+                                                      K* __restrict__ kout, u32* __restrict__ vout, i64 n, int shift,
+                                                      const int* __restrict__ hist, int ntiles,
+                                                      int* __restrict__ sizes) {
+    RAMA_SC_SHAPE(NT)
+    constexpr int kParts = NT / 256;  // threads adding up one digit's column
+    __shared__ K sk[kRsTile];
+    u32* const sv = reinterpret_cast<u32*>(sk);
+    __shared__ int wcnt[kScWaves][256];
+    __shared__ int dstart[256];
+    __shared__ int gbase[256];
+    __shared__ int part[2][kParts][256];
+
+    const int tid = threadIdx.x, lane = lane_id(), w = tid >> 6;
+    const i64 tile0 = (i64)blockIdx.x * kRsTile;
+    const i64 wbase = tile0 + (i64)w * (64 * kScItems);
+    K key[kScItems];
+    u32 val[kScItems];
+    int rnk[kScItems];
+#pragma unroll
+    for (int k = 0; k < kScItems; ++k) {
+        const i64 i = wbase + (i64)k * 64 + lane;
+        const bool ok = i < n;
+        key[k] = ok ? __builtin_nontemporal_load(&kin[i]) : ~K(0);
+        val[k] = ok ? __builtin_nontemporal_load(&vin[i]) : 0u;
+    }
+    for (int k = tid; k < kScWaves * 256; k += kScThreads) (&wcnt[0][0])[k] = 0;
+    {
+        const int d = tid & 255, g = tid >> 8;
+        int mine = 0, all = 0;
+        for (int t = g * 16; t < ntiles; t += kParts * 16) {
+            int x[16];
+#pragma unroll
+            for (int u = 0; u < 16; ++u) x[u] = t + u < ntiles ? hist[(i64)(t + u) * 256 + d] : 0;
+#pragma unroll
+            for (int u = 0; u < 16; ++u) {
+                mine += t + u < (int)blockIdx.x ? x[u] : 0;
+                all += x[u];
+            }
+        }
+        part[0][g][d] = mine;
+        part[1][g][d] = all;
+    }
+    __syncthreads();
+    const unsigned long long lt = (1ull << lane) - 1ull;
+#pragma unroll
+    for (int k = 0; k < kScItems; ++k) {
+        const u32 d = (u32)(key[k] >> shift) & 255u;
+        const unsigned long long peers = digit_peers(d, 8);
+        const int r = __popcll(peers & lt);
+        const int c = __popcll(peers);
+        const int before = wcnt[w][d];
+        __builtin_amdgcn_wave_barrier();
+        if (r == 0) wcnt[w][d] = before + c;
+        __builtin_amdgcn_wave_barrier();
+        rnk[k] = before + r;
+    }
+    int mine = 0;
+    if (tid < 256) {
+        int all = 0;
+#pragma unroll
+        for (int g = 0; g < kParts; ++g) {
+            mine += part[0][g][tid];
+            all += part[1][g][tid];
+        }
+        gbase[tid] = all;
+        if (blockIdx.x == 0) sizes[tid] = all;
+    }
+    __syncthreads();
+    if (tid < 256) {
+        int tot = 0;
+#pragma unroll
+        for (int q = 0; q < kScWaves; ++q) {
+            const int c = wcnt[q][tid];
+            wcnt[q][tid] = tot;
+            tot += c;
+        }
+        dstart[tid] = tot;
+    }
+    scan256(gbase);
+    scan256(dstart);
+    if (tid < 256) gbase[tid] += mine;
+    int pos[kScItems];
+#pragma unroll
+    for (int k = 0; k < kScItems; ++k) {
+        const u32 d = (u32)(key[k] >> shift) & 255u;
+        pos[k] = dstart[d] + wcnt[w][d] + rnk[k];
+        sk[pos[k]] = key[k];
+    }
+    __syncthreads();
+    const int nvalid = (int)((n - tile0) < kRsTile ? (n - tile0) : kRsTile);
+    i64 outp[kScItems];
+#pragma unroll
+    for (int q = 0; q < kScItems; ++q) {
+        const int p = tid + q * kScThreads;
+        outp[q] = -1;
+        if (p < nvalid) {
+            const K k = sk[p];
+            const u32 d = (u32)(k >> shift) & 255u;
+            const i64 o = (i64)gbase[d] + (p - dstart[d]);
+            kout[o] = k;
+            outp[q] = o;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kScItems; ++k) sv[pos[k]] = val[k];
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kScItems; ++q) {
         const int p = tid + q * kScThreads;
         if (p < nvalid) vout[outp[q]] = sv[p];
     }
@@ -411,6 +558,7 @@ __global__ __launch_bounds__(NT) void k_onesweep(const K* __restrict__ kin, cons
 constexpr int kTsThreads = 1024;
 constexpr int kTsItems = 8;
 constexpr int kTsTile = kTsThreads * kTsItems;
+constexpr int kTsMaxWork = 28;  // passes x items per thread that one block takes on
 constexpr int kTsWaves = kTsThreads / 64;
 
 template <class K>
@@ -429,7 +577,7 @@ struct TsSmem {
 // waves, s.dstart[d] the block's items of digit d, and rnk[k] is item k's
 // rank among its wave's items of the same digit.  Block-uniform call.
 template <class K>
-__device__ __forceinline__ void tile_rank(TsSmem<K>& s, const K (&key)[kTsItems], int shift, int bits,
+__device__ __forceinline__ void tile_rank(TsSmem<K>& s, const K (&key)[kTsItems], int items, int shift, int bits,
                                           int (&rnk)[kTsItems]) {
     const int tid = threadIdx.x, lane = lane_id(), w = tid >> 6;
     const u32 mask = (1u << bits) - 1u;
@@ -438,6 +586,7 @@ __device__ __forceinline__ void tile_rank(TsSmem<K>& s, const K (&key)[kTsItems]
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < kTsItems; ++k) {
+        if (k >= items) break;
         const u32 d = (u32)(key[k] >> shift) & mask;
         const unsigned long long peers = digit_peers(d, bits);
         const int r = __popcll(peers & lt);
@@ -464,18 +613,19 @@ __device__ __forceinline__ void tile_rank(TsSmem<K>& s, const K (&key)[kTsItems]
 
 // Every pass of `plan` over the block's register-held items, through LDS.
 template <class K>
-__device__ __forceinline__ void tile_sort_regs(TsSmem<K>& s, K (&key)[kTsItems], u32 (&val)[kTsItems],
+__device__ __forceinline__ void tile_sort_regs(TsSmem<K>& s, K (&key)[kTsItems], u32 (&val)[kTsItems], int items,
                                                const PassPlan& plan) {
     const int lane = lane_id(), w = threadIdx.x >> 6;
-    const int wbase = w * 64 * kTsItems;
+    const int wbase = w * 64 * items;
     int rnk[kTsItems];
     for (int p = 0; p < plan.passes; ++p) {
         const int shift = plan.shift[p], bits = plan.width[p];
         const u32 mask = (1u << bits) - 1u;
-        tile_rank(s, key, shift, bits, rnk);
+        tile_rank(s, key, items, shift, bits, rnk);
         scan256(s.dstart);
 #pragma unroll
         for (int k = 0; k < kTsItems; ++k) {
+            if (k >= items) break;
             const u32 d = (u32)(key[k] >> shift) & mask;
             const int pos = s.dstart[d] + s.wcnt[w][d] + rnk[k];
             s.sk[pos] = key[k];
@@ -484,6 +634,7 @@ __device__ __forceinline__ void tile_sort_regs(TsSmem<K>& s, K (&key)[kTsItems],
         __syncthreads();
 #pragma unroll
         for (int k = 0; k < kTsItems; ++k) {
+            if (k >= items) break;
             const int i = wbase + k * 64 + lane;
             key[k] = s.sk[i];
             val[k] = s.sv[i];
@@ -492,15 +643,21 @@ __device__ __forceinline__ void tile_sort_regs(TsSmem<K>& s, K (&key)[kTsItems],
     }
 }
 
-// Loads up to kTsTile pairs from (ki, vi) [0, n) into registers in
+// Items per thread that hold n <= kTsTile pairs.  A tile ranks, scatters and
+// reloads only those: with all kTsItems a bucket of a few hundred pairs cost
+// as much as a full one (most buckets hold 200 to 3000).
+__host__ __device__ __forceinline__ int tile_items(int n) { return (n + kTsThreads - 1) / kTsThreads; }
+
+// Loads up to kTsThreads * items pairs from (ki, vi) [0, n) into registers in
 // (wave, item, lane) order; the padding sorts after every real key (it
 // starts after them and has the largest digit in every pass).
 template <class K>
-__device__ __forceinline__ void tile_load(const K* __restrict__ ki, const u32* __restrict__ vi, int n,
+__device__ __forceinline__ void tile_load(const K* __restrict__ ki, const u32* __restrict__ vi, int n, int items,
                                           K (&key)[kTsItems], u32 (&val)[kTsItems]) {
-    const int lane = lane_id(), wbase = (threadIdx.x >> 6) * 64 * kTsItems;
+    const int lane = lane_id(), wbase = (threadIdx.x >> 6) * 64 * items;
 #pragma unroll
     for (int k = 0; k < kTsItems; ++k) {
+        if (k >= items) break;
         const int i = wbase + k * 64 + lane;
         const bool ok = i < n;
         key[k] = ok ? ki[i] : ~K(0);
@@ -509,11 +666,12 @@ __device__ __forceinline__ void tile_load(const K* __restrict__ ki, const u32* _
 }
 
 template <class K>
-__device__ __forceinline__ void tile_store(K* __restrict__ ko, u32* __restrict__ vo, int n, const K (&key)[kTsItems],
-                                           const u32 (&val)[kTsItems]) {
-    const int lane = lane_id(), wbase = (threadIdx.x >> 6) * 64 * kTsItems;
+__device__ __forceinline__ void tile_store(K* __restrict__ ko, u32* __restrict__ vo, int n, int items,
+                                           const K (&key)[kTsItems], const u32 (&val)[kTsItems]) {
+    const int lane = lane_id(), wbase = (threadIdx.x >> 6) * 64 * items;
 #pragma unroll
     for (int k = 0; k < kTsItems; ++k) {
+        if (k >= items) break;
         const int i = wbase + k * 64 + lane;
         if (i < n) {
             ko[i] = key[k];
@@ -528,9 +686,10 @@ __global__ __launch_bounds__(kTsThreads) void k_tile_sort(K* __restrict__ keys, 
     __shared__ TsSmem<K> s;
     K key[kTsItems];
     u32 val[kTsItems];
-    tile_load(keys, vals, n, key, val);
-    tile_sort_regs(s, key, val, plan);
-    tile_store(keys, vals, n, key, val);
+    const int items = tile_items(n);
+    tile_load(keys, vals, n, items, key, val);
+    tile_sort_regs(s, key, val, items, plan);
+    tile_store(keys, vals, n, items, key, val);
 }
 
 // Second stage of the top-digit sort.  An LSD pass on the top digit has
@@ -581,9 +740,10 @@ __global__ __launch_bounds__(kTsThreads) void k_bucket_sort(K* __restrict__ kin,
     K key[kTsItems];
     u32 val[kTsItems];
     if (m <= kTsTile) {
-        tile_load(ka, va, m, key, val);
-        tile_sort_regs(s, key, val, plan);
-        tile_store(kb, vb, m, key, val);
+        const int items = tile_items(m);
+        tile_load(ka, va, m, items, key, val);
+        tile_sort_regs(s, key, val, items, plan);
+        tile_store(kb, vb, m, items, key, val);
         return;
     }
     const int lane = lane_id(), w = tid >> 6, wbase = w * 64 * kTsItems;
@@ -609,8 +769,8 @@ __global__ __launch_bounds__(kTsThreads) void k_bucket_sort(K* __restrict__ kin,
         scan256(s.base);
         for (int t0 = 0; t0 < m; t0 += kTsTile) {  // uniform
             const int nt = min(kTsTile, m - t0);
-            tile_load(ks + t0, vs + t0, nt, key, val);
-            tile_rank(s, key, shift, bits, rnk);
+            tile_load(ks + t0, vs + t0, nt, kTsItems, key, val);
+            tile_rank(s, key, kTsItems, shift, bits, rnk);
 #pragma unroll
             for (int k = 0; k < kTsItems; ++k) {
                 if (wbase + k * 64 + lane < nt) {
@@ -690,7 +850,11 @@ static bool radix_sort_core(Ctx& ctx, K* keys, u32* vals, K* tk, u32* tv, i64 n,
     K* kb = tk;
     u32* vb = tv;
     const double pair_bytes = (double)(sizeof(K) + sizeof(u32));
-    if (n <= kTsTile) {
+    // one block sorts the lot where its passes cost less than the bucket path's
+    // three launches (about 28 to 34 us on up to 100k pairs): each pass is about
+    // 1 us per 1024 pairs, and 8000 pairs of 35 bits take 44 us in one block, 31
+    // in buckets
+    if (n <= kTsTile && tile_items((int)n) * plan.passes <= kTsMaxWork) {
         prof::Scope ps(ctx, "radix_tile_sort", 2.0 * pair_bytes * n);
         k_tile_sort<K><<<1, kTsThreads, 0, ctx.stream>>>(keys, vals, (int)n, plan);
         RAMA_LAUNCHED();
@@ -714,19 +878,18 @@ static bool radix_sort_core(Ctx& ctx, K* keys, u32* vals, K* tk, u32* tv, i64 n,
             low.shift[p] = sh;
             sh += low.width[p];
         }
-        const unsigned hb = (unsigned)std::min<i64>(ntiles, 1024);
-        DBuf<int> hist = ctx.buf<int>((i64)(hb + 1) * 256);
-        int* hsum = hist.get() + (i64)hb * 256;
+        DBuf<int> hist = ctx.buf<int>((i64)(ntiles + 1) * 256);
+        int* hsum = hist.get() + (i64)ntiles * 256;
         {
-            prof::Scope ps(ctx, "radix_hist_all", (double)sizeof(K) * n);
-            k_radix_hist_all<K><<<hb, kBlock, 0, ctx.stream>>>(keys, n, top, hist.get(), hsum, ctx.reduce_ticket());
+            prof::Scope ps(ctx, "radix_split_hist", (double)sizeof(K) * n);
+            k_split_hist<K, 1024><<<ntiles, 1024, 0, ctx.stream>>>(keys, n, top.shift[0], hist.get());
             RAMA_LAUNCHED();
         }
-        u32 epoch;
-        u64* st = ctx.scan_begin((i64)ntiles * 256, &epoch);
         {
-            prof::Scope ps(ctx, "radix_onesweep", 2.0 * pair_bytes * n);
-            launch_onesweep<K>(ctx, threads, ntiles, keys, vals, tk, tv, n, top.shift[0], 8, hsum, st, epoch);
+            prof::Scope ps(ctx, "radix_split_scatter", 2.0 * pair_bytes * n);
+            k_split_scatter<K, 1024><<<ntiles, 1024, 0, ctx.stream>>>(keys, vals, tk, tv, n, top.shift[0], hist.get(),
+                                                                      ntiles, hsum);
+            RAMA_LAUNCHED();
         }
         {
             prof::Scope ps(ctx, "radix_bucket_sort", 2.0 * pair_bytes * n);

@@ -18,7 +18,7 @@ namespace tune {
 
 enum Knob : int {
     // size = pairs; 0 = three launches per pass (histogram, scan, scatter),
-    // 1 = one onesweep launch per pass, 2 = a top-digit onesweep pass then one
+    // 1 = one onesweep launch per pass, 2 = a top-digit pass then one
     // block per bucket (keys wider than 8 bits, at most kBucketPathMaxTiles
     // tiles; otherwise 1)
     SortPathU64 = 0,

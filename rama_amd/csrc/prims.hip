@@ -204,44 +204,108 @@ __global__ __launch_bounds__(NT) void k_radix_scatter(const K* __restrict__ kin,
     }
 }
 
-// The top-digit pass of the bucket path: k_radix_scatter without an offset
-// scan before it.  The tiles' counts lie tile-major (hist[tile * 256 + d]);
-// every block adds up the columns itself, NT / 256 threads per digit with 16
-// loads in flight each, and block 0 leaves the bucket sizes in `sizes`.  Up to
-// a few hundred tiles this is cheaper than an order between blocks.  Whole
+// The bucket path's first pass: into 256 buckets of about equal size, by ranges
+// of the key's top 12 bits (4096 bins).  Every block of the histogram launch
+// samples the array at the same places, so all agree on the bins' share of
+// the buckets; block 0 leaves the table for the launches after it.  (Buckets
+// of equal key ranges leave most pairs of a graph's keys in a few of them: node
+// ids end below the next power of two, low ids hold the supernodes.  The
+// bucket sorts of a packed batch of 48 instances averaged 123 us with them, 23
+// with these; on uniform keys the sampling costs 3 to 8 us a sort.)
+constexpr int kSplitBins = 4096;
+struct SplitMap {
+    unsigned char bucket[kSplitBins];
+    int lo[257];    // first bin of each bucket
+    int sizes[256]; // pairs of each bucket
+};
+template <class K>
+__device__ __forceinline__ int split_bin(K key, int shift) {
+    const u64 b = (u64)(key >> shift);
+    return b < kSplitBins ? (int)b : kSplitBins - 1;  // padding keys: the last bin
+}
+
+// The scatter is k_radix_scatter without an offset scan before it.  The tiles'
+// counts lie tile-major (hist[tile * 256 + d]); every block adds up the
+// columns itself, NT / 256 threads per bucket with 16 loads in flight each.  Up
+// to a few hundred tiles this is cheaper than an order between blocks.  Whole
 // sorts of 35-bit u64 keys, with the buckets' items counted (tile_items),
-// against a onesweep pass behind a histogram that one block combines: 16k
-// pairs 39.5 -> 23.0 us, 260k 52.4 -> 28.6, 1M 79.8 -> 48.3; bound by the three
-// launches' load chains up to about 200k pairs, by the LDS passes above.
+// against a onesweep pass on the top 8 bits behind a histogram that one block
+// combines: 16k pairs 39.5 -> 25.8 us, 260k 52.4 -> 36.4, 1M 79.8 -> 66.0;
+// bound by the three launches' load chains up to about 200k pairs, by the LDS
+// passes above.
 template <class K, int NT>
-__global__ __launch_bounds__(NT) void k_split_hist(const K* __restrict__ keys, i64 n, int shift, int* hist) {
+__global__ __launch_bounds__(NT) void k_split_hist(const K* __restrict__ keys, i64 n, int shift, int log2samp, int* hist,
+                                                   SplitMap* __restrict__ sm) {
     RAMA_SC_SHAPE(NT)
+    constexpr int kPer = kSplitBins / NT;
+    __shared__ int cnt[kSplitBins];
+    __shared__ unsigned char bucket[kSplitBins];
+    __shared__ int ws[kScWaves];
     __shared__ int h[256];
-    if (threadIdx.x < 256) h[threadIdx.x] = 0;
-    __syncthreads();
+    const int tid = threadIdx.x, lane = lane_id(), w = tid >> 6;
     const i64 base = (i64)blockIdx.x * kRsTile;
     K key[kScItems];
 #pragma unroll
     for (int k = 0; k < kScItems; ++k) {
-        const i64 i = base + (i64)k * kScThreads + threadIdx.x;
+        const i64 i = base + (i64)k * kScThreads + tid;
         key[k] = i < n ? keys[i] : K(0);
     }
 #pragma unroll
-    for (int k = 0; k < kScItems; ++k) {
-        const i64 i = base + (i64)k * kScThreads + threadIdx.x;
-        wave_count(h, (u32)(key[k] >> shift) & 255u, i < n);
+    for (int k = 0; k < kPer; ++k) cnt[tid + k * NT] = 0;
+    if (tid < 256) h[tid] = 0;
+    __syncthreads();
+    for (int q = tid; q < (1 << log2samp); q += NT)
+        atomicAdd(&cnt[split_bin(keys[((u64)q * (u64)n) >> log2samp], shift)], 1);
+    __syncthreads();
+    {
+        int x[kPer], sum = 0;
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) {
+            x[k] = cnt[tid * kPer + k];
+            sum += x[k];
+        }
+        const int inc = wave_incl_scan(sum);
+        if (lane == 63) ws[w] = inc;
+        __syncthreads();
+        int run = inc - sum;
+#pragma unroll
+        for (int q = 0; q < kScWaves; ++q) run += q < w ? ws[q] : 0;
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) {
+            const int b = (run << 8) >> log2samp;
+            bucket[tid * kPer + k] = (unsigned char)(b < 255 ? b : 255);
+            run += x[k];
+        }
     }
     __syncthreads();
-    if (threadIdx.x < 256) hist[(i64)blockIdx.x * 256 + threadIdx.x] = h[threadIdx.x];
+#pragma unroll
+    for (int k = 0; k < kScItems; ++k) {
+        const i64 i = base + (i64)k * kScThreads + tid;
+        wave_count(h, (u32)bucket[split_bin(key[k], shift)], i < n);
+    }
+    if (blockIdx.x == 0) {
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) {
+            const int bin = tid + k * NT;
+            const int b = bucket[bin], pb = bin > 0 ? (int)bucket[bin - 1] : -1;
+            sm->bucket[bin] = (unsigned char)b;
+            for (int q = pb + 1; q <= b; ++q) sm->lo[q] = bin;
+            if (bin == kSplitBins - 1)
+                for (int q = b + 1; q <= 256; ++q) sm->lo[q] = kSplitBins;
+        }
+    }
+    __syncthreads();
+    if (tid < 256) hist[(i64)blockIdx.x * 256 + tid] = h[tid];
 }
 
 template <class K, int NT>
 __global__ __launch_bounds__(NT) void k_split_scatter(const K* __restrict__ kin, const u32* __restrict__ vin,
                                                       K* __restrict__ kout, u32* __restrict__ vout, i64 n, int shift,
                                                       const int* __restrict__ hist, int ntiles,
-                                                      int* __restrict__ sizes) {
+                                                      SplitMap* __restrict__ sm) {
     RAMA_SC_SHAPE(NT)
-    constexpr int kParts = NT / 256;  // threads adding up one digit's column
+    constexpr int kParts = NT / 256;  // threads adding up one bucket's column
+    __shared__ __align__(4) unsigned char bucket[kSplitBins];
     __shared__ K sk[kRsTile];
     u32* const sv = reinterpret_cast<u32*>(sk);
     __shared__ int wcnt[kScWaves][256];
@@ -263,6 +327,8 @@ __global__ __launch_bounds__(NT) void k_split_scatter(const K* __restrict__ kin,
         val[k] = ok ? __builtin_nontemporal_load(&vin[i]) : 0u;
     }
     for (int k = tid; k < kScWaves * 256; k += kScThreads) (&wcnt[0][0])[k] = 0;
+    for (int k = tid; k < kSplitBins / 4; k += kScThreads)
+        reinterpret_cast<u32*>(bucket)[k] = reinterpret_cast<const u32*>(sm->bucket)[k];
     {
         const int d = tid & 255, g = tid >> 8;
         int mine = 0, all = 0;
@@ -283,7 +349,7 @@ __global__ __launch_bounds__(NT) void k_split_scatter(const K* __restrict__ kin,
     const unsigned long long lt = (1ull << lane) - 1ull;
 #pragma unroll
     for (int k = 0; k < kScItems; ++k) {
-        const u32 d = (u32)(key[k] >> shift) & 255u;
+        const u32 d = bucket[split_bin(key[k], shift)];
         const unsigned long long peers = digit_peers(d, 8);
         const int r = __popcll(peers & lt);
         const int c = __popcll(peers);
@@ -302,7 +368,7 @@ __global__ __launch_bounds__(NT) void k_split_scatter(const K* __restrict__ kin,
             all += part[1][g][tid];
         }
         gbase[tid] = all;
-        if (blockIdx.x == 0) sizes[tid] = all;
+        if (blockIdx.x == 0) sm->sizes[tid] = all;
     }
     __syncthreads();
     if (tid < 256) {
@@ -321,7 +387,7 @@ __global__ __launch_bounds__(NT) void k_split_scatter(const K* __restrict__ kin,
     int pos[kScItems];
 #pragma unroll
     for (int k = 0; k < kScItems; ++k) {
-        const u32 d = (u32)(key[k] >> shift) & 255u;
+        const u32 d = bucket[split_bin(key[k], shift)];
         pos[k] = dstart[d] + wcnt[w][d] + rnk[k];
         sk[pos[k]] = key[k];
     }
@@ -334,7 +400,7 @@ __global__ __launch_bounds__(NT) void k_split_scatter(const K* __restrict__ kin,
         outp[q] = -1;
         if (p < nvalid) {
             const K k = sk[p];
-            const u32 d = (u32)(k >> shift) & 255u;
+            const u32 d = bucket[split_bin(k, shift)];
             const i64 o = (i64)gbase[d] + (p - dstart[d]);
             kout[o] = k;
             outp[q] = o;
@@ -611,15 +677,25 @@ __device__ __forceinline__ void tile_rank(TsSmem<K>& s, const K (&key)[kTsItems]
     __syncthreads();
 }
 
-// Every pass of `plan` over the block's register-held items, through LDS.
+// Balanced passes over `bits` key bits: pass p sorts `width(p)` bits from
+// `shift(p)` on.
+struct Passes {
+    int n, base, extra;
+    __host__ __device__ __forceinline__ explicit Passes(int bits)
+        : n((bits + 7) / 8), base(n ? bits / n : 0), extra(n ? bits % n : 0) {}
+    __host__ __device__ __forceinline__ int width(int p) const { return base + (p < extra ? 1 : 0); }
+    __host__ __device__ __forceinline__ int shift(int p) const { return p * base + (p < extra ? p : extra); }
+};
+
+// Every pass over the block's register-held items, through LDS.
 template <class K>
 __device__ __forceinline__ void tile_sort_regs(TsSmem<K>& s, K (&key)[kTsItems], u32 (&val)[kTsItems], int items,
-                                               const PassPlan& plan) {
+                                               const Passes& plan) {
     const int lane = lane_id(), w = threadIdx.x >> 6;
     const int wbase = w * 64 * items;
     int rnk[kTsItems];
-    for (int p = 0; p < plan.passes; ++p) {
-        const int shift = plan.shift[p], bits = plan.width[p];
+    for (int p = 0; p < plan.n; ++p) {
+        const int shift = plan.shift(p), bits = plan.width(p);
         const u32 mask = (1u << bits) - 1u;
         tile_rank(s, key, items, shift, bits, rnk);
         scan256(s.dstart);
@@ -649,24 +725,24 @@ __device__ __forceinline__ void tile_sort_regs(TsSmem<K>& s, K (&key)[kTsItems],
 __host__ __device__ __forceinline__ int tile_items(int n) { return (n + kTsThreads - 1) / kTsThreads; }
 
 // Loads up to kTsThreads * items pairs from (ki, vi) [0, n) into registers in
-// (wave, item, lane) order; the padding sorts after every real key (it
-// starts after them and has the largest digit in every pass).
+// (wave, item, lane) order, less `base`; the padding sorts after every real key
+// (it starts after them and has the largest digit in every pass).
 template <class K>
 __device__ __forceinline__ void tile_load(const K* __restrict__ ki, const u32* __restrict__ vi, int n, int items,
-                                          K (&key)[kTsItems], u32 (&val)[kTsItems]) {
+                                          K base, K (&key)[kTsItems], u32 (&val)[kTsItems]) {
     const int lane = lane_id(), wbase = (threadIdx.x >> 6) * 64 * items;
 #pragma unroll
     for (int k = 0; k < kTsItems; ++k) {
         if (k >= items) break;
         const int i = wbase + k * 64 + lane;
         const bool ok = i < n;
-        key[k] = ok ? ki[i] : ~K(0);
+        key[k] = ok ? (K)(ki[i] - base) : ~K(0);
         val[k] = ok ? vi[i] : 0u;
     }
 }
 
 template <class K>
-__device__ __forceinline__ void tile_store(K* __restrict__ ko, u32* __restrict__ vo, int n, int items,
+__device__ __forceinline__ void tile_store(K* __restrict__ ko, u32* __restrict__ vo, int n, int items, K base,
                                            const K (&key)[kTsItems], const u32 (&val)[kTsItems]) {
     const int lane = lane_id(), wbase = (threadIdx.x >> 6) * 64 * items;
 #pragma unroll
@@ -674,7 +750,7 @@ __device__ __forceinline__ void tile_store(K* __restrict__ ko, u32* __restrict__
         if (k >= items) break;
         const int i = wbase + k * 64 + lane;
         if (i < n) {
-            ko[i] = key[k];
+            ko[i] = key[k] + base;
             vo[i] = val[k];
         }
     }
@@ -682,54 +758,48 @@ __device__ __forceinline__ void tile_store(K* __restrict__ ko, u32* __restrict__
 
 template <class K>
 __global__ __launch_bounds__(kTsThreads) void k_tile_sort(K* __restrict__ keys, u32* __restrict__ vals, int n,
-                                                          PassPlan plan) {
+                                                          int bits) {
     __shared__ TsSmem<K> s;
     K key[kTsItems];
     u32 val[kTsItems];
     const int items = tile_items(n);
-    tile_load(keys, vals, n, items, key, val);
-    tile_sort_regs(s, key, val, items, plan);
-    tile_store(keys, vals, n, items, key, val);
+    tile_load(keys, vals, n, items, K(0), key, val);
+    tile_sort_regs(s, key, val, items, Passes(bits));
+    tile_store(keys, vals, n, items, K(0), key, val);
 }
 
-// Second stage of the top-digit sort.  An LSD pass on the top digit has
-// grouped the pairs into 256 buckets (kin/vin, stable); block b sorts bucket
-// b stably by the remaining low bits (`plan`) and writes it to the same
-// range of kout/vout.  Bucket bounds: with stride 0, `bnd` holds the 256
-// bucket sizes; otherwise bucket d starts at bnd[d * stride] (a scanned
-// digit-major tile table) and the last one ends at n.  A bucket that fits in
-// LDS is sorted as a tile.  A larger one is sorted by the block alone: the
-// histograms of every pass in one sweep, then per pass its tiles in order,
-// each ranked in LDS and scattered after the earlier tiles' items of each
-// digit, ping-ponging between the bucket's two ranges.
+// Second stage of the bucket path.  k_split_scatter has grouped the pairs into
+// 256 buckets (kin/vin, stable); block b sorts bucket b stably by its keys'
+// offset from the bucket's first bin and writes it to the same range of
+// kout/vout.  A bucket that fits in LDS is sorted as a tile.  A larger one (many
+// equal keys) is sorted by the block alone: the histograms of every pass in
+// one sweep, then per pass its tiles in order, each ranked in LDS and
+// scattered after the earlier tiles' items of each digit, ping-ponging between
+// the bucket's two ranges.
 template <class K>
 __global__ __launch_bounds__(kTsThreads) void k_bucket_sort(K* __restrict__ kin, u32* __restrict__ vin,
                                                             K* __restrict__ kout, u32* __restrict__ vout,
-                                                            const int* __restrict__ bnd, int stride, int n,
-                                                            PassPlan plan) {
+                                                            const SplitMap* __restrict__ sm, int shift12) {
     __shared__ TsSmem<K> s;
     const int tid = threadIdx.x, b = blockIdx.x;
-    if (stride == 0) {
-        if (tid < 64) {
-            // start of bucket b: the sizes of the buckets before it
-            int acc = 0;
+    if (tid < 64) {
+        // start of bucket b: the sizes of the buckets before it
+        int acc = 0;
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int d = tid * 4 + q;
-                acc += d < b ? bnd[d] : 0;
-            }
-#pragma unroll
-            for (int o = 32; o >= 1; o >>= 1) acc += __shfl_xor(acc, o, 64);
-            if (tid == 0) {
-                s.misc[0] = acc;
-                s.misc[1] = bnd[b];
-            }
+        for (int q = 0; q < 4; ++q) {
+            const int d = tid * 4 + q;
+            acc += d < b ? sm->sizes[d] : 0;
         }
-    } else if (tid == 0) {
-        const int b0 = bnd[(i64)b * stride];
-        s.misc[0] = b0;
-        s.misc[1] = (b < 255 ? bnd[(i64)(b + 1) * stride] : n) - b0;
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1) acc += __shfl_xor(acc, o, 64);
+        if (tid == 0) {
+            s.misc[0] = acc;
+            s.misc[1] = sm->sizes[b];
+        }
     }
+    const int bin0 = sm->lo[b], bins = sm->lo[b + 1] - bin0;
+    const K first = (K)bin0 << shift12;
+    const Passes plan(shift12 + (bins > 1 ? 32 - __clz(bins - 1) : 0));
     __syncthreads();
     const int beg = s.misc[0], m = s.misc[1];
     if (m == 0) return;  // uniform
@@ -741,9 +811,9 @@ __global__ __launch_bounds__(kTsThreads) void k_bucket_sort(K* __restrict__ kin,
     u32 val[kTsItems];
     if (m <= kTsTile) {
         const int items = tile_items(m);
-        tile_load(ka, va, m, items, key, val);
+        tile_load(ka, va, m, items, first, key, val);
         tile_sort_regs(s, key, val, items, plan);
-        tile_store(kb, vb, m, items, key, val);
+        tile_store(kb, vb, m, items, first, key, val);
         return;
     }
     const int lane = lane_id(), w = tid >> 6, wbase = w * 64 * kTsItems;
@@ -752,13 +822,13 @@ __global__ __launch_bounds__(kTsThreads) void k_bucket_sort(K* __restrict__ kin,
     for (int k = tid; k < 8 * 256; k += kTsThreads) (&s.ph[0][0])[k] = 0;
     __syncthreads();
     for (int i = tid; i < m; i += kTsThreads) {
-        const K x = ka[i];
-        for (int p = 0; p < plan.passes; ++p)
-            atomicAdd(&s.ph[p][(u32)(x >> plan.shift[p]) & ((1u << plan.width[p]) - 1u)], 1);
+        const K x = ka[i] - first;
+        for (int p = 0; p < plan.n; ++p)
+            atomicAdd(&s.ph[p][(u32)(x >> plan.shift(p)) & ((1u << plan.width(p)) - 1u)], 1);
     }
     __syncthreads();
-    for (int p = 0; p < plan.passes; ++p) {
-        const int shift = plan.shift[p], bits = plan.width[p];
+    for (int p = 0; p < plan.n; ++p) {
+        const int shift = plan.shift(p), bits = plan.width(p);
         const u32 mask = (1u << bits) - 1u;
         K* ks = (p & 1) ? kb : ka;
         u32* vs = (p & 1) ? vb : va;
@@ -769,14 +839,14 @@ __global__ __launch_bounds__(kTsThreads) void k_bucket_sort(K* __restrict__ kin,
         scan256(s.base);
         for (int t0 = 0; t0 < m; t0 += kTsTile) {  // uniform
             const int nt = min(kTsTile, m - t0);
-            tile_load(ks + t0, vs + t0, nt, kTsItems, key, val);
+            tile_load(ks + t0, vs + t0, nt, kTsItems, first, key, val);
             tile_rank(s, key, kTsItems, shift, bits, rnk);
 #pragma unroll
             for (int k = 0; k < kTsItems; ++k) {
                 if (wbase + k * 64 + lane < nt) {
                     const u32 d = (u32)(key[k] >> shift) & mask;
                     const int o = s.base[d] + s.wcnt[w][d] + rnk[k];
-                    kd[o] = key[k];
+                    kd[o] = key[k] + first;
                     vd[o] = val[k];
                 }
             }
@@ -786,7 +856,7 @@ __global__ __launch_bounds__(kTsThreads) void k_bucket_sort(K* __restrict__ kin,
             __syncthreads();
         }
     }
-    if ((plan.passes & 1) == 0) {
+    if ((plan.n & 1) == 0) {
         // an even pass count ends in the input range: copy to the output
         for (int i = tid; i < m; i += kTsThreads) {
             kb[i] = ka[i];
@@ -856,7 +926,7 @@ static bool radix_sort_core(Ctx& ctx, K* keys, u32* vals, K* tk, u32* tv, i64 n,
     // in buckets
     if (n <= kTsTile && tile_items((int)n) * plan.passes <= kTsMaxWork) {
         prof::Scope ps(ctx, "radix_tile_sort", 2.0 * pair_bytes * n);
-        k_tile_sort<K><<<1, kTsThreads, 0, ctx.stream>>>(keys, vals, (int)n, plan);
+        k_tile_sort<K><<<1, kTsThreads, 0, ctx.stream>>>(keys, vals, (int)n, bits);
         RAMA_LAUNCHED();
         return false;
     }
@@ -864,36 +934,26 @@ static bool radix_sort_core(Ctx& ctx, K* keys, u32* vals, K* tk, u32* tv, i64 n,
     if (threads < 0) threads = (int)tune::get(tune::SortThreads, ntiles);
     if (path == 2 && (bits <= 8 || ntiles > tune::kBucketPathMaxTiles)) path = 1;
     if (path == 2) {
-        // one pass on the top 8 bits into 256 buckets (histogram +
-        // onesweep), then each bucket's low bits in one block
-        PassPlan top{}, low{};
-        top.passes = 1;
-        top.shift[0] = bits - 8;
-        top.width[0] = 8;
-        const int lb = bits - 8;
-        low.passes = (lb + 7) / 8;
-        const int bw = lb / low.passes, ex = lb % low.passes;
-        for (int p = 0, sh = 0; p < low.passes; ++p) {
-            low.width[p] = bw + (p < ex ? 1 : 0);
-            low.shift[p] = sh;
-            sh += low.width[p];
-        }
-        DBuf<int> hist = ctx.buf<int>((i64)(ntiles + 1) * 256);
-        int* hsum = hist.get() + (i64)ntiles * 256;
+        // one pass into 256 buckets (histogram + scatter), then each bucket in
+        // one block; more samples where a bucket twice the mean would not fit in LDS
+        const int shift12 = bits > 12 ? bits - 12 : 0;
+        const int log2samp = n <= ((i64)1 << 18) ? 11 : 13;
+        DBuf<int> hist = ctx.buf<int>((i64)ntiles * 256);
+        DBuf<SplitMap> sm = ctx.buf<SplitMap>(1);
         {
             prof::Scope ps(ctx, "radix_split_hist", (double)sizeof(K) * n);
-            k_split_hist<K, 1024><<<ntiles, 1024, 0, ctx.stream>>>(keys, n, top.shift[0], hist.get());
+            k_split_hist<K, 1024><<<ntiles, 1024, 0, ctx.stream>>>(keys, n, shift12, log2samp, hist.get(), sm.get());
             RAMA_LAUNCHED();
         }
         {
             prof::Scope ps(ctx, "radix_split_scatter", 2.0 * pair_bytes * n);
-            k_split_scatter<K, 1024><<<ntiles, 1024, 0, ctx.stream>>>(keys, vals, tk, tv, n, top.shift[0], hist.get(),
-                                                                      ntiles, hsum);
+            k_split_scatter<K, 1024><<<ntiles, 1024, 0, ctx.stream>>>(keys, vals, tk, tv, n, shift12, hist.get(),
+                                                                      ntiles, sm.get());
             RAMA_LAUNCHED();
         }
         {
             prof::Scope ps(ctx, "radix_bucket_sort", 2.0 * pair_bytes * n);
-            k_bucket_sort<K><<<256, kTsThreads, 0, ctx.stream>>>(tk, tv, keys, vals, hsum, 0, (int)n, low);
+            k_bucket_sort<K><<<256, kTsThreads, 0, ctx.stream>>>(tk, tv, keys, vals, sm.get(), shift12);
             RAMA_LAUNCHED();
         }
         return false;

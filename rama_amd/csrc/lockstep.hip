@@ -36,6 +36,7 @@ struct Slot {
     int n0;          // number of labels
     double lb;       // lower bound of the initial dual
     int iter;        // the instance's next round (0 = first)
+    bool quiet;      // its last cycle search found nothing
 };
 
 struct Pack {
@@ -446,6 +447,7 @@ void packed_dual_update(Ctx& ctx, Pack& P, int c, int steps, float factor, float
     for (int q = 0; q < Q; ++q) {
         if (!on[q]) continue;
         num_tri[q] = T.raw[q];
+        P.s[q].quiet = T.raw[q] == 0;
         if (T.raw[q] == 0) need_lb = true;
         else mp_on[q] = 1, any_mp = true;
     }
@@ -563,14 +565,23 @@ std::vector<int32_t> gather_labels(Ctx& ctx, const Pack& P, const std::vector<in
 }
 
 // ------------------------------------------------------------ handoff
+// What a group of slots takes along, read back together; each slot's share
+// lies at its Handoff's offsets.
+struct HandoffData {
+    std::vector<int32_t> row, col;  // ids of the pack
+    std::vector<float> val;
+    std::vector<int32_t> labels;
+};
 struct Handoff {
     int id = 0;
     int next_iter = 0;
-    std::vector<int32_t> row, col;  // local ids
-    std::vector<float> val;
+    std::shared_ptr<HandoffData> data;
+    i64 edge = 0, nnz = 0;  // edges [edge, edge + nnz)
+    i64 label = 0, n0 = 0;
+    int base = 0;           // the instance's first id in the pack
     int rows = 0, cols = 0, max_node = -1;
-    std::vector<int32_t> labels;
     double lb = 0.0;
+    bool use_mm = false;  // matching still picks the contractions
 };
 
 }  // namespace
@@ -580,8 +591,9 @@ struct Handoff {
 // The lockstep solver: instances are admitted in groups (each group runs
 // its initial dual on arrival), and every call of round() advances all
 // admitted instances by one contraction round.  Instances leave when they
-// finish; those that switch to the forest contraction are continued by
-// `workers` threads with the single-instance rounds.
+// finish; those that switch to the forest contraction, and those whose rounds
+// the single-instance solver runs without read-backs (kLeaveEdges), are
+// continued by `workers` threads with the single-instance rounds.
 class Lockstep {
    public:
     Lockstep(Ctx& ctx, const Options& o, int workers, LockstepSink& sink) : ctx_(ctx), o_(o), sink_(sink) {
@@ -592,6 +604,15 @@ class Lockstep {
     ~Lockstep() { finish(); }
 
     static constexpr int kMaxSlots = kLockstepMaxSlots;
+    // An instance of at most kLeaveEdges edges whose cycle searches find nothing
+    // any more leaves a pack of at most kLeavePack edges: its remaining rounds
+    // take a worker one launch (small_rounds), where the pack's rounds cost
+    // 0.4 ms however few instances are left (48 instances of up to 60k nodes:
+    // 49.8 -> 43.0 ms; a burst of 24 requests 45.6 -> 38.2).  In a larger pack
+    // the rounds are bound by their bytes and the small instances ride along
+    // (512 instances, 57.6M edges: 1% slower if they leave).
+    static constexpr i64 kLeaveEdges = kSmallMaxEdges;
+    static constexpr i64 kLeavePack = (i64)1 << 22;
     int slots() const { return P_.Q(); }
     bool empty() const { return P_.Q() == 0; }
 
@@ -646,8 +667,9 @@ class Lockstep {
     }
     // Keeps only the slots with keep[q] (edges, labels, ids shifted down).
     void compact(const std::vector<char>& keep);
-    // Hands the slots in `which` to the workers (next round of each: its iter).
-    void hand_off_slots(const std::vector<int>& which);
+    // Hands the slots in `which` to the workers (next round of each: its
+    // iter), mm[x] telling whether which[x] still matches.
+    void hand_off_slots(const std::vector<int>& which, const std::vector<char>& mm);
 
     Ctx& ctx_;
     Options o_;
@@ -678,22 +700,31 @@ void Lockstep::worker() {
             if (!wctx) wctx.reset(new Ctx(ctx_.device, nullptr, false));
             Ctx& w = *wctx;
             DCoo A;
-            A.nnz = (i64)h.val.size();
+            A.nnz = h.nnz;
             A.row = w.buf<int>(A.nnz);
             A.col = w.buf<int>(A.nnz);
             A.val = w.buf<float>(A.nnz);
-            w.h2d(A.row.get(), h.row.data(), A.nnz);
-            w.h2d(A.col.get(), h.col.data(), A.nnz);
-            w.h2d(A.val.get(), h.val.data(), A.nnz);
+            w.h2d(A.row.get(), h.data->row.data() + h.edge, A.nnz);
+            w.h2d(A.col.get(), h.data->col.data() + h.edge, A.nnz);
+            w.h2d(A.val.get(), h.data->val.data() + h.edge, A.nnz);
+            {
+                int* R = A.row.get();
+                int* C = A.col.get();
+                const int base = h.base;
+                for_each(w, A.nnz, [=] __device__(i64 e) {
+                    R[e] -= base;
+                    C[e] -= base;
+                });
+            }
             A.rows = h.rows;
             A.cols = h.cols;
             A.max_node = h.max_node;
             SolveResult out;
-            out.num_labels = (i64)h.labels.size();
+            out.num_labels = h.n0;
             out.labels = w.buf<int>(out.num_labels);
-            w.h2d(out.labels.get(), h.labels.data(), out.num_labels);
+            w.h2d(out.labels.get(), h.data->labels.data() + h.label, out.num_labels);
             out.lb = h.lb;
-            solve_rounds(w, A, out, o_, h.next_iter, false);
+            solve_rounds(w, A, out, o_, h.next_iter, h.use_mm, h.use_mm);
             std::vector<int32_t> lab((size_t)out.num_labels);
             if (out.num_labels > 0) w.d2h(lab.data(), out.labels.get(), out.num_labels);
             sink_.done(h.id, 0, "", lab.data(), out.num_labels, h.lb);
@@ -765,7 +796,7 @@ void Lockstep::compact(const std::vector<char>& keep) {
     pack_index(ctx_, P_);
 }
 
-void Lockstep::hand_off_slots(const std::vector<int>& which) {
+void Lockstep::hand_off_slots(const std::vector<int>& which, const std::vector<char>& mm) {
     if (which.empty()) return;
     scan_check(ctx_);
     const int Q = P_.Q();
@@ -777,8 +808,10 @@ void Lockstep::hand_off_slots(const std::vector<int>& which) {
         hoff.push_back(mh);
         mh += P_.s[q].nnz;
     }
-    std::vector<int32_t> er((size_t)mh), ec((size_t)mh);
-    std::vector<float> ev((size_t)mh);
+    auto data = std::make_shared<HandoffData>();
+    data->row.resize((size_t)mh);
+    data->col.resize((size_t)mh);
+    data->val.resize((size_t)mh);
     if (mh > 0) {
         // the slots' edges, gathered on the device in slot order
         DBuf<int> din = upload_vec(ctx_, isin);
@@ -801,11 +834,11 @@ void Lockstep::hand_off_slots(const std::vector<int>& which) {
                 GW[p] = AW[e];
             },
             cnt.get());
-        ctx_.d2h(er.data(), gr.get(), mh);
-        ctx_.d2h(ec.data(), gc.get(), mh);
-        ctx_.d2h(ev.data(), gw.get(), mh);
+        ctx_.d2h(data->row.data(), gr.get(), mh);
+        ctx_.d2h(data->col.data(), gc.get(), mh);
+        ctx_.d2h(data->val.data(), gw.get(), mh);
     }
-    const std::vector<int32_t> hl = gather_labels(ctx_, P_, which);
+    data->labels = gather_labels(ctx_, P_, which);
     i64 lo = 0;
     for (size_t x = 0; x < which.size(); ++x) {
         const int q = which[x];
@@ -817,16 +850,14 @@ void Lockstep::hand_off_slots(const std::vector<int>& which) {
         h.cols = s.cols;
         h.max_node = s.max_node;
         h.lb = s.lb;
-        h.labels.assign(hl.begin() + lo, hl.begin() + lo + s.n0);
+        h.use_mm = mm[x] != 0;
+        h.data = data;
+        h.edge = hoff[x];
+        h.nnz = s.nnz;
+        h.label = lo;
+        h.n0 = s.n0;
+        h.base = P_.base[q];
         lo += s.n0;
-        h.row.resize((size_t)s.nnz);
-        h.col.resize((size_t)s.nnz);
-        h.val.resize((size_t)s.nnz);
-        for (i64 e = 0; e < s.nnz; ++e) {
-            h.row[e] = er[hoff[x] + e] - P_.base[q];
-            h.col[e] = ec[hoff[x] + e] - P_.base[q];
-            h.val[e] = ev[hoff[x] + e];
-        }
         hand_off(std::move(h));
     }
 }
@@ -996,7 +1027,7 @@ void Lockstep::admit(int k, const int64_t* edge_off, const int32_t* i, const int
             which.push_back(q);
             keep[q] = 0;
         }
-        hand_off_slots(which);
+        hand_off_slots(which, std::vector<char>(which.size(), 0));
         compact(keep);
     }
 }
@@ -1176,9 +1207,11 @@ void Lockstep::round() {
     pack_index(ctx_, P_);
     mark("s:contract", 0, Qc);
     // slots leaving: failed (bad contraction), done (no edges left), handed
-    // off (switching to the forest contraction)
+    // off (switching to the forest contraction, or small and quiet)
     std::vector<int> done, hand;
-    std::vector<char> keep((size_t)Qc, 1);
+    std::vector<char> keep((size_t)Qc, 1), mm;
+    const bool duals = o_.max_cycle_length_primal >= 3 && o_.num_dual_itr_primal != 0;
+    const bool leave = nnz <= kLeavePack;
     for (int c = 0; c < Qc; ++c) {
         if (hst[c].bad) {
             sink_.done(P_.s[c].id, RAMA_ERR_BAD_CONTRACTION, "Found bad contractions", nullptr, 0, P_.s[c].lb);
@@ -1186,13 +1219,14 @@ void Lockstep::round() {
         } else if (P_.s[c].nnz == 0) {
             done.push_back(c);  // A.nnz == 0 ends the rounds
             keep[c] = 0;
-        } else if (swc[c]) {
+        } else if (swc[c] || (leave && P_.s[c].nnz <= kLeaveEdges && (!duals || P_.s[c].quiet))) {
             hand.push_back(c);
+            mm.push_back(swc[c] ? 0 : 1);
             keep[c] = 0;
         }
     }
     if (!done.empty()) publish(done);
-    hand_off_slots(hand);
+    hand_off_slots(hand, mm);
     compact(keep);
 }
 

@@ -287,6 +287,8 @@ struct SolveResult {
     std::vector<std::vector<int>> timeline;
 };
 SolveResult solve(Ctx& ctx, DCoo& A, const Options& o);
-void solve_rounds(Ctx& ctx, DCoo& A, SolveResult& out, const Options& o, int start_iter, bool use_mm);
+// quiet: the last cycle search on the instance found nothing (start_iter > 0).
+void solve_rounds(Ctx& ctx, DCoo& A, SolveResult& out, const Options& o, int start_iter, bool use_mm,
+                  bool quiet = false);
 
 }  // namespace rama

@@ -80,9 +80,9 @@ SolveResult solve(Ctx& ctx, DCoo& A, const Options& o) {
 // The contraction rounds from round `start_iter` on (src/rama_cuda.cu:88-158):
 // out.labels (out.num_labels entries) holds the labels composed so far and
 // use_mm whether matching still picks the contractions.
-void solve_rounds(Ctx& ctx, DCoo& A, SolveResult& out, const Options& o, int start_iter, bool use_mm) {
+void solve_rounds(Ctx& ctx, DCoo& A, SolveResult& out, const Options& o, int start_iter, bool use_mm, bool quiet) {
     StageTimes st;
-    if (start_iter > 0) ctx.last_cycles_empty = false;  // resumed on another context: no hint
+    if (start_iter > 0) ctx.last_cycles_empty = quiet;  // resumed on another context
     const auto t0 = out.t0;  // the time budget counts from the start of the solve
     const i64 N = out.num_labels;
     const bool duals = o.max_cycle_length_primal >= 3 && o.num_dual_itr_primal != 0;

@@ -10,9 +10,11 @@ namespace rama {
 // dual_update_cycle_length (src/dual_solver.cu:7-35).  Returns the lower
 // bound; `num_tri` receives the raw triangle count of the search.
 static double dual_update_cycle_length(Ctx& ctx, DCoo& A, int c, int steps, float factor, float tol, i64* num_tri,
-                                       bool want_lb) {
-    Triangles tri = conflicted_cycles(ctx, A, c, factor, tol);
+                                       bool want_lb, CycleSearch& known) {
+    // a verbose run prints every stage's count, so it searches from scratch
+    Triangles tri = conflicted_cycles(ctx, A, c, factor, tol, ctx.verbose ? nullptr : &known);
     *num_tri = tri.raw;
+    if (tri.raw > 0) known = CycleSearch();  // the graph changes
     if (tri.raw == 0) return want_lb ? dcoo_lb(ctx, A.val.get(), A.nnz) : 0.0;
     MPState S;
     mp_build(ctx, A, tri, S);
@@ -46,8 +48,9 @@ double dual_solver(Ctx& ctx, DCoo& A, int max_len, int num_iter, float factor, i
     i64 num_tri = 0;
     try {
         for (int o = 0; o < num_outer; ++o) {
+            CycleSearch known;
             for (int c = 3; c <= max_len; ++c)
-                fin = dual_update_cycle_length(ctx, A, c, num_iter, factor, tol, &num_tri, need);
+                fin = dual_update_cycle_length(ctx, A, c, num_iter, factor, tol, &num_tri, need, known);
             if (num_tri == 0 || (o > 0 && (fin - prev) < 1e-3)) break;
             prev = fin;
         }

@@ -114,7 +114,18 @@ struct Triangles {
     i64 raw = 0;  // slots filled by the search (reference triangles_v1.size())
     int max_id = -1;  // known bound on the vertex ids (-1: unknown, scan them)
 };
-Triangles conflicted_cycles(Ctx& ctx, const DCoo& A, int max_cycle_length, float tri_memory_factor, float tol_ratio);
+// What a search that found nothing leaves for the next one on the same,
+// unchanged graph with the same factor and tolerance but longer cycles: the
+// attractive CSR, the repulsive edges and how far the search has come.
+struct CycleSearch {
+    int empty_to = 0;  // cycles of up to this length are known not to exist (0: nothing known)
+    bool none = false; // no attractive or no repulsive edge: no cycles at all
+    Csr G;
+    DBuf<int> rv1, rv2;
+    i64 R = 0;
+};
+Triangles conflicted_cycles(Ctx& ctx, const DCoo& A, int max_cycle_length, float tri_memory_factor, float tol_ratio,
+                            CycleSearch* known = nullptr);
 template <int S>
 void run_stage_packed(Ctx& ctx, const Csr& G, const int* rv1, const int* rv2, i64 R, const int* nslot, int Q,
                       const i64* d_base, const i64* d_budget, const i64* d_out, int* t1, int* t2, int* t3,

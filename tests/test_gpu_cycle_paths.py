@@ -58,3 +58,23 @@ def test_cycle_paths_batched_equal(gpu, monkeypatch):
         for (la, lba), (lg, lbg) in zip(ref, got):
             assert lba == lbg, (tables, form)
             assert np.array_equal(la, lg), (tables, form)
+
+
+@pytest.mark.parametrize("length", [4, 5])
+def test_dual_pass_first_cycles_are_longer(gpu, oracle, length):
+    """No 3-cycles (nor 4-cycles): the dual pass's later searches take over
+    what the fruitless ones before them built."""
+    k, n = 300, 300 * length
+    v = np.arange(n, dtype=np.int32).reshape(k, length)
+    i, j = v.ravel(), np.roll(v, -1, axis=1).ravel()
+    rng = np.random.Generator(np.random.PCG64(length))
+    c = rng.uniform(0.5, 1.5, size=n).astype(np.float32)
+    c[::length] *= -1.0
+    r, co, w, (rows, cols) = oracle.dcoo_init(i, j, c)
+    for factor in (2.0, 0.5):
+        g = gpu.dual_solver(r, co, w, rows, cols, 5, 5, factor, 2)
+        o = oracle.dual_solver(r, co, w, rows, cols, 5, 5, factor, 2)
+        assert np.array_equal(g[0], o[0]) and np.array_equal(g[1], o[1]) and g[3] == o[3]
+        np.testing.assert_allclose(g[2], o[2], rtol=1e-6, atol=1e-6)
+        assert abs(g[4] - o[4]) <= 1e-9 * max(1.0, abs(o[4]))
+        assert g[4] > np.minimum(w, 0).sum(dtype=np.float64)

@@ -3,15 +3,19 @@
 // After the first contractions a graph has some ten or hundred thousand
 // edges for dozens of rounds.  Stage by stage such a round is 33 launches and
 // 4 host waits, about 0.25 ms whatever its size, most of it launch gaps and
-// 2 us kernels.  Here a round is nine launches whose sizes are read on the
-// device: the host queues several rounds over buffers sized by the graph it
+// 2 us kernels; with searches for cycles of up to five nodes 48 to 59 launches
+// and 18 waits, 0.45 to 0.6 ms.  Here a round is nine to eleven launches (three
+// more where matchings are long) whose sizes are read on the device: the host queues several rounds over buffers sized by the graph it
 // last saw, then reads one small state.  A round that the driver has to
-// handle itself (a conflicted cycle, more than three matching rounds, a
+// handle itself (a conflicted cycle, a matching of more than six rounds, a
 // bucket too large for LDS, the switch to the spanning forest) raises the
-// state's stop word, and the launches queued behind it leave at once.
+// state's stop word, and the launches queued behind it leave at once.  So does
+// the first matching of more than three rounds: from it on six are queued.
 //
-//   k_mid_begin    sums of the matching threshold, 3-cycle test
-//   k_mid_pick x3  best neighbours of matching rounds 0, 1, 2
+//   k_mid_begin    sums of the matching threshold, attractive neighbour lists
+//   k_mid_prune    (cycles of 4 and 5) the lists without their leaves
+//   k_mid_cycles   (rounds with duals) is there a conflicted cycle
+//   k_mid_pick     best neighbours, a launch per matching round (3 or 6)
 //   k_mid_resolve  per round's outcome: matched and representative counts
 //   k_mid_keys     round that ends the matching, labels, row buckets and each
 //                  tile of edges' count per bucket
@@ -27,11 +31,13 @@
 // Bound by each launch's chain of dependent loads (0.5 to 1 us each: what the
 // launch before wrote comes from memory, not from this XCD's L2), hence the
 // merged launches and the loads issued together.  Measured per round of
-// 20k to 200k edges: about 60 us on the device (picks 3 x 6.4, bucket 10.6,
-// keys 10, scatter 8, finish 6, resolve and begin 3.6 each) against 220 to
-// 320 us stage by stage.  Solves: 1024x2048 grid with long-range edges P
-// 20.2 -> 15.6 ms, PD 55.2 -> 49.5; 257x509 PD 18.7 -> 15.2.  Up to 2^18 edges,
-// the lists whose contraction leaves the symmetric CSR.
+// 20k to 200k edges: about 60 us on the device (picks 3 x 5.3, bucket 11,
+// keys 12, scatter 9, begin 7, finish 6, resolve and prune 4.6 each, cycles 4 to
+// 20, up to 90 where hubs are many) against 220 to 320 us stage by stage, 450 to
+// 600 with cycles of up to five nodes.  Solves: 1024x2048 grid with long-range
+// edges P 20.2 -> 15.6 ms, PD 55.2 -> 46.9; 257x509 PD 18.7 -> 14.3; 71^3 grid PD+
+// 31.8 -> 24.3; rounds of 7k to 2k edges of a 187x211 grid PD+ 1.85 -> 0.54.  Up
+// to 2^18 edges, the lists whose contraction leaves the symmetric CSR.
 //
 // Every sum and order is the stage-by-stage path's, so are the results.
 #include "rama_internal.hpp"
@@ -46,7 +52,8 @@ constexpr int kMidWaves = kMidThreads / 64;
 constexpr int kMidEdgeItems = kMidTileEdges / kMidThreads;
 constexpr int kMidItems = 16;         // sorted items per thread at most
 constexpr int kMidBucketMax = kMidThreads * kMidItems;
-constexpr int kMidPicks = 3;          // matching rounds queued per contraction round
+constexpr int kMidPicks = 6;          // matching rounds queued per contraction round at most
+constexpr int kMidFewPicks = 3;       // and at first
 constexpr int kMidVertBlocks = kMidMaxNodes / kBlock;
 constexpr int kMidGrid = 1024;        // grid bound of the strided launches
 
@@ -81,8 +88,13 @@ struct MidArgs {
     float* hval;
     int* bstat;                   // 256 x 8: entries, forward entries, largest row, col, kept col, bad, min (bits)
     int* label;
+    int* pos;                     // attractive neighbours, from each row's offset on
+    int* npos;                    // and how many
+    int* npath;                   // and how many of them a path can pass through
     int n0;
-    int duals;
+    int picks;                    // matching rounds queued
+    int len;                      // longest conflicted cycles looked for (0: none)
+    int small_words;              // hand over from this many words of bit matrix down
     int small_edges;              // hand over to small_rounds from this many edges down (0: never)
     float mult, ratio, tol;
 };
@@ -104,15 +116,54 @@ __device__ __forceinline__ u64 mid_pack(u32 lo, u32 hi, u32 blo, u32 bhi) {
 }
 static_assert(kMidMaxNodes <= 1 << 18, "labels in mid_pack");
 
-// Threshold partials in reduce_pair_to's blocks and order, and the 3-cycle
-// test: a repulsive edge's ends with a common attractive neighbour (lanes
-// take the shorter row's entries and search the longer row).
+// Per row v of the present graph: the entries l in [off[v], end(v)) that keep
+// accepts, as get(l), in order from the row's offset on in pos, their number in
+// count[v].  A group of lanes per row, a wave per long row; get may read pos.
+template <class Keep, class Get, class End>
+__device__ __forceinline__ void mid_compact(const MidArgs& a, int n, int* count, Keep keep, Get get, End end) {
+    constexpr int kLong = 16 * kMidGroup;
+    const int lane = lane_id(), sub = lane % kMidGroup, first = lane - sub;
+    const unsigned long long lt = (1ull << lane) - 1ull;
+    const unsigned long long group = ((1ull << kMidGroup) - 1ull) << first;
+    const int stride = (int)gridDim.x * (kBlock / kMidGroup);
+    for (int v0 = ((int)xcd_block() * (kBlock / 64) + (threadIdx.x >> 6)) * (64 / kMidGroup); v0 < n; v0 += stride) {
+        const int v = v0 + lane / kMidGroup;
+        const int b0 = v < n ? a.g.off[v] : 0, e0 = v < n ? end(v) : 0;
+        const bool big = e0 - b0 > kLong;
+        int k = 0;
+        for (int l = b0 + sub; !big && l - sub < e0; l += kMidGroup) {  // uniform per group
+            const bool on = l < e0 && keep(l);
+            const int x = on ? get(l) : 0;
+            const unsigned long long m = __ballot(on) & group;
+            if (on) a.pos[b0 + k + __popcll(m & lt)] = x;
+            k += __popcll(m);
+        }
+        if (sub == 0 && v < n && !big) count[v] = k;
+        for (unsigned long long rows = __ballot(sub == 0 && big); rows; rows &= rows - 1ull) {
+            const int src = __ffsll(rows) - 1;
+            const int rb = __shfl(b0, src, 64), re = __shfl(e0, src, 64);
+            int q = 0;
+            for (int l = rb + lane; l - lane < re; l += 64) {
+                const bool on = l < re && keep(l);
+                const int x = on ? get(l) : 0;
+                const unsigned long long m = __ballot(on);
+                if (on) a.pos[rb + q + __popcll(m & lt)] = x;
+                q += __popcll(m);
+            }
+            if (lane == src) count[v] = q;
+        }
+    }
+}
+
+// Threshold partials in reduce_pair_to's blocks and order, and each row's
+// attractive neighbours, in order from the row's offset on: a group of lanes
+// per row, a wave per long row.
 __global__ __launch_bounds__(kBlock) void k_mid_begin(MidArgs a) {
     __shared__ double ws[kWaves];
     __shared__ int wi[kWaves];
-    MidState* st = a.st;
+    const MidState* st = a.st;
     if (st->stop) return;
-    const int nnz = 2 * st->nf, nf = st->nf;
+    const int nnz = 2 * st->nf, n = st->n;
     const int nb = min((nnz + kBlock - 1) / kBlock, (int)kReduceMaxBlocks);
     if ((int)blockIdx.x < nb) {  // uniform per block; the grid covers nb
         double s = 0.0;
@@ -129,40 +180,135 @@ __global__ __launch_bounds__(kBlock) void k_mid_begin(MidArgs a) {
             a.pcnt[blockIdx.x] = rc;
         }
     }
-    if (!a.duals || st->iter == 0) return;
-    const float t = st->minw * a.tol, at = -1.0f * t;
-    const int sub = threadIdx.x % kMidGroup;
-    const int stride = (int)gridDim.x * (kBlock / kMidGroup);
-    for (int e = (int)xcd_block() * (kBlock / kMidGroup) + threadIdx.x / kMidGroup; e < nf; e += stride) {
-        if (!(a.g.val[e] < t)) continue;
-        const int u = a.g.row[e], v = a.g.col[e];
-        int s0 = a.g.off[u], s1 = a.g.off[u + 1], l0 = a.g.off[v], l1 = a.g.off[v + 1];
-        if (s1 - s0 > l1 - l0) {
-            int x = s0;
-            s0 = l0;
-            l0 = x;
-            x = s1;
-            s1 = l1;
-            l1 = x;
-        }
-        for (int i = s0 + sub; i < s1; i += kMidGroup) {
-            if (!(a.g.w[i] > at)) continue;
-            const int m = a.g.adj[i];
-            int lo = l0, hi = l1;
-            while (lo < hi) {
-                const int mid = (lo + hi) >> 1;
-                if (a.g.adj[mid] < m) lo = mid + 1; else hi = mid;
-            }
-            if (lo < l1 && a.g.adj[lo] == m && a.g.w[lo] > at) st->found = 1;
-        }
-    }
+    if (a.len == 0) return;
+    const float at = -1.0f * (st->minw * a.tol);
+    mid_compact(
+        a, n, a.npos, [&](int l) { return a.g.w[l] > at; }, [&](int l) { return a.g.adj[l]; },
+        [&](int v) { return a.g.off[v + 1]; });
 }
 
-// Matching round T's best neighbours (k_pick_best's choice: strongest
+// An attractive path from u to v passes only through vertices with two
+// attractive neighbours.  In late rounds most have one: stars remain, of which
+// a matching contracts one leaf each.  Without the leaves the lists are one or
+// two entries long (k_mid_cycles with them: 123 us a round of the 71^3 grid).
+__global__ __launch_bounds__(kBlock) void k_mid_prune(MidArgs a) {
+    const MidState* st = a.st;
+    if (st->stop) return;
+    mid_compact(
+        a, st->n, a.npath, [&](int l) { return a.npos[a.pos[l]] > 1; }, [&](int l) { return a.pos[l]; },
+        [&](int v) { return a.g.off[v] + a.npos[v]; });
+}
+
+// Is x in the ascending list p[0..n)?
+__device__ __forceinline__ bool mid_has(const int* __restrict__ p, int n, int x) {
+    int lo = 0, hi = n;
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (p[mid] < x) lo = mid + 1; else hi = mid;
+    }
+    return lo < n && p[lo] == x;
+}
+
+// Is there an attractive path of at most len - 1 edges between u and v, whose
+// lists of neighbours to pass through have nu and nv entries?  kLanes lanes
+// take the pairs of neighbours (x, y), one each or, of few pairs, a part of
+// their lists, and ask for x = y, x next to y, a common neighbour.
+template <int kLanes>
+__device__ __forceinline__ bool mid_joined(const MidArgs& a, const int* num, int u, int v, int nu, int nv, int sub) {
+    const int* off = a.g.off;
+    const int* pu = a.pos + off[u];
+    const int* pv = a.pos + off[v];
+    const int pairs = nu * nv, lanes = pairs * 2 > kLanes ? 1 : (pairs * 4 > kLanes ? 2 : (pairs * 8 > kLanes ? 4 : 8));
+    const int p0 = sub / lanes, step = kLanes / lanes, k0 = sub % lanes;
+    int x = p0 / nv, y = p0 % nv;
+    const int dx = step / nv, dy = step % nv;
+    while (x < nu) {
+        const int vx = pu[x], vy = pv[y];
+        const int* px = a.pos + off[vx];
+        const int* py = a.pos + off[vy];
+        int nx = num[vx], ny = num[vy];
+        int z = vy;  // looked for in x's list
+        if (nx > ny) {
+            const int* p = px;
+            px = py;
+            py = p;
+            const int k = nx;
+            nx = ny;
+            ny = k;
+            z = vx;
+        }
+        bool hit = vx == vy;
+        for (int k = k0; k < nx; k += lanes) {
+            const int q = px[k];
+            hit |= q == z || (a.len > 4 && mid_has(py, ny, q));
+        }
+        if (hit) return true;
+        x += dx;
+        y += dy;
+        if (y >= nv) {
+            y -= nv;
+            ++x;
+        }
+    }
+    return false;
+}
+
+// Are a repulsive edge's ends joined by an attractive path of at most len - 1
+// edges?  A conflicted cycle exists exactly then: the shortest such path has
+// no chord.  A group of lanes per edge, the wave for one with many pairs of
+// neighbours.
+//
+// In the rounds that get here (the search before found nothing) that is one or
+// two pairs per edge, of two or three neighbours each: bound by the chain of
+// six loads, hence a group for every edge (groups that take eight edges in
+// turn: 80 us at 7k edges), and by the few edges between hubs.
+__global__ __launch_bounds__(kBlock) void k_mid_cycles(MidArgs a) {
+    MidState* st = a.st;
+    if (st->stop) return;
+    constexpr int kMany = 4 * kMidGroup;  // pairs
+    const int nf = st->nf, lane = lane_id(), sub = lane % kMidGroup;
+    const float t = st->minw * a.tol;
+    const int* off = a.g.off;
+    const int* num = a.len > 3 ? a.npath : a.npos;  // of the lists to walk
+    const int stride = (int)gridDim.x * (kBlock / kMidGroup);
+    bool hit = false;
+    for (int e0 = ((int)xcd_block() * kWaves + (threadIdx.x >> 6)) * (64 / kMidGroup); e0 < nf; e0 += stride) {
+        const int e = e0 + lane / kMidGroup;
+        int u = 0, v = 0, nu = 0, nv = 0;
+        if (e < nf) {
+            const float c = a.g.val[e];
+            u = a.g.row[e];
+            v = a.g.col[e];
+            if (c < t) {
+                nu = num[u];
+                nv = num[v];
+            }
+        }
+        const bool on = nu > 0 && nv > 0;
+        const bool many = on && a.len > 3 && (float)nu * (float)nv > (float)kMany;
+        if (on && a.len == 3) {
+            // the shorter list's entries in the longer list
+            const int* ps = a.pos + off[nu < nv ? u : v];
+            const int* pl = a.pos + off[nu < nv ? v : u];
+            for (int k = sub; k < min(nu, nv); k += kMidGroup) hit |= mid_has(pl, max(nu, nv), ps[k]);
+        } else if (on && !many) {
+            hit = mid_joined<kMidGroup>(a, num, u, v, nu, nv, sub);
+        }
+        for (unsigned long long rest = __ballot(many && sub == 0); rest && !__any(hit); rest &= rest - 1ull) {
+            const int src = __ffsll(rest) - 1;
+            hit = mid_joined<64>(a, num, __shfl(u, src, 64), __shfl(v, src, 64), __shfl(nu, src, 64),
+                                 __shfl(nv, src, 64), lane);
+        }
+        if (__any(hit) || __hip_atomic_load(&st->found, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) break;
+    }
+    if (__any(hit) && lane == 0) __hip_atomic_store(&st->found, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Matching round t's best neighbours (k_pick_best's choice: strongest
 // unmatched neighbour above the threshold, first in row order on ties) on
-// round T - 1's outcome.  Round 0 combines the threshold first.
-template <int T>
-__global__ __launch_bounds__(kBlock) void k_mid_pick(MidArgs a) {
+// round t - 1's outcome.  Round 0 combines the threshold first.
+template <bool kFirst>
+__global__ __launch_bounds__(kBlock) void k_mid_pick(MidArgs a, int t) {
     __shared__ double ws[kWaves];
     __shared__ int wi[kWaves];
     MidState* st = a.st;
@@ -170,7 +316,7 @@ __global__ __launch_bounds__(kBlock) void k_mid_pick(MidArgs a) {
     const int n = st->n;
     float thr;
     bool any;
-    if (T == 0) {
+    if (kFirst) {
         const int nnz = 2 * st->nf;
         const int nb = min((nnz + kBlock - 1) / kBlock, (int)kReduceMaxBlocks);
         const double sum = combine_partials(a.psum, (unsigned)nb, 0.0, OpSum(), ws);
@@ -185,14 +331,14 @@ __global__ __launch_bounds__(kBlock) void k_mid_pick(MidArgs a) {
         thr = st->thr;
         any = st->any != 0;
     }
-    const int* prev = T > 0 ? a.best[T > 0 ? T - 1 : 0] : nullptr;
-    int* best = a.best[T];
+    const int* prev = !kFirst ? a.best[t - 1] : nullptr;
+    int* best = a.best[t];
     const int sub = threadIdx.x % kMidGroup;
     const int stride = (int)gridDim.x * (kBlock / kMidGroup);
     for (int v = (int)xcd_block() * (kBlock / kMidGroup) + threadIdx.x / kMidGroup; v < n; v += stride) {
         const int b0 = a.g.off[v], e0 = a.g.off[v + 1];
         int pb = -1;
-        if (T > 0) {
+        if (!kFirst) {
             pb = prev[v];
             if (pb >= 0 && prev[pb] != v) pb = -1;  // not matched
         }
@@ -203,7 +349,7 @@ __global__ __launch_bounds__(kBlock) void k_mid_pick(MidArgs a) {
             const float c = a.g.w[l];
             const int u = a.g.adj[l];
             if (!(c > bv) || u == v) continue;
-            if (T > 0) {
+            if (!kFirst) {
                 const int pu = prev[u];
                 if (pu >= 0 && prev[pu] == u) continue;  // matched
             }
@@ -238,6 +384,7 @@ __global__ __launch_bounds__(kBlock) void k_mid_resolve(MidArgs a) {
     const int w = threadIdx.x >> 6;
 #pragma unroll
     for (int t = 0; t < kMidPicks; ++t) {
+        if (t >= a.picks) break;
         const int b = v < n ? a.best[t][v] : -1;
         const bool m = b >= 0 && a.best[t][b] == v;
         const unsigned long long reps = __ballot(v < n && !(m && b < v));
@@ -249,7 +396,7 @@ __global__ __launch_bounds__(kBlock) void k_mid_resolve(MidArgs a) {
         }
     }
     __syncthreads();
-    if (threadIdx.x < kMidPicks) {
+    if ((int)threadIdx.x < a.picks) {
         int r = 0, m = 0;
 #pragma unroll
         for (int k = 0; k < kWaves; ++k) {
@@ -314,8 +461,9 @@ __global__ __launch_bounds__(kMidThreads) void k_mid_keys(MidArgs a) {
 #pragma unroll
         for (int k = 0; k < kPer; ++k) {
             const int b = tid * kPer + k;
-            rc[t][k] = b < nblk ? a.rcnt[t][b] : 0;
-            mc[t] += b < nblk ? a.mcnt[t][b] : 0;
+            const bool on = t < a.picks && b < nblk;
+            rc[t][k] = on ? a.rcnt[t][b] : 0;
+            mc[t] += on ? a.mcnt[t][b] : 0;
         }
     }
 #pragma unroll
@@ -326,11 +474,11 @@ __global__ __launch_bounds__(kMidThreads) void k_mid_keys(MidArgs a) {
     }
     if (tid < 256) hist[tid] = 0;
     __syncthreads();
-    int tr = kMidPicks - 1, matched = 0;
+    int tr = 0, matched = 0;
     bool ended = false;
 #pragma unroll
     for (int t = 0; t < kMidPicks; ++t) {
-        if (ended) break;  // uniform
+        if (ended || t >= a.picks) break;  // uniform
         int cur = 0;
 #pragma unroll
         for (int k = 0; k < kMidWaves; ++k) cur += cnt[t][k];
@@ -351,7 +499,9 @@ __global__ __launch_bounds__(kMidThreads) void k_mid_keys(MidArgs a) {
         int x[kPer], s = 0;
 #pragma unroll
         for (int k = 0; k < kPer; ++k) {
-            x[k] = tr == 0 ? rc[0][k] : (tr == 1 ? rc[1][k] : rc[2][k]);
+            x[k] = rc[0][k];
+#pragma unroll
+            for (int t = 1; t < kMidPicks; ++t) x[k] = tr == t ? rc[t][k] : x[k];
             s += x[k];
         }
         int run = mid_block_scan(s, ws, &reps);
@@ -809,7 +959,9 @@ __global__ __launch_bounds__(kBlock) void k_mid_finish(MidArgs a) {
         x.stop = bad ? kSmallBad
                      : (ftot == 0 ? kSmallDone
                                   : (cross ? kSmallForest
-                                           : (ftot <= a.small_edges && top <= kSmallMaxNodes ? kMidSmall : 0)));
+                                           : (ftot <= a.small_edges && top <= kSmallMaxNodes && x.n * ((x.n + 31) / 32) <= a.small_words
+                                                  ? kMidSmall
+                                                  : 0)));
         *a.nx = x;
         if (a.mirror) *a.mirror = x;
     }
@@ -818,7 +970,7 @@ __global__ __launch_bounds__(kBlock) void k_mid_finish(MidArgs a) {
 bool mid_rounds_fit(const DCoo& A, const Options& o) {
     const int n = A.max_node + 1;
     const int len = o.num_dual_itr_primal == 0 ? 0 : o.max_cycle_length_primal;
-    return n >= 2 && A.max_dim() <= kMidMaxNodes && A.nnz <= kMidMaxEdges && len <= 3 && A.sym &&
+    return n >= 2 && A.max_dim() <= kMidMaxNodes && A.nnz <= kMidMaxEdges && len <= 5 && A.sym &&
            A.sym->n >= n && tune::get(tune::MidRounds, A.nnz) != 0;
 }
 
@@ -875,7 +1027,17 @@ MidState mid_rounds(Ctx& ctx, DCoo& A, const Options& o, int iter, int first, in
     a.bstat = bstat.get();
     a.label = lab.get();
     a.n0 = n0;
-    a.duals = o.num_dual_itr_primal != 0 && o.max_cycle_length_primal >= 3 ? 1 : 0;
+    a.picks = kMidFewPicks;
+    a.len = o.num_dual_itr_primal != 0 && o.max_cycle_length_primal >= 3 ? o.max_cycle_length_primal : 0;
+    DBuf<int> pos, npos;
+    if (a.len) {
+        pos = ctx.buf<int>(2 * nf0);
+        npos = ctx.buf<int>(2 * (i64)n0);
+        a.pos = pos.get();
+        a.npos = npos.get();
+        a.npath = a.npos + n0;
+    }
+    a.small_words = a.len > 3 ? kSmallBitWords : 0x7fffffff;  // small_rounds_fit's limit
     a.small_edges = tune::get(tune::SmallRounds, kSmallMaxEdges) ? kSmallMaxEdges : 0;
     a.mult = o.mean_multiplier_mm;
     a.ratio = o.matching_thresh_crossover_ratio;
@@ -890,7 +1052,7 @@ MidState mid_rounds(Ctx& ctx, DCoo& A, const Options& o, int iter, int first, in
             L[v] = (int)v;
             if (v == 0) *s0 = init;
         });
-        if (a.duals)
+        if (a.len)
             reduce_to<float>(ctx, [=] __device__(i64 e) { return W[e]; }, nf0, 3.402823466e38f, OpMin(), &s0->minw);
     }
     MidState h{};
@@ -901,7 +1063,8 @@ MidState mid_rounds(Ctx& ctx, DCoo& A, const Options& o, int iter, int first, in
     for (int batch = first;; batch = std::min(2 * batch, 16)) {
         const unsigned ntiles = (unsigned)((h.nf + kMidTileEdges - 1) / kMidTileEdges);
         const unsigned gb = (unsigned)std::min<i64>(
-            std::max<i64>((2 * (i64)h.nf + kBlock - 1) / kBlock, ((i64)h.nf * kMidGroup + kBlock - 1) / kBlock), kMidGrid);
+            std::max<i64>((2 * (i64)h.nf + kBlock - 1) / kBlock, ((i64)h.n * kMidGroup + kBlock - 1) / kBlock), kMidGrid);
+        const unsigned gc = (unsigned)std::min<i64>(((i64)h.nf * kMidGroup + kBlock - 1) / kBlock, 2 * kMidGrid);
         const unsigned gp = (unsigned)std::min<i64>(((i64)h.n * kMidGroup + kBlock - 1) / kBlock, kMidGrid);
         const unsigned gr = (unsigned)((h.n + kBlock - 1) / kBlock);
         const unsigned gk = std::max(ntiles, 1u);
@@ -914,12 +1077,20 @@ MidState mid_rounds(Ctx& ctx, DCoo& A, const Options& o, int iter, int first, in
             prof::Scope ps(ctx, "mid_round", 0.0);
             k_mid_begin<<<gb, kBlock, 0, ctx.stream>>>(a);
             RAMA_LAUNCHED();
-            k_mid_pick<0><<<gp, kBlock, 0, ctx.stream>>>(a);
+            if (a.len > 3) {
+                k_mid_prune<<<gp, kBlock, 0, ctx.stream>>>(a);
+                RAMA_LAUNCHED();
+            }
+            if (a.len) {
+                k_mid_cycles<<<gc, kBlock, 0, ctx.stream>>>(a);
+                RAMA_LAUNCHED();
+            }
+            k_mid_pick<true><<<gp, kBlock, 0, ctx.stream>>>(a, 0);
             RAMA_LAUNCHED();
-            k_mid_pick<1><<<gp, kBlock, 0, ctx.stream>>>(a);
-            RAMA_LAUNCHED();
-            k_mid_pick<2><<<gp, kBlock, 0, ctx.stream>>>(a);
-            RAMA_LAUNCHED();
+            for (int t = 1; t < a.picks; ++t) {
+                k_mid_pick<false><<<gp, kBlock, 0, ctx.stream>>>(a, t);
+                RAMA_LAUNCHED();
+            }
             k_mid_resolve<<<gr, kBlock, 0, ctx.stream>>>(a);
             RAMA_LAUNCHED();
             k_mid_keys<<<gk, kMidThreads, 0, ctx.stream>>>(a);
@@ -932,6 +1103,19 @@ MidState mid_rounds(Ctx& ctx, DCoo& A, const Options& o, int iter, int first, in
             RAMA_LAUNCHED();
         }
         ctx.read_mirror(states.get() + (queued & 1), ctx.mirror<MidState>(), &h);
+        if (h.stop == kMidMatching && a.picks < kMidPicks) {
+            // queue this round again with more matching rounds, and the ones after it
+            a.picks = kMidPicks;
+            const MidState* from = states.get() + (queued & 1);
+            queued = h.rounds;  // parity of the set that holds the graph
+            MidState* s = states.get() + (queued & 1);
+            for_each(ctx, 1, [=] __device__(i64) {
+                MidState x = *from;
+                x.stop = 0;
+                *s = x;
+            });
+            continue;
+        }
         if (h.stop) break;
     }
     map_node_labels(ctx, lab.get(), n0, labels, num_labels);

@@ -64,3 +64,42 @@ def test_queued_equals_stages(gpu, table, kind, preset):
             except gpu.RamaError as e:
                 got.append(str(e))
         assert got[0] == got[1], "kind %s seed %d" % (kind, seed)
+
+
+def _rings(seed):
+    """Attractive rings of 9 to 40 nodes with one repulsive edge, joined to
+    two hubs: contraction shortens the conflicted cycles round by round."""
+    rng = np.random.default_rng(seed)
+    i, j, c = [], [], []
+    base = 2
+    for length in rng.integers(9, 41, size=500):
+        v = base + np.arange(length)
+        w = rng.uniform(0.1, 1.0, size=length)
+        w[0] *= -1.0
+        i.append(v), j.append(np.roll(v, -1)), c.append(w)
+        hub = rng.integers(0, 2, size=2)
+        i.append(hub), j.append(rng.choice(v, 2, replace=False)), c.append(rng.normal(-0.2, 0.3, size=2))
+        base += length
+    i, j = np.concatenate(i), np.concatenate(j)
+    perm = rng.permutation(base)  # ids in no order
+    i, j = perm[i], perm[j]
+    return np.minimum(i, j).astype(np.int32), np.maximum(i, j).astype(np.int32), np.concatenate(c).astype(np.float32)
+
+
+@pytest.mark.parametrize("length", [3, 4, 5])
+@pytest.mark.parametrize("kind", ["rings", "grid_long", "grid3d", "limit", "sparse", "dense", "hub", "hubs", "ties"])
+def test_queued_longer_cycles(gpu, table, kind, length):
+    for seed in range(2):
+        i, j, c = _rings(seed) if kind == "rings" else _instance(kind, seed)
+        opts = gpu.options("PD+", verbose=0)
+        opts.max_cycle_length_primal = length
+        got = []
+        for on in (1, 0):
+            assert table.rama_tuning_set(b"mid_rounds", 1 << 18, on) == 0
+            assert table.rama_tuning_set(b"small_rounds", 4096, on and seed) == 0
+            try:
+                labels, lb, _, _ = gpu.solve(i, j, c, opts)
+                got.append((labels.tolist(), lb))
+            except gpu.RamaError as e:
+                got.append(str(e))
+        assert got[0] == got[1], "kind %s seed %d" % (kind, seed)

@@ -50,19 +50,20 @@ struct CycArgs {
     // end of the expansions they covered ([1], a maximum).
     unsigned blk0 = 0;
     i64* counted = nullptr;
-    // diagnostic (RAMA_CYCLE_STATS): threads of the 5-cycle count, and those
-    // that counted through a 2-hop table
-    unsigned long long* stats = nullptr;
-    // 5-cycle count: node ids fit the 2-hop tables' keys (below kT5MaxNode)
-    int tables = 0;
-    // 4-cycle count: wave-wide counting of long lists allowed
-    int wide4 = 1;
+    // 4- and 5-cycle counts: 1 if entries are looked up in the 2-hop sets, 0 if
+    // all are resolved; the queue of entries to resolve (kQueueParts parts of
+    // qcap entries), its counters 128 bytes apart
+    int sets = 1;
+    int qcap = 0;
+    int3* queue = nullptr;
+    unsigned* qcount = nullptr;
+    int2* wide = nullptr;  // rep edges left to the wide kernel (first, number), count behind qcount's parts
 };
 
 // Diagnostic switches (tests force each path on the same inputs; every
 // path gives the same counts and triangles):
-//   RAMA_CYCLE_TABLES=0   no 2-hop tables (5-cycles) and no wave-wide sets
-//                         (4-cycles): every expansion counted by its thread
+//   RAMA_CYCLE_TABLES=0   4- and 5-cycle counts without the 2-hop sets: every
+//                         list entry resolved against the lists
 //   RAMA_EMIT_FORM=dense | queue   the emit form, instead of the choice by
 //                         the share of expansions with mids
 static bool cycle_tables_on() {
@@ -232,23 +233,6 @@ __device__ __forceinline__ int probe_count(const int* __restrict__ adj, int sb, 
     return c;
 }
 
-// count_common of the lists [ia, ie) and [ib, ib + nb) by one lane: from
-// the shorter list by binary searches when the pair is heavy and that list
-// is short, else the merge walk.
-__device__ __forceinline__ int lane_count_common(const int* __restrict__ adj, int ia, int ie, int ib, int nb) {
-    const int na = ie - ia;
-    if (na + nb > kHeavy && min(na, nb) <= kProbe)
-        return na <= nb ? probe_count(adj, ia, ie, ib, ib + nb) : probe_count(adj, ib, ib + nb, ia, ie);
-    int i = ia, j = ib, je = ib + nb, c = 0;
-    while (i < ie && j < je) {
-        const int x = adj[i], y = adj[j];
-        c += (x == y);
-        i += (x <= y);
-        j += (y <= x);
-    }
-    return c;
-}
-
 // count_common by the whole wave (qa, qb wave-uniform): each lane takes
 // entries of the shorter list and binary-searches the longer one.
 __device__ __forceinline__ int wave_count_common(const int* __restrict__ off, const int* __restrict__ adj, int qa,
@@ -354,26 +338,6 @@ __device__ __forceinline__ void reg_list_props(const int (&rb)[kRegList], int nb
     }
 }
 
-// Adds `v` to the total of the tile holding expansion x, flushing the
-// running sum whenever the thread's expansions cross into the next tile.
-struct TileAcc {
-    i64 tile = -1;
-    i64 sum = 0;
-    __device__ __forceinline__ void add(i64* tot, i64 x, i64 v) {
-        const i64 t = x / kCycTile;
-        if (t != tile) {
-            flush(tot);
-            tile = t;
-        }
-        sum += v;
-    }
-    __device__ __forceinline__ void flush(i64* tot) {
-        if (tile >= 0 && sum != 0)
-            atomicAdd(reinterpret_cast<unsigned long long*>(tot + tile), (unsigned long long)sum);
-        sum = 0;
-    }
-};
-
 // 3-cycles: one thread per repulsive edge r = expansion r; N(v2) in
 // registers, N(v1) streamed.  Tile totals by block reduction.
 __global__ __launch_bounds__(kBlock) void k_cycle_count3(CycArgs a, unsigned char* __restrict__ cnt8,
@@ -419,489 +383,496 @@ __global__ __launch_bounds__(kBlock) void k_cycle_count3(CycArgs a, unsigned cha
     if (threadIdx.x == 0) tile_tot[blk] = tot;
 }
 
-// 4-cycles: one thread per repulsive edge; its expansions n1 ∈ N(v1) are
-// xoff[r] .. xoff[r+1]-1 in order, each intersecting N(n1) with N(v2)
-// (held in registers).  tile_tot must be zero on entry.
-// Rep edges whose v1 has at least kWideRep neighbours, or whose v2 has more
-// than kRegList, are counted by the whole wave, one rep edge at a time: the
-// wave puts N(v2) in an LDS hash set (kSetSlots slots, lists of at most
-// kSetMax entries) and lane l takes expansions l, l + 64, ..., streaming
-// N(n1) and probing each entry.  After contraction supernodes have dozens
-// of neighbours: one lane per rep edge would walk long merge walks serially
-// while its wave waits.  A repeated value in either list (the min(a, b)
-// rule) or a longer N(v2) keeps the merge walk for that expansion.
-constexpr int kWideRep = 48;
-constexpr int kSetSlots = 256;
-constexpr int kSetMax = 128;
-
-__device__ __forceinline__ int set_hash(int m) { return (int)(((unsigned)m * 2654435761u) >> 24); }
-
-__global__ __launch_bounds__(kBlock) void k_cycle_count4(CycArgs a, unsigned char* __restrict__ cnt8,
-                                                         i64* __restrict__ tile_tot) {
-    __shared__ int wset[kWaves][4 * kSetSlots];
-    const int w = threadIdx.x >> 6;
-    const i64 r = (i64)(a.blk0 + xcd_block()) * kBlock + threadIdx.x;
-    const bool on = r < a.R;
-    i64 mine = 0, xend = 0;
-    int v1 = 0, v2 = 0, b1 = 0, d1 = 0, b2 = 0, n2 = 0;
-    i64 x0 = 0;
-    if (on) {
-        v1 = a.rv1[r];
-        v2 = a.rv2[r];
-        b1 = a.off[v1];
-        d1 = a.off[v1 + 1] - b1;
-        b2 = a.off[v2];
-        n2 = a.off[v2 + 1] - b2;
-        x0 = a.xoff[r];
-        xend = x0 + d1;
-    }
-    const bool wide = on && a.wide4 && (d1 >= kWideRep || n2 > kRegList);
-    if (on && !wide) {
-        int rb[kRegList];
-        const bool regs = n2 <= kRegList;
-        int rmax = -1, kw = kRegList;
-        bool rdup = false;
-        if (regs) {
-            load_reg_list(a.adj, b2, n2, rb);
-            reg_list_props(rb, n2, rmax, rdup);
-            kw = reg_width(n2);
-        }
-        TileAcc acc;
-        // the next n1's list bounds are loaded while this one is walked
-        int ia = 0, ie = 0;
-        if (d1 > 0) {
-            const int n1 = a.adj[b1];
-            ia = a.off[n1];
-            ie = a.off[n1 + 1];
-        }
-        for (int l = 0; l < d1; ++l) {
-            int na = 0, ne = 0;
-            if (l + 1 < d1) {
-                const int nn = a.adj[b1 + l + 1];
-                na = a.off[nn];
-                ne = a.off[nn + 1];
-            }
-            const int c = regs ? count_vs_regs_fast(a.adj, ia, ie, rb, rmax, rdup, kw)
-                               : lane_count_common(a.adj, ia, ie, b2, n2);
-            cnt8[x0 + l] = (unsigned char)(c < 255 ? c : 255);
-            acc.add(tile_tot, x0 + l, 2 * (i64)c);
-            mine += 2 * (i64)c;
-            ia = na;
-            ie = ne;
-        }
-        acc.flush(tile_tot);
-    }
-    // wide rep edges: the wave works as four groups of 16 lanes, group g
-    // taking the wide rep edges of lanes 16g .. 16g + 15 one after another
-    // (four rep edges in flight per wave); the attempted writes are credited
-    // to the rep's own lane (its instance, its block total)
-    const int lane = lane_id(), g = lane >> 4, gl = lane & 15;
-    const unsigned long long wm = __ballot(wide);
-    unsigned gm = (unsigned)((wm >> (16 * g)) & 0xffffull);  // this group's wide lanes
-    int niter = 0;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) niter = max(niter, __popcll((wm >> (16 * q)) & 0xffffull));
-    int* gset = &wset[w][g * kSetSlots];
-    const unsigned long long gmask = 0xffffull << (16 * g);
-    for (int it = 0; it < niter; ++it) {
-        const bool gact = gm != 0u;  // uniform within the group
-        const int h = gact ? 16 * g + __builtin_ctz(gm) : lane;
-        if (gact) gm &= gm - 1u;
-        const int hb1 = __shfl(b1, h, 64), hd1 = gact ? __shfl(d1, h, 64) : 0;
-        const int hb2 = __shfl(b2, h, 64), hn2 = gact ? __shfl(n2, h, 64) : 0;
-        const i64 hx0 = __shfl(x0, h, 64);
-        // N(v2) into the group's set (a repeated value, or too long a list:
-        // merge walks instead)
-        bool use_set = gact && hn2 <= kSetMax;
-        int vmax = -1;
-        bool dup = false;
-        if (use_set) {
-            for (int k = gl; k < kSetSlots; k += 16) gset[k] = -1;
-        }
-        __builtin_amdgcn_wave_barrier();
-        if (use_set) {
-            for (int k = gl; k < hn2; k += 16) {
-                const int m = a.adj[hb2 + k];
-                dup |= k > 0 && a.adj[hb2 + k - 1] == m;
-                int hs = set_hash(m);
-                while (true) {
-                    const int old = atomicCAS(&gset[hs], -1, m);
-                    if (old == -1 || old == m) break;
-                    hs = (hs + 1) & (kSetSlots - 1);
-                }
-            }
-            vmax = hn2 > 0 ? a.adj[hb2 + hn2 - 1] : -1;
-        }
-        use_set = use_set && (__ballot(dup) & gmask) == 0ull;
-        __builtin_amdgcn_wave_barrier();
-        TileAcc acc;
-        i64 part = 0;
-        for (int l = gl; l < hd1; l += 16) {
-            const int n1 = a.adj[hb1 + l];
-            const int ia = a.off[n1], ie = a.off[n1 + 1];
-            int c = 0;
-            bool merge = !use_set;
-            if (use_set) {
-                // four entries per round of loads (past the end reads as
-                // above vmax), walked in order up to the first above vmax
-                int prev = -1;
-                bool stop = false;
-                for (int k = ia; k < ie && !stop; k += 4) {
-                    int xs[4];
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) xs[u] = k + u < ie ? a.adj[k + u] : 0x7fffffff;
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                        const int x = xs[u];
-                        if (stop || x > vmax) {
-                            stop = true;
-                            continue;
-                        }
-                        if (x == prev) {  // N(n1) repeats a value: the merge walk counts it
-                            merge = true;
-                            stop = true;
-                            continue;
-                        }
-                        prev = x;
-                        int hs = set_hash(x);
-                        while (true) {
-                            const int key = gset[hs];
-                            if (key == x) {
-                                ++c;
-                                break;
-                            }
-                            if (key == -1) break;
-                            hs = (hs + 1) & (kSetSlots - 1);
-                        }
-                    }
-                }
-            }
-            if (merge) c = lane_count_common(a.adj, ia, ie, hb2, hn2);
-            cnt8[hx0 + l] = (unsigned char)(c < 255 ? c : 255);
-            acc.add(tile_tot, hx0 + l, 2 * (i64)c);
-            part += 2 * (i64)c;
-        }
-        acc.flush(tile_tot);
-#pragma unroll
-        for (int d = 8; d >= 1; d >>= 1) part += __shfl_xor(part, d, 64);  // within the group
-        if (gact && lane == h) mine += part;
-        __builtin_amdgcn_wave_barrier();
-    }
-    if (a.nslot) wave_add_keyed(a.slot_total, on ? a.nslot[v1] : 0, mine, on);
-    if (a.counted) block_counted(a.counted, mine, xend);
-}
-
-// 5-cycles: one thread per (repulsive edge r, n2 = l2-th neighbour of v2);
-// its expansions (n1 = l1-th neighbour of v1, n2) are xoff[r] + l2*d1 + l1
-// for l1 = 0 .. d1-1, each intersecting N(n1) with N(n2); n1 == n2 is
-// skipped.  Threads of rep r are yoff[r] .. yoff[r+1]-1; ytile_rep gives
-// each block's first rep.  tile_tot must be zero on entry.
+// 4- and 5-cycles.  Expansions of rep edge r = (v1, v2) are xoff[r] ..
+// xoff[r+1]-1: for 4-cycles the neighbours n1 of v1 (l1 = 0 .. d1-1), each
+// intersecting N(n1) with N(v2); for 5-cycles the pairs (n1, n2) at
+// l2 * d1 + l1, each intersecting N(n1) with N(n2), n1 == n2 left out.
 //
-// Two ways to count one thread's d1 expansions, with identical counts:
-//  * 2-hop table (the common case): the block builds, for each distinct v1
-//    among its threads, an LDS hash table of v1's 2-hop neighbourhood,
-//    mid -> bitmask of the l1 whose list N(n1) holds mid.  The thread then
-//    walks N(n2) once, looks every mid up and adds its mask to bit-sliced
-//    per-l1 counters, instead of streaming every N(n1) against N(n2).  Valid
-//    when no list involved holds a value twice (then |N(n1) ∩ N(n2)| is the
-//    merge walk's min(a, b) count), d1 <= 32 and the 2-hop lists fit.
-//  * per expansion (otherwise): N(n2) in registers (or the merge walk /
-//    probes for long lists), each N(n1) streamed against it.
-constexpr int kT5Tables = 16;      // 2-hop tables (distinct v1 runs) per block
-constexpr int kT5SlotBits = 11;
-constexpr int kT5Slots = 1 << kT5SlotBits;  // slots of the block's shared hash table
-constexpr int kT5MaxFill = 1536;   // entries of all tables together at most this (load <= 3/4)
-constexpr int kT5MaxD1 = 32;       // d(v1) at most this (32-bit masks)
-constexpr int kT5RepWin = 256;     // rep edges a block locates its threads among in LDS
-constexpr int kT5MaxNode = 1 << 27;  // node ids below this: (mid, run) fits one key
+// Nearly all of these intersections are empty, so the lists are not walked
+// against each other.  Rep edges lie in row order, those of one v1 are a run.
+// A group of 16 lanes takes a run, marks the 2-hop neighbourhood of v1 (every
+// entry of every N(n1)) in a set of bits in LDS, and looks up, for each rep
+// edge of the run, the entries of N(v2) (4-cycles) or of every N(n2)
+// (5-cycles): ten entries of one list instead of a hundred of ten lists.
+// Entries that pass are queued, first per wave, then in memory, and a second
+// launch resolves them against the lists themselves, a lane each: an entry m
+// belongs to expansion l1 if n1 is in N(m).  So the counts are exact whatever
+// the set lets through, and the few rep edges with most of the cycles (chords
+// gather on some vertices) are shared by the whole chip.
+//
+// A set is words of 32 bits, three bits of one word marked per entry: one LDS
+// read per look-up, about one entry in two hundred passes by accident (146
+// entries marked on average in the 2D grid).  Runs of hubs (more than
+// kSetLists lists or kSetFill entries) and rep edges whose v2 is one are
+// listed, and a launch of blocks takes a few of them each with a set of
+// kBigWords words.
+//
+// One thread per rep edge walking every N(n1) against N(v2) in registers, or
+// per (rep edge, n2) through per-block hash tables, took 9300 vector
+// instructions per wave and waited on the longest of its lanes' lists.  D mode
+// on the 12.47M-edge grid, all 4- and 5-cycle counts of a solve: 54.5 + 59.7 ms
+// so, 14 + 36 with the sets (a full pass: 9.3M rep edges and 100M expansions
+// 5.0 -> 1.4 ms, 1.1G expansions 11 -> 8.2); the 192^3 grid's PD+ 14.0 + 8.1 ->
+// 11.0 + 7.7.  5-cycles are bound by the lists' load latency at 5 waves per SIMD
+// and by about 60 instructions per step of four lists.
+constexpr int kSetLanes = 16;                  // lanes per run
+constexpr int kSetGroups = kBlock / kSetLanes;
+constexpr int kSetWords = 64;                  // words of a group's set
+constexpr int kBigWords = 2048;                // words of the block's set
+constexpr int kSetLists = 2 * kSetLanes;       // lists of v1 at most
+constexpr int kSetFill = 768;                  // entries marked at most
+constexpr int kSetQueue = 128;                 // waiting entries per wave
+constexpr int kQueueParts = 64;                // of the queue in memory
+constexpr int kSetMinReps = 16;                // rep edges per block, at least and at most
+constexpr int kSetMaxReps = kBlock;
+constexpr int kRunReps = 16;                   // rep edges per run at most: a group takes them in turn
+constexpr int kWideReps = 8;                   // rep edges per entry of the list of hubs' runs
 
-// The tables of a block share one open-addressing hash table of keys
-// mid * kT5Tables + run.
-__device__ __forceinline__ int t5_hash(int key) {
-    return (int)(((unsigned)key * 2654435761u) >> (32 - kT5SlotBits));
+// Word and bits of an entry in a set of 2^kLog words.
+template <int kLog>
+__device__ __forceinline__ unsigned set_bits(int m, unsigned* bits) {
+    const unsigned h = (unsigned)m * 2654435761u;
+    *bits = (1u << ((h >> (27 - kLog)) & 31)) | (1u << ((h >> (22 - kLog)) & 31)) | (1u << ((h >> (17 - kLog)) & 31));
+    return h >> (32 - kLog);
 }
 
-// The per-expansion form for one thread (see above).
-__device__ __forceinline__ void count5_direct(const CycArgs& a, int b1, int d1, int n2, int bq, int nq, i64 x0,
-                                              unsigned char* __restrict__ cnt8, i64* __restrict__ tile_tot,
-                                              i64& mine) {
-    int rb[kRegList];
-    const bool regs = nq <= kRegList;
-    int rmax = -1, kw = kRegList;
-    bool rdup = false;
-    if (regs) {
-        load_reg_list(a.adj, bq, nq, rb);
-        reg_list_props(rb, nq, rmax, rdup);
-        kw = reg_width(nq);
-    }
-    TileAcc acc;
-    // the next n1 and its list bounds are loaded while this one is walked
-    int n1 = d1 > 0 ? a.adj[b1] : 0;
-    int ia = d1 > 0 ? a.off[n1] : 0, ie = d1 > 0 ? a.off[n1 + 1] : 0;
-    for (int l = 0; l < d1; ++l) {
-        const int nn = l + 1 < d1 ? a.adj[b1 + l + 1] : 0;
-        const int na = l + 1 < d1 ? a.off[nn] : 0, ne = l + 1 < d1 ? a.off[nn + 1] : 0;
-        int c = 0;
-        if (n1 != n2)
-            c = regs ? count_vs_regs_fast(a.adj, ia, ie, rb, rmax, rdup, kw)
-                     : lane_count_common(a.adj, ia, ie, bq, nq);
-        cnt8[x0 + l] = (unsigned char)(c < 255 ? c : 255);
-        acc.add(tile_tot, x0 + l, 3 * (i64)c);
-        mine += 3 * (i64)c;
-        n1 = nn;
-        ia = na;
-        ie = ne;
-    }
-    acc.flush(tile_tot);
+// Orders the wave's LDS accesses around it (the lanes of a group share a set).
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-__global__ __launch_bounds__(kBlock) void k_cycle_count5(CycArgs a, const i64* __restrict__ yoff,
-                                                         const int* __restrict__ ytile_rep, i64 Y,
-                                                         unsigned char* __restrict__ cnt8,
-                                                         i64* __restrict__ tile_tot) {
-    __shared__ int tkey[kT5Slots];
-    __shared__ unsigned tmask[kT5Slots];
-    __shared__ int tv1[kT5Tables];
-    __shared__ int tok[kT5Tables];
-    __shared__ int tfill[kT5Tables];
-    __shared__ int sv1[kBlock];
-    __shared__ int wruns[kWaves];
-    const unsigned blk = a.blk0 + xcd_block();
-    const int tid = threadIdx.x, lane = lane_id(), w = tid >> 6;
-    const i64 y = (i64)blk * kCycTile + tid;
-    const bool on = y < Y;
-    i64 mine = 0, xend = 0;
-    int slot = 0;
-    int v1 = -1, b1 = 0, d1 = 0, n2 = 0, bq = 0, nq = 0;
-    i64 x0 = 0;
-    // rep owning each thread: the block's threads belong to reps r0, r0 + 1,
-    // ...; their thread offsets are loaded once (coalesced) and every thread
-    // marks where its rep starts, so a block max-scan (kept as a running max
-    // over the marks) hands each thread its rep.  Blocks whose threads span
-    // more than kT5RepWin reps fall back to a galloping search.
-    const i64 y0 = (i64)blk * kCycTile;
-    const i64 r0 = y0 < Y ? (i64)ytile_rep[blk] : 0;
-    sv1[tid] = -1;
-    __syncthreads();
-    bool wide = false;
-    for (int k = tid; k < kT5RepWin; k += kBlock) {
-        const i64 r = r0 + k;
-        if (r < a.R) {
-            const i64 ys = yoff[r];
-            if (ys >= y0 && ys < y0 + kCycTile && yoff[r + 1] > ys) sv1[ys - y0] = k;
+// f(x) for the entries x of up to 16 lists, lane i of the group holding the
+// bounds [p0, p1) of list i (lists from cnt on are empty); the group's lanes share each list,
+// four lists are loaded at a time.
+template <class F>
+__device__ __forceinline__ void walk_lists(const CycArgs& a, int p0, int p1, int cnt, F f) {
+    const int lane = threadIdx.x & (kSetLanes - 1);
+    for (int u0 = 0; u0 < cnt; u0 += 4) {  // uniform within the group
+        int s[4], e[4], x[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            s[u] = __shfl(p0, u0 + u, kSetLanes);
+            e[u] = __shfl(p1, u0 + u, kSetLanes);
+            x[u] = s[u] + lane < e[u] ? a.adj[s[u] + lane] : -1;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            if (x[u] >= 0) f(x[u]);
+            for (int k = s[u] + kSetLanes + lane; k < e[u]; k += kSetLanes) f(a.adj[k]);
         }
     }
-    if (y0 < Y) {
-        const i64 rl = r0 + kT5RepWin - 1;
-        wide = rl < a.R && yoff[rl + 1] < (y0 + kCycTile < Y ? y0 + kCycTile : Y);
-    }
-    __syncthreads();
-    int mark = sv1[tid];
-    // inclusive max-scan of the marks over the block (first thread: its rep
-    // r0 starts before the block, mark 0)
-    if (tid == 0 && mark < 0) mark = 0;
+}
+// Of the same lists: hit(i, k) for the entries x = adj[k] of list i with
+// test(x).
+template <class T, class F>
+__device__ __forceinline__ void find_in_lists(const CycArgs& a, int p0, int p1, int cnt, T test, F hit) {
+    const int lane = threadIdx.x & (kSetLanes - 1);
+        for (int u0 = 0; u0 < cnt; u0 += 4) {  // uniform within the group
+            int s[4], e[4], x[4];
 #pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const int t = __shfl_up(mark, d, 64);
-        if (lane >= d) mark = max(mark, t);
-    }
-    __shared__ int wmax[kWaves];
-    if (lane == 63) wmax[w] = mark;
-    __syncthreads();
-    for (int q = 0; q < w; ++q) mark = max(mark, wmax[q]);
-    __syncthreads();
-    if (on) {
-        i64 r = r0 + mark;
-        if (wide) {
-            // rep owning thread y (galloping from the block's first rep)
-            i64 lo = r0, hi = a.R - 1, step = 1;
-            while (lo + step <= hi && yoff[lo + step] <= y) {
-                lo += step;
-                step <<= 1;
+            for (int u = 0; u < 4; ++u) {
+                s[u] = __shfl(p0, u0 + u, kSetLanes);
+                e[u] = __shfl(p1, u0 + u, kSetLanes);
+                x[u] = s[u] + lane < e[u] ? a.adj[s[u] + lane] : -1;
             }
-            hi = lo + step < a.R - 1 ? lo + step : a.R - 1;
-            while (lo < hi) {
-                const i64 mid = (lo + hi + 1) >> 1;
-                if (yoff[mid] <= y) lo = mid; else hi = mid - 1;
+            unsigned hits = 0u, more = 0u;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                hits |= x[u] >= 0 && test(x[u]) ? 1u << u : 0u;
+                more |= e[u] - s[u] > kSetLanes ? 1u << u : 0u;
             }
-            r = lo;
-        }
-        v1 = a.rv1[r];
-        const int v2 = a.rv2[r];
-        const int l2 = (int)(y - yoff[r]);
-        b1 = a.off[v1];
-        d1 = a.off[v1 + 1] - b1;
-        n2 = a.adj[a.off[v2] + l2];
-        bq = a.off[n2];
-        nq = a.off[n2 + 1] - bq;
-        x0 = a.xoff[r] + (i64)l2 * d1;
-        if (a.nslot) slot = a.nslot[v1];
-    }
-    // runs of equal v1 over the block's threads (rep edges are in row order,
-    // so a run is usually all threads of one v1); run k < kT5Tables gets
-    // table k
-    sv1[tid] = v1;
-    for (int k = tid; k < kT5Slots; k += kBlock) {
-        tkey[k] = -1;
-        tmask[k] = 0u;
-    }
-    __syncthreads();
-    const bool start = on && (tid == 0 || sv1[tid - 1] != v1);
-    const unsigned long long sm = __ballot(start);
-    if (lane == 0) wruns[w] = __popcll(sm);
-    __syncthreads();
-    int before = 0, runs = 0;
-    for (int q = 0; q < kWaves; ++q) {
-        before += q < w ? wruns[q] : 0;
-        runs += wruns[q];
-    }
-    // this thread's run index (its run starts at or before it)
-    const int run = before + __popcll(sm & ((2ull << lane) - 1ull)) - 1;
-    if (start && run < kT5Tables) {
-        tv1[run] = v1;
-        tok[run] = 1;
-    }
-    const int ntab = runs < kT5Tables ? runs : kT5Tables;
-    __syncthreads();
-    // build, in three steps: each wave sizes its tables (w, w + kWaves, ...:
-    // lane l holds the bounds of the list of v1's l-th neighbour n1); the
-    // tables that fit the shared capacity in run order are kept; each wave
-    // inserts its kept tables' (mid, l) pairs, flattened over its 64 lanes
-    constexpr int kPerWave = kT5Tables / kWaves;
-    int s0[kPerWave], s1[kPerWave];
+            auto pick = [](int v0, int v1, int v2, int v3, int u) {
+                const int lo = u & 1 ? v1 : v0, hi = u & 1 ? v3 : v2;
+                return u & 2 ? hi : lo;
+            };
+            for (; hits; hits &= hits - 1u) {
+                const int u = __builtin_ctz(hits);
+                hit(u0 + u, pick(s[0], s[1], s[2], s[3], u) + lane);
+            }
+            for (; more; more &= more - 1u) {
+                const int u = __builtin_ctz(more);
+                const int z = pick(e[0], e[1], e[2], e[3], u);
+                for (int k = pick(s[0], s[1], s[2], s[3], u) + kSetLanes + lane; k < z; k += 4 * kSetLanes) {
+                    int y[4];
 #pragma unroll
-    for (int i = 0; i < kPerWave; ++i) {
-        const int k = w + i * kWaves;
-        s0[i] = s1[i] = 0;
-        if (k >= ntab) continue;
-        const int v = tv1[k];
-        const int bv = a.off[v], dv = a.off[v + 1] - bv;
-        if (dv <= kT5MaxD1 && lane < dv) {
-            const int n1 = a.adj[bv + lane];
-            s0[i] = a.off[n1];
-            s1[i] = a.off[n1 + 1];
-        }
-        int fill = s1[i] - s0[i];
+                    for (int v = 0; v < 4; ++v) y[v] = k + v * kSetLanes < z ? a.adj[k + v * kSetLanes] : -1;
+                    unsigned far = 0u;
 #pragma unroll
-        for (int d = 32; d >= 1; d >>= 1) fill += __shfl_xor(fill, d, 64);
-        if (lane == 0) tfill[k] = dv <= kT5MaxD1 && a.tables ? fill : kT5MaxFill + 1;
-    }
-    __syncthreads();
-    if (tid == 0) {
-        int used = 0;
-        for (int k = 0; k < ntab; ++k) {
-            const bool fits = used + tfill[k] <= kT5MaxFill;
-            tok[k] = fits ? 1 : 0;
-            used += fits ? tfill[k] : 0;
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < kPerWave; ++i) {
-        const int k = w + i * kWaves;
-        if (k >= ntab || !tok[k]) continue;  // wave-uniform
-        bool dup = false;
-        const int fill = tfill[k];
-        const int len = s1[i] - s0[i];
-        int excl = len;  // where list l starts among the table's pairs
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const int t = __shfl_up(excl, d, 64);
-            if (lane >= d) excl += t;
-        }
-        excl -= len;
-        const int dv = a.off[tv1[k] + 1] - a.off[tv1[k]];
-        for (int f0 = 0; f0 < fill; f0 += 64) {  // wave-uniform: every lane takes part in the shuffles
-            const int f = f0 + lane;
-            int l = 0;
-            for (int j = 1; j < dv; ++j) l = __builtin_amdgcn_readlane(excl, j) <= f ? j : l;
-            const int q = __shfl(s0[i], l, 64) + (f - __shfl(excl, l, 64));
-            if (f >= fill) continue;
-            const int key = a.adj[q] * kT5Tables + k;
-            const unsigned bit = 1u << l;
-            int h = t5_hash(key);
-            while (true) {
-                const int old = atomicCAS(&tkey[h], -1, key);
-                if (old == -1 || old == key) {
-                    dup |= (atomicOr(&tmask[h], bit) & bit) != 0u;
-                    break;
+                    for (int v = 0; v < 4; ++v) far |= y[v] >= 0 && test(y[v]) ? 1u << v : 0u;
+                    for (; far; far &= far - 1u) hit(u0 + u, k + __builtin_ctz(far) * kSetLanes);
                 }
-                h = (h + 1) & (kT5Slots - 1);
             }
         }
-        // a list that repeats a value disables its table
-        if (__ballot(dup) != 0ull && lane == 0) tok[k] = 0;
+}
+
+// Adds c to the (saturating) count byte of expansion x, whose count is at
+// most `most`.
+__device__ __forceinline__ void bump_count(unsigned char* cnt8, i64 x, int c, int most) {
+    unsigned* p = reinterpret_cast<unsigned*>(cnt8 + (x & ~(i64)3));
+    const int sh = 8 * (int)(x & 3);
+    if (most <= 255) {  // nothing to wait for
+        atomicAdd(p, (unsigned)c << sh);
+        return;
+    }
+    unsigned old = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    while (true) {
+        const unsigned b = (old >> sh) & 255u, nb = min(255u, b + (unsigned)c);
+        if (b == nb) return;
+        const unsigned prev = atomicCAS(p, old, (old & ~(255u << sh)) | (nb << sh));
+        if (prev == old) return;
+        old = prev;
+    }
+}
+
+// Counts entry k of N(v2) (4-cycles) or of N(n2), n2 the l2-th neighbour of
+// v2 (5-cycles), into the expansions of rep edge r; returns the attempted
+// writes.  Values repeated in a list count as the merge walk would count
+// them, min(a, b) times.
+template <int S>
+__device__ __forceinline__ i64 resolve_entry(const CycArgs& a, i64 r, int l2, int k, unsigned char* cnt8,
+                                             i64* tile_tot) {
+    const int v1 = a.rv1[r], v2 = a.rv2[r];
+    const int b1 = a.off[v1], e1 = a.off[v1 + 1];
+    const int y = S == 4 ? v2 : a.adj[a.off[v2] + l2];
+    const int ys = a.off[y], ye = a.off[y + 1];
+    const int m = a.adj[k];
+    if (k > ys && a.adj[k - 1] == m) return 0;  // counted with the value's first entry
+    int mb = 1;
+    while (k + mb < ye && a.adj[k + mb] == m) ++mb;
+    const int bm = a.off[m], em = a.off[m + 1];
+    const i64 x0 = a.xoff[r] + (S == 5 ? (i64)l2 * (e1 - b1) : 0);
+    i64 writes = 0;
+    auto hit = [&](int l, int c) {
+        bump_count(cnt8, x0 + l, c, ye - ys);
+        atomicAdd(reinterpret_cast<unsigned long long*>(tile_tot + (x0 + l) / kCycTile),
+                  (unsigned long long)(c * (S - 2)));
+        writes += c * (S - 2);
+    };
+    // N(v1) against N(m), which holds n1 as often as N(n1) holds m: a merge
+    // walk, or where one list is much longer the other's entries in it
+    int i = b1, j = bm;
+    const bool far = e1 - b1 > 8 * (em - bm), near = em - bm > 8 * (e1 - b1);
+    while (i < e1 && j < em) {
+        const int p = a.adj[i], q = a.adj[j];
+        if (p != q) {
+            if (p < q) i = far ? lower_in(a.adj, i, e1, q) : i + 1;
+            else j = near ? lower_in(a.adj, j, em, p) : j + 1;
+            continue;
+        }
+        int ma = 1;
+        while (j + ma < em && a.adj[j + ma] == p) ++ma;
+        j += ma;
+        for (; i < e1 && a.adj[i] == p; ++i)
+            if (S == 4 || p != y) hit(i - b1, min(ma, mb));
+    }
+    return writes;
+}
+
+// An entry into part `part` of the queue, in memory (lanes that call it
+// together take one place after another), or resolved at once if it is full.
+template <int S>
+__device__ __forceinline__ i64 queue_entry(const CycArgs& a, int part, i64 r, i64 r0, int l2, int k,
+                                           unsigned char* cnt8, i64* tile_tot) {
+    const unsigned long long m = __ballot(1);
+    const int rank = __popcll(m & ((1ull << lane_id()) - 1ull));
+    unsigned at = 0;
+    if (rank == 0) at = atomicAdd(a.qcount + part * 32, (unsigned)__popcll(m));
+    at = (unsigned)__builtin_amdgcn_readfirstlane((int)at) + (unsigned)rank;
+    if (at < (unsigned)a.qcap) {
+        a.queue[(i64)part * a.qcap + at] = make_int3((int)(unsigned)(r - r0), l2, k);
+        return 0;
+    }
+    const i64 add = resolve_entry<S>(a, r, l2, k, cnt8, tile_tot);
+    if (a.nslot && add)
+        atomicAdd(reinterpret_cast<unsigned long long*>(a.slot_total + a.nslot[a.rv1[r]]), (unsigned long long)add);
+    return add;
+}
+
+// Resolves the queued entries of a count launch, whose first rep edge is r0.
+template <int S>
+__global__ __launch_bounds__(kBlock) void k_cycle_resolve(CycArgs a, i64 r0, unsigned char* __restrict__ cnt8,
+                                                          i64* __restrict__ tile_tot) {
+    const int part = blockIdx.x % kQueueParts, step = (int)(gridDim.x / kQueueParts) * kBlock;
+    const int n = (int)min(a.qcount[part * 32], (unsigned)a.qcap);
+    i64 mine = 0;
+    for (int q0 = (int)(blockIdx.x / kQueueParts) * kBlock; q0 < n; q0 += step) {  // uniform
+        const int q = q0 + (int)threadIdx.x;
+        i64 add = 0;
+        int slot = 0;
+        if (q < n) {
+            const int3 e = a.queue[(i64)part * a.qcap + q];
+            const i64 r = r0 + (i64)(unsigned)e.x;
+            add = resolve_entry<S>(a, r, e.y, e.z, cnt8, tile_tot);
+            if (a.nslot) slot = a.nslot[a.rv1[r]];
+        }
+        if (a.nslot) wave_add_keyed(a.slot_total, slot, add, q < n);
+        mine += add;
+    }
+    if (a.counted) block_counted(a.counted, mine, 0);
+}
+
+// A wave's waiting entries, in LDS.
+struct WaveQueue {
+    int k[kSetQueue], l[kSetQueue];
+    unsigned r[kSetQueue];  // from the launch's first rep edge on
+    int n;
+};
+// An entry that passed: into the wave's queue, or past it if it is full.
+template <int S>
+__device__ __forceinline__ i64 push_entry(const CycArgs& a, WaveQueue& q, i64 r, i64 r0, int l2, int k,
+                                          unsigned char* cnt8, i64* tile_tot) {
+    const unsigned long long m = __ballot(1);
+    const int rank = __popcll(m & ((1ull << lane_id()) - 1ull));
+    int at = 0;
+    if (rank == 0) at = atomicAdd(&q.n, __popcll(m));
+    at = __builtin_amdgcn_readfirstlane(at) + rank;
+    if (at >= kSetQueue) return queue_entry<S>(a, blockIdx.x % kQueueParts, r, r0, l2, k, cnt8, tile_tot);
+    q.k[at] = k;
+    q.l[at] = l2;
+    q.r[at] = (unsigned)(r - r0);
+    return 0;
+}
+// Passes the wave's entries on once there are `least` (wave-uniform call).
+template <int S>
+__device__ __forceinline__ i64 drain_entries(const CycArgs& a, WaveQueue& q, i64 r0, int least, unsigned char* cnt8,
+                                             i64* tile_tot) {
+    wave_lds_fence();
+    const int n = min(q.n, kSetQueue);
+    if (n < least) return 0;
+    i64 mine = 0;
+    for (int i = lane_id(); i < n; i += 64)
+        mine += queue_entry<S>(a, blockIdx.x % kQueueParts, r0 + q.r[i], r0, q.l[i], q.k[i], cnt8, tile_tot);
+    wave_lds_fence();
+    if (lane_id() == 0) q.n = 0;
+    wave_lds_fence();
+    return mine;
+}
+
+// A block takes `reps` rep edges.  tile_tot and cnt8 must be zero on entry;
+// cnt8 is accessed in whole words.
+template <int S>
+__global__ __launch_bounds__(kBlock) void k_cycle_count(CycArgs a, int reps, unsigned char* __restrict__ cnt8,
+                                                        i64* __restrict__ tile_tot) {
+    __shared__ unsigned sets[kSetGroups * kSetWords];
+    __shared__ int sb2[kSetMaxReps], sn2[kSetMaxReps];  // N(v2)
+    __shared__ unsigned short runs[kSetMaxReps];        // first rep edge of each run
+    __shared__ int rb1[kSetMaxReps], rd1[kSetMaxReps];  // and N(v1)
+    __shared__ WaveQueue queue[kWaves];
+    __shared__ int wsum[kWaves], next;
+    const int tid = threadIdx.x, w = tid >> 6, wl = lane_id(), lane = tid & (kSetLanes - 1);
+    const i64 r0 = (i64)(a.blk0 + xcd_block()) * reps, chunk0 = (i64)a.blk0 * reps;
+    const int nr = (int)(a.R - r0 < reps ? a.R - r0 : reps);
+    WaveQueue& wq = queue[w];
+    i64 mine = 0;
+    // runs of equal v1, lists of v2
+    {
+        bool head = false;
+        int b1 = 0, e1 = 0;
+        if (tid < nr) {
+            const i64 r = r0 + tid;
+            const int v1 = a.rv1[r], v2 = a.rv2[r];
+            head = tid % kRunReps == 0 || a.rv1[r - 1] != v1;
+            b1 = a.off[v1];
+            e1 = a.off[v1 + 1];
+            sb2[tid] = a.off[v2];
+            sn2[tid] = a.off[v2 + 1] - sb2[tid];
+        }
+        const unsigned long long hm = __ballot(head);
+        if (wl == 0) {
+            wsum[w] = __popcll(hm);
+            wq.n = 0;
+        }
+        if (tid == 0) next = 0;
+        __syncthreads();
+        int before = 0;
+        for (int q = 0; q < w; ++q) before += wsum[q];
+        if (head) {
+            const int q = before + __popcll(hm & ((1ull << wl) - 1ull));
+            runs[q] = (unsigned short)tid;
+            rb1[q] = b1;
+            rd1[q] = e1 - b1;
+        }
     }
     __syncthreads();
-    if (on) {
-        const bool table = run < ntab && tok[run] && nq <= 255;
-        bool direct = !table;
-        if (table) {
-            // per-l1 counts of N(n2)'s mids, bit-sliced over 8 planes
-            unsigned p[8] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
-            int prev = -1;
-            // four entries of N(n2) per round of loads
-            for (int q0 = bq; q0 < bq + nq && !direct; q0 += 4) {
-                int ms[4];
+    int nruns = 0;
 #pragma unroll
-                for (int u = 0; u < 4; ++u) ms[u] = q0 + u < bq + nq ? a.adj[q0 + u] : -1;
+    for (int q = 0; q < kWaves; ++q) nruns += wsum[q];
+    unsigned* set = sets + tid / kSetLanes * kSetWords;
+    constexpr int kMaxN2 = S == 4 ? 16 * kSetLanes : kSetLists;
+    while (true) {
+        int q = 0;
+        if (lane == 0) q = atomicAdd(&next, 1);
+        q = __shfl(q, 0, kSetLanes);
+        if (!__any(q < nruns)) break;
+        if (q < nruns) {
+            const int ra = runs[q], rz = q + 1 < nruns ? (int)runs[q + 1] : nr, b1 = rb1[q], d1 = rd1[q];
+            // the lists' bounds, two per lane, and their entries together
+            int p0[2] = {0, 0}, p1[2] = {0, 0}, fill = 0;
+            if (d1 <= kSetLists) {
 #pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    if (direct || q0 + u >= bq + nq) continue;
-                    const int m = ms[u];
-                    if (m == prev) {  // N(n2) repeats a value: the min(a, b) rule needs the direct form
-                        direct = true;
+                for (int h = 0; h < 2; ++h) {
+                    const int l = lane + h * kSetLanes;
+                    if (l < d1) {
+                        const int y = a.adj[b1 + l];
+                        p0[h] = a.off[y];
+                        p1[h] = a.off[y + 1];
+                    }
+                    fill += p1[h] - p0[h];
+                }
+#pragma unroll
+                for (int d = kSetLanes / 2; d >= 1; d >>= 1) fill += __shfl_xor(fill, d, kSetLanes);
+            }
+            if (d1 > kSetLists || fill > kSetFill) {
+                const int n = (rz - ra + kWideReps - 1) / kWideReps;
+                unsigned at = 0;
+                if (lane == 0) at = atomicAdd(a.qcount + kQueueParts * 32, (unsigned)n);
+                at = __shfl(at, 0, kSetLanes);
+                for (int i = lane; i < n; i += kSetLanes) {
+                    const int rf = ra + i * kWideReps;
+                    a.wide[at + i] = make_int2((int)(unsigned)(r0 + rf - chunk0), min(kWideReps, rz - rf));
+                }
+            } else if (d1 > 0) {
+                for (int k = lane; k < kSetWords; k += kSetLanes) set[k] = 0u;
+                wave_lds_fence();
+                auto mark = [&](int x) {
+                    unsigned bits;
+                    const unsigned h = set_bits<6>(x, &bits);
+                    atomicOr(&set[h], bits);
+                };
+                // N(v2) of the rep edge, for 5-cycles the bounds of its lists,
+                // are loaded while the one before is looked at
+                auto ends = [&](int rl) { return rl < rz && lane < sn2[rl] ? a.adj[sb2[rl] + lane] : -1; };
+                int y = ends(ra);
+                walk_lists(a, p0[0], p1[0], min(d1, kSetLanes), mark);
+                if (d1 > kSetLanes) walk_lists(a, p0[1], p1[1], d1 - kSetLanes, mark);
+                int f0 = 0, f1 = 0;
+                if (S == 5) {
+                    if (y >= 0) {
+                        f0 = a.off[y];
+                        f1 = a.off[y + 1];
+                    }
+                    y = ends(ra + 1);
+                }
+                wave_lds_fence();
+                for (int rl = ra; rl < rz; ++rl) {
+                    const int n2 = sn2[rl], x = y, c0 = f0, c1 = f1;
+                    if (S == 4) {
+                        y = ends(rl + 1);
+                    } else {
+                        f0 = f1 = 0;
+                        if (x >= 0) {
+                            f0 = a.off[x];
+                            f1 = a.off[x + 1];
+                        }
+                        y = ends(rl + 2);
+                    }
+                    if (n2 > kMaxN2) {  // v2 is a hub
+                        if (lane == 0)
+                            a.wide[atomicAdd(a.qcount + kQueueParts * 32, 1u)] =
+                                make_int2((int)(unsigned)(r0 + rl - chunk0), 1);
                         continue;
                     }
-                    prev = m;
-                    const int want = m * kT5Tables + run;
-                    int h = t5_hash(want);
-                    unsigned mk = 0u;
-                    while (true) {
-                        const int key = tkey[h];
-                        if (key == want) {
-                            mk = tmask[h];
-                            break;
+                    auto test = [&](int m) {
+                        unsigned bits;
+                        const unsigned h = set_bits<6>(m, &bits);
+                        return !a.sets || (set[h] & bits) == bits;
+                    };
+                    auto hit = [&](int l2, int k) {
+                        mine += push_entry<S>(a, wq, r0 + rl, chunk0, l2, k, cnt8, tile_tot);
+                    };
+                    const int b2 = sb2[rl];
+                    if (S == 4) {
+                        if (x >= 0 && test(x)) hit(0, b2 + lane);
+                        for (int k = b2 + kSetLanes + lane; k < b2 + n2; k += kSetLanes)
+                            if (test(a.adj[k])) hit(0, k);
+                    } else {
+                        find_in_lists(a, c0, c1, min(n2, kSetLanes), test, hit);
+                        if (n2 > kSetLanes) {
+                            int g0 = 0, g1 = 0;
+                            if (kSetLanes + lane < n2) {
+                                const int z = a.adj[b2 + kSetLanes + lane];
+                                g0 = a.off[z];
+                                g1 = a.off[z + 1];
+                            }
+                            find_in_lists(a, g0, g1, n2 - kSetLanes, test, [&](int i, int k) { hit(kSetLanes + i, k); });
                         }
-                        if (key == -1) break;
-                        h = (h + 1) & (kT5Slots - 1);
-                    }
-#pragma unroll
-                    for (int b = 0; b < 8; ++b) {
-                        const unsigned carry = p[b] & mk;
-                        p[b] ^= mk;
-                        mk = carry;
                     }
                 }
-            }
-            if (!direct) {
-                unsigned nz = 0u;
-#pragma unroll
-                for (int b = 0; b < 8; ++b) nz |= p[b];
-                TileAcc acc;
-                for (int l = 0; l < d1; ++l) {
-                    int c = 0;
-                    if ((nz >> l) & 1u) {
-#pragma unroll
-                        for (int b = 0; b < 8; ++b) c |= (int)((p[b] >> l) & 1u) << b;
-                        if (a.adj[b1 + l] == n2) c = 0;
-                    }
-                    cnt8[x0 + l] = (unsigned char)(c < 255 ? c : 255);
-                    acc.add(tile_tot, x0 + l, 3 * (i64)c);
-                    mine += 3 * (i64)c;
-                }
-                acc.flush(tile_tot);
             }
         }
-        if (direct) count5_direct(a, b1, d1, n2, bq, nq, x0, cnt8, tile_tot, mine);
-        xend = x0 + d1;
-        if (a.stats) {
-            atomicAdd(a.stats, 1ull);
-            if (!direct) atomicAdd(a.stats + 1, 1ull);
+        mine += drain_entries<S>(a, wq, chunk0, 64, cnt8, tile_tot);
+    }
+    mine += drain_entries<S>(a, wq, chunk0, 1, cnt8, tile_tot);
+    if (a.counted) block_counted(a.counted, mine, a.xoff[r0 + nr]);
+}
+
+// The listed rep edges of hubs, up to kWideReps of one v1 per block and step.
+template <int S>
+__global__ __launch_bounds__(kBlock) void k_cycle_count_wide(CycArgs a, i64 chunk0, unsigned char* __restrict__ cnt8,
+                                                             i64* __restrict__ tile_tot) {
+    __shared__ unsigned set[kBigWords];
+    __shared__ WaveQueue queue[kWaves];
+    const int tid = threadIdx.x, lane = tid & (kSetLanes - 1), g = tid / kSetLanes;
+    const unsigned n = a.qcount[kQueueParts * 32];
+    WaveQueue& wq = queue[tid >> 6];
+    if (lane_id() == 0) wq.n = 0;
+    i64 mine = 0;
+    for (unsigned i = blockIdx.x; i < n; i += gridDim.x) {  // uniform
+        const int2 e = a.wide[i];
+        const i64 ra = chunk0 + (i64)(unsigned)e.x;
+        const int v1 = a.rv1[ra], b1 = a.off[v1], d1 = a.off[v1 + 1] - b1;
+        __syncthreads();
+        for (int k = tid; k < kBigWords; k += kBlock) set[k] = 0u;
+        __syncthreads();
+        for (int l0 = g; l0 < d1; l0 += kSetGroups * kSetLanes) {
+            const int l = l0 + kSetGroups * lane;
+            int p0 = 0, p1 = 0;
+            if (l < d1) {
+                const int y = a.adj[b1 + l];
+                p0 = a.off[y];
+                p1 = a.off[y + 1];
+            }
+            walk_lists(a, p0, p1, min(kSetLanes, (d1 - l0 + kSetGroups - 1) / kSetGroups), [&](int x) {
+                unsigned bits;
+                const unsigned h = set_bits<11>(x, &bits);
+                atomicOr(&set[h], bits);
+            });
+        }
+        __syncthreads();
+        for (int c = 0; c < e.y; ++c) {
+            const i64 r = ra + c;
+            auto test = [&](int x) {
+                unsigned bits;
+                const unsigned h = set_bits<11>(x, &bits);
+                return !a.sets || (set[h] & bits) == bits;
+            };
+            auto hit = [&](int l2, int k) {
+                mine += push_entry<S>(a, wq, r, chunk0, l2, k, cnt8, tile_tot);
+            };
+            const int v2 = a.rv2[r], b2 = a.off[v2], n2 = a.off[v2 + 1] - b2;
+            if (S == 4) {
+                for (int k = b2 + tid; k < b2 + n2; k += kBlock)
+                    if (test(a.adj[k])) hit(0, k);
+            } else {
+                for (int l0 = g; l0 < n2; l0 += kSetGroups * kSetLanes) {
+                    const int l = l0 + kSetGroups * lane;
+                    int p0 = 0, p1 = 0;
+                    if (l < n2) {
+                        const int y = a.adj[b2 + l];
+                        p0 = a.off[y];
+                        p1 = a.off[y + 1];
+                    }
+                    find_in_lists(a, p0, p1, min(kSetLanes, (n2 - l0 + kSetGroups - 1) / kSetGroups), test,
+                                  [&](int i, int k) { hit(l0 + kSetGroups * i, k); });
+                }
+            }
+            mine += drain_entries<S>(a, wq, chunk0, 64, cnt8, tile_tot);
         }
     }
-    if (a.nslot) wave_add_keyed(a.slot_total, slot, mine, on);
-    if (a.counted) block_counted(a.counted, mine, xend);
+    mine += drain_entries<S>(a, wq, chunk0, 1, cnt8, tile_tot);
+    if (a.counted) block_counted(a.counted, mine, 0);
 }
 
 __device__ __forceinline__ void put_tri(int* t1, int* t2, int* t3, i64 g, i64 budget, int a, int b, int c) {
@@ -1201,17 +1172,12 @@ __global__ void k_tile_rep(const i64* __restrict__ xoff, i64 R, int* __restrict_
 
 // Work of one count launch for the profiler (only while it is on): the
 // expansions the launch covers and the neighbour-list entries a merge walk
-// of each expansion's two lists reads, deg(a) + deg(b).  S = 3 and 4: the
-// launch covers rep edges [lo, hi); S = 5: threads [lo, hi), thread k of
-// rep edge r being (r, the (k - yoff[r])-th neighbour n2 of v2), whose
-// expansions are (n1, n2) for every n1 of v1 (n1 = n2 included: the count
-// skips it after loading both bounds).  nsum[v] = sum of the degrees of v's
-// neighbours.
+// of each expansion's two lists reads, deg(a) + deg(b); the launch covers rep
+// edges [lo, hi).  nsum[v] = sum of the degrees of v's neighbours.
 template <int S>
-static void count_work(Ctx& ctx, const Csr& G, const int* rv1, const int* rv2, i64 R, const i64* yoff, const i64* nsum,
-                       i64 lo, i64 hi, double& x, double& entries) {
+static void count_work(Ctx& ctx, const Csr& G, const int* rv1, const int* rv2, const i64* nsum, i64 lo, i64 hi,
+                       double& x, double& entries) {
     const int* OFF = G.off.get();
-    const int* ADJ = G.adj.get();
     x = entries = 0.0;
     if (hi <= lo) return;
     if (S == 3) {
@@ -1237,28 +1203,60 @@ static void count_work(Ctx& ctx, const Csr& G, const int* rv1, const int* rv2, i
     } else {
         x = (double)reduce<i64>(
             ctx,
-            [=] __device__(i64 r) {
-                const i64 a = yoff[r] > lo ? yoff[r] : lo, b = yoff[r + 1] < hi ? yoff[r + 1] : hi;
-                const int v = rv1[r];
-                return a < b ? (i64)(OFF[v + 1] - OFF[v]) * (b - a) : (i64)0;
+            [=] __device__(i64 k) {
+                const int v = rv1[lo + k], u = rv2[lo + k];
+                return (i64)(OFF[v + 1] - OFF[v]) * (i64)(OFF[u + 1] - OFF[u]);
             },
-            R, (i64)0, OpSum());
+            hi - lo, (i64)0, OpSum());
         entries = (double)reduce<i64>(
             ctx,
-            [=] __device__(i64 r) {
-                const i64 a = yoff[r] > lo ? yoff[r] : lo, b = yoff[r + 1] < hi ? yoff[r + 1] : hi;
-                if (a >= b) return (i64)0;
-                const int v = rv1[r], u = rv2[r];
-                const i64 d1 = OFF[v + 1] - OFF[v], base = (i64)OFF[u] - yoff[r];
-                i64 s = 0;
-                for (i64 k = a; k < b; ++k) {
-                    const int n2 = ADJ[base + k];
-                    s += nsum[v] + d1 * (i64)(OFF[n2 + 1] - OFF[n2]);
-                }
-                return s;
+            [=] __device__(i64 k) {
+                const int v = rv1[lo + k], u = rv2[lo + k];
+                return nsum[v] * (i64)(OFF[u + 1] - OFF[u]) + nsum[u] * (i64)(OFF[v + 1] - OFF[v]);
             },
-            R, (i64)0, OpSum());
+            hi - lo, (i64)0, OpSum());
     }
+}
+
+// Rep edges per block of a 4- or 5-cycle count: few where there are few, so
+// that every CU has some.
+static int count_reps(i64 R) {
+    return (int)std::min<i64>(std::max<i64>((R + 2047) / 2048, kSetMinReps), kSetMaxReps);
+}
+
+// The queue of a 4- or 5-cycle count over R rep edges with X expansions; where
+// there is no memory for it, entries are resolved as they come.
+struct CountQueue {
+    DBuf<int3> entries;
+    DBuf<int2> wide;
+    DBuf<unsigned> count;
+    CountQueue(Ctx& ctx, int S, i64 R, i64 X, CycArgs& a) {
+        count = ctx.buf<unsigned>((kQueueParts + 1) * 32);
+        a.qcount = count.get();
+        wide = ctx.buf<int2>(R);
+        a.wide = wide.get();
+        a.qcap = (int)std::min<i64>(X / (S == 4 ? 16 : 64) / kQueueParts + 1024, (i64)1 << 24);
+        try {
+            entries = ctx.buf<int3>((i64)kQueueParts * a.qcap);
+            a.queue = entries.get();
+        } catch (const Error& e) {
+            if (e.status != RAMA_ERR_OOM) throw;
+            a.qcap = 0;
+        }
+    }
+};
+// Counts blocks [a.blk0, a.blk0 + n) of `reps` rep edges.
+template <int S>
+static void count_blocks(Ctx& ctx, const CycArgs& a, unsigned n, int reps, unsigned char* cnt8, i64* tile) {
+    const i64 r0 = (i64)a.blk0 * reps;
+    ctx.zero(a.qcount, (kQueueParts + 1) * 32);
+    k_cycle_count<S><<<n, kBlock, 0, ctx.stream>>>(a, reps, cnt8, tile);
+    RAMA_LAUNCHED();
+    k_cycle_count_wide<S><<<std::min(n, 1024u), kBlock, 0, ctx.stream>>>(a, r0, cnt8, tile);
+    RAMA_LAUNCHED();
+    const unsigned per_part = std::min<unsigned>(std::max<unsigned>(n * (unsigned)reps / 4096u, 1u), 64u);
+    k_cycle_resolve<S><<<kQueueParts * per_part, kBlock, 0, ctx.stream>>>(a, r0, cnt8, tile);
+    RAMA_LAUNCHED();
 }
 
 // Runs one stage over all expansions; returns the number of attempted writes.
@@ -1293,9 +1291,8 @@ static i64 run_stage(Ctx& ctx, const Csr& G, const int* rv1, const int* rv2, i64
         RAMA_LAUNCHED();
     }
     CycArgs a{OFF, G.adj.get(), rv1, rv2, S > 3 ? xoff.get() : nullptr, S > 3 ? tile_rep.get() : nullptr, R, X};
-    a.tables = G.n < kT5MaxNode && cycle_tables_on() ? 1 : 0;
-    a.wide4 = cycle_tables_on() ? 1 : 0;
-    DBuf<unsigned char> cnt8 = ctx.buf<unsigned char>(X);
+    a.sets = cycle_tables_on() ? 1 : 0;
+    DBuf<unsigned char> cnt8 = ctx.buf<unsigned char>(X + 3);  // counted up in whole words
     DBuf<i64> tile = ctx.buf<i64>(ntiles + 1);
     RAMA_REQUIRE(ntiles < ((i64)1 << 31), "too many cycle expansions");
     // profiling only: each count launch's expansions and list entries, and
@@ -1314,7 +1311,7 @@ static i64 run_stage(Ctx& ctx, const Csr& G, const int* rv1, const int* rv2, i64
     }
     double wx = 0.0, wy = 0.0;
     if (S == 3) {
-        if (work_on) count_work<3>(ctx, G, rv1, rv2, R, nullptr, nullptr, 0, R, wx, wy);
+        if (work_on) count_work<3>(ctx, G, rv1, rv2, nullptr, 0, R, wx, wy);
         prof::Scope ps(ctx, "cycles3_count", 4.0 * wy + 8.0 * wx, wx, wy);
         k_cycle_count3<<<(unsigned)ntiles, kBlock, 0, ctx.stream>>>(a, cnt8.get(), tile.get());
         RAMA_LAUNCHED();
@@ -1327,41 +1324,15 @@ static i64 run_stage(Ctx& ctx, const Csr& G, const int* rv1, const int* rv2, i64
     // then a lower bound of the full one; verbose runs count everything, as
     // they print it.
     i64 tiles_used = ntiles;
-    if (S > 3) {
+    if constexpr (S > 3) {
         ctx.zero(tile.get(), ntiles);
+        ctx.zero(cnt8.get(), X + 3);
         DBuf<i64> cnt = ctx.buf<i64>(kCountedLines * 16);
         ctx.zero(cnt.get(), kCountedLines * 16);
         a.counted = cnt.get();
-        DBuf<i64> yoff;
-        DBuf<int> ytile_rep;
-        i64 Y = 0;
-        unsigned nblk = 0;
-        if (S == 4) {
-            nblk = grid_for(R);
-        } else {
-            // thread space: one thread per (rep edge, neighbour of v2)
-            yoff = ctx.buf<i64>(R + 1);
-            i64* ym = ctx.mirror<i64>();
-            scan_exclusive<i64>(ctx,
-                                [=] __device__(i64 r) { const int u = rv2[r]; return (i64)(OFF[u + 1] - OFF[u]); },
-                                yoff.get(), R, ym);
-            ctx.read_mirror(yoff.get() + R, ym, &Y);
-            if (Y > 0) {
-                const i64 ytiles = (Y + kCycTile - 1) / kCycTile;
-                RAMA_REQUIRE(ytiles < ((i64)1 << 31), "too many cycle expansions");
-                ytile_rep = ctx.buf<int>(ytiles);
-                k_tile_rep<<<grid_for(R), kBlock, 0, ctx.stream>>>(yoff.get(), R, ytile_rep.get());
-                RAMA_LAUNCHED();
-                nblk = (unsigned)ytiles;
-            }
-        }
-        static const bool cyc_stats = std::getenv("RAMA_CYCLE_STATS") != nullptr;
-        DBuf<unsigned long long> st;
-        if (cyc_stats && S == 5) {
-            st = ctx.buf<unsigned long long>(2);
-            ctx.zero(st.get(), 2);
-            a.stats = st.get();
-        }
+        const int reps = count_reps(R);
+        const unsigned nblk = (unsigned)((R + reps - 1) / reps);
+        CountQueue queue(ctx, S, R, X, a);
         const bool early = !ctx.verbose && budget > base;
         const i64 need = budget - base;
         // the first chunk: a sixteenth of the blocks (a count that runs to
@@ -1373,19 +1344,11 @@ static i64 run_stage(Ctx& ctx, const Csr& G, const int* rv1, const int* rv2, i64
             const unsigned n = std::min(chunk, nblk - done);
             a.blk0 = done;
             if (work_on) {
-                const i64 lo = (i64)done * kBlock, hi = std::min<i64>((i64)(done + n) * kBlock, S == 4 ? R : Y);
-                count_work<S>(ctx, G, rv1, rv2, R, S == 5 ? yoff.get() : nullptr, nsum.get(), lo, hi, wx, wy);
+                const i64 lo = (i64)done * reps, hi = std::min<i64>((i64)(done + n) * reps, R);
+                count_work<S>(ctx, G, rv1, rv2, nsum.get(), lo, hi, wx, wy);
             }
-            if (S == 4) {
-                prof::Scope ps(ctx, "cycles4_count", 4.0 * wy + 8.0 * wx, wx, wy);
-                k_cycle_count4<<<n, kBlock, 0, ctx.stream>>>(a, cnt8.get(), tile.get());
-                RAMA_LAUNCHED();
-            } else {
-                prof::Scope ps(ctx, "cycles5_count", 4.0 * wy + 8.0 * wx, wx, wy);
-                k_cycle_count5<<<n, kBlock, 0, ctx.stream>>>(a, yoff.get(), ytile_rep.get(), Y, cnt8.get(),
-                                                             tile.get());
-                RAMA_LAUNCHED();
-            }
+            prof::Scope ps(ctx, S == 4 ? "cycles4_count" : "cycles5_count", 4.0 * wy + 8.0 * wx, wx, wy);
+            count_blocks<S>(ctx, a, n, reps, cnt8.get(), tile.get());
             done += n;
             if (!early || done >= nblk) break;
             {
@@ -1407,19 +1370,10 @@ static i64 run_stage(Ctx& ctx, const Csr& G, const int* rv1, const int* rv2, i64
             const double want = per_block > 0.0 ? grow * (double)(need - hc[0]) / per_block + 64.0 : 1e30;
             chunk = want >= (double)(nblk - done) ? nblk - done : (unsigned)want;
         }
-        if (a.stats) {
-            unsigned long long h[2];
-            ctx.read(a.stats, h, 2);
-            std::fprintf(stderr, "5-cycle count: %llu threads, %llu through 2-hop tables (%d blocks)\n", h[0], h[1], (int)done);
-            a.stats = nullptr;
-        }
         if (done < nblk) {
-            // counted expansions [0, x_end): emit the tiles they touch; the
+            // counted expansions [0, hc[1]): emit the tiles they touch; the
             // rest of the last tile contributes nothing
-            const i64 x_end = hc[1];
-            tiles_used = (x_end + kCycTile - 1) / kCycTile;
-            const i64 tail = std::min<i64>(tiles_used * kCycTile, X) - x_end;
-            if (tail > 0) ctx.zero(cnt8.get() + x_end, tail);
+            tiles_used = (hc[1] + kCycTile - 1) / kCycTile;
         }
     }
     i64* wm = ctx.mirror<i64>();
@@ -1475,39 +1429,24 @@ void run_stage_packed(Ctx& ctx, const Csr& G, const int* rv1, const int* rv2, i6
     i64* TOT = slot.get();
     ctx.zero(TOT, Q);
     CycArgs a{OFF, G.adj.get(), rv1, rv2, S > 3 ? xoff.get() : nullptr, S > 3 ? tile_rep.get() : nullptr, R, X};
-    a.tables = G.n < kT5MaxNode && cycle_tables_on() ? 1 : 0;
-    a.wide4 = cycle_tables_on() ? 1 : 0;
+    a.sets = cycle_tables_on() ? 1 : 0;
     a.nslot = nslot;
     a.slot_total = TOT;
     a.slot_first = TOT + Q;
     a.slot_base = d_base;
     a.slot_budget = d_budget;
     a.slot_out = d_out;
-    DBuf<unsigned char> cnt8 = ctx.buf<unsigned char>(X);
+    DBuf<unsigned char> cnt8 = ctx.buf<unsigned char>(X + 3);  // counted up in whole words
     DBuf<i64> tile = ctx.buf<i64>(ntiles + 1);
-    if (S == 3) {
+    if constexpr (S == 3) {
         k_cycle_count3<<<(unsigned)ntiles, kBlock, 0, ctx.stream>>>(a, cnt8.get(), tile.get());
         RAMA_LAUNCHED();
-    } else if (S == 4) {
-        ctx.zero(tile.get(), ntiles);
-        k_cycle_count4<<<grid_for(R), kBlock, 0, ctx.stream>>>(a, cnt8.get(), tile.get());
-        RAMA_LAUNCHED();
     } else {
-        DBuf<i64> yoff = ctx.buf<i64>(R + 1);
-        scan_exclusive<i64>(ctx, [=] __device__(i64 r) { const int u = rv2[r]; return (i64)(OFF[u + 1] - OFF[u]); },
-                            yoff.get(), R);
-        const i64 Y = ctx.read1(yoff.get() + R);
         ctx.zero(tile.get(), ntiles);
-        if (Y > 0) {
-            const i64 ytiles = (Y + kCycTile - 1) / kCycTile;
-            RAMA_REQUIRE(ytiles < ((i64)1 << 31), "too many cycle expansions");
-            DBuf<int> ytile_rep = ctx.buf<int>(ytiles);
-            k_tile_rep<<<grid_for(R), kBlock, 0, ctx.stream>>>(yoff.get(), R, ytile_rep.get());
-            RAMA_LAUNCHED();
-            k_cycle_count5<<<(unsigned)ytiles, kBlock, 0, ctx.stream>>>(a, yoff.get(), ytile_rep.get(), Y,
-                                                                        cnt8.get(), tile.get());
-            RAMA_LAUNCHED();
-        }
+        ctx.zero(cnt8.get(), X + 3);
+        const int reps = count_reps(R);
+        CountQueue queue(ctx, S, R, X, a);
+        count_blocks<S>(ctx, a, (unsigned)((R + reps - 1) / reps), reps, cnt8.get(), tile.get());
     }
     scan_exclusive_arr<i64>(ctx, tile.get(), tile.get(), ntiles);
     scan_exclusive_arr<i64>(ctx, TOT, TOT + Q, Q);

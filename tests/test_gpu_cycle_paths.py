@@ -78,3 +78,46 @@ def test_dual_pass_first_cycles_are_longer(gpu, oracle, length):
         np.testing.assert_allclose(g[2], o[2], rtol=1e-6, atol=1e-6)
         assert abs(g[4] - o[4]) <= 1e-9 * max(1.0, abs(o[4]))
         assert g[4] > np.minimum(w, 0).sum(dtype=np.float64)
+
+
+def _shared_hubs(seed):
+    """Hubs that share hundreds of attractive neighbours (counts past a byte,
+    2-hop neighbourhoods past a group's set, lists past a group's lanes) with
+    long runs of repulsive edges, beside ordinary ones."""
+    rng = np.random.Generator(np.random.PCG64(seed))
+    hubs, leaves = 6, 700
+    n = hubs + leaves
+    e = {}
+    for h in range(hubs):
+        for x in rng.choice(leaves, size=420, replace=False):
+            e[(h, hubs + int(x))] = 1.0
+        for x in rng.choice(leaves, size=60, replace=False):
+            e.setdefault((h, hubs + int(x)), -1.0)
+    for h in range(hubs):
+        for g in range(h + 1, hubs):
+            e[(h, g)] = -1.0 if (h + g) % 2 else 1.0
+    for a, b in rng.integers(hubs, n, size=(900, 2)):
+        if a != b:
+            e.setdefault((int(min(a, b)), int(max(a, b))), 1.0 if rng.random() < 0.7 else -1.0)
+    keys = sorted(e)
+    i, j = (np.array(x, dtype=np.int32) for x in zip(*keys))
+    c = np.array([e[k] for k in keys]) * rng.uniform(0.5, 1.5, size=len(keys))
+    return i, j, c.astype(np.float32)
+
+
+@pytest.mark.parametrize("repeats", [False, True])
+def test_cycle_counts_of_hubs_equal_oracle(gpu, oracle, monkeypatch, repeats):
+    i, j, c = _shared_hubs(3)
+    if repeats:  # some pairs twice or three times
+        pick = np.random.Generator(np.random.PCG64(5)).choice(len(i), size=len(i) // 4)
+        i, j, c = (np.concatenate([x, x[pick]]) for x in (i, j, c))
+    r, co, v, (rows, cols) = oracle.dcoo_init(i, j, c)
+    for max_len in (4, 5):
+        for factor in (4.0, 0.4, 30000.0):
+            o = oracle.conflicted_cycles(r, co, v, rows, cols, max_len, factor)
+            for tables in ("1", "0"):
+                monkeypatch.setenv("RAMA_CYCLE_TABLES", tables)
+                g = gpu.conflicted_cycles(r, co, v, rows, cols, max_len, factor)
+                assert g[3] == o[3], (max_len, factor, tables)
+                for a, b in zip(g[:3], o[:3]):
+                    assert np.array_equal(a, b), (max_len, factor, tables)

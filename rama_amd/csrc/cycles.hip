@@ -57,7 +57,8 @@ struct CycArgs {
     int qcap = 0;
     int3* queue = nullptr;
     unsigned* qcount = nullptr;
-    int2* wide = nullptr;  // rep edges left to the wide kernel (first, number), count behind qcount's parts
+    int2* wide = nullptr;  // rep edges left to the wide kernel (first, number), count behind qcount's parts;
+                           // null: none are, all their entries are resolved
 };
 
 // Diagnostic switches (tests force each path on the same inputs; every
@@ -724,7 +725,8 @@ __global__ __launch_bounds__(kBlock) void k_cycle_count(CycArgs a, int reps, uns
 #pragma unroll
                 for (int d = kSetLanes / 2; d >= 1; d >>= 1) fill += __shfl_xor(fill, d, kSetLanes);
             }
-            if (d1 > kSetLists || fill > kSetFill) {
+            const bool hub = d1 > kSetLists || fill > kSetFill;
+            if (hub && a.wide) {
                 const int n = (rz - ra + kWideReps - 1) / kWideReps;
                 unsigned at = 0;
                 if (lane == 0) at = atomicAdd(a.qcount + kQueueParts * 32, (unsigned)n);
@@ -745,8 +747,10 @@ __global__ __launch_bounds__(kBlock) void k_cycle_count(CycArgs a, int reps, uns
                 // are loaded while the one before is looked at
                 auto ends = [&](int rl) { return rl < rz && lane < sn2[rl] ? a.adj[sb2[rl] + lane] : -1; };
                 int y = ends(ra);
-                walk_lists(a, p0[0], p1[0], min(d1, kSetLanes), mark);
-                if (d1 > kSetLanes) walk_lists(a, p0[1], p1[1], d1 - kSetLanes, mark);
+                if (!hub) {
+                    walk_lists(a, p0[0], p1[0], min(d1, kSetLanes), mark);
+                    if (d1 > kSetLanes) walk_lists(a, p0[1], p1[1], d1 - kSetLanes, mark);
+                }
                 int f0 = 0, f1 = 0;
                 if (S == 5) {
                     if (y >= 0) {
@@ -768,7 +772,7 @@ __global__ __launch_bounds__(kBlock) void k_cycle_count(CycArgs a, int reps, uns
                         }
                         y = ends(rl + 2);
                     }
-                    if (n2 > kMaxN2) {  // v2 is a hub
+                    if (n2 > kMaxN2 && a.wide) {  // v2 is a hub
                         if (lane == 0)
                             a.wide[atomicAdd(a.qcount + kQueueParts * 32, 1u)] =
                                 make_int2((int)(unsigned)(r0 + rl - chunk0), 1);
@@ -777,7 +781,7 @@ __global__ __launch_bounds__(kBlock) void k_cycle_count(CycArgs a, int reps, uns
                     auto test = [&](int m) {
                         unsigned bits;
                         const unsigned h = set_bits<6>(m, &bits);
-                        return !a.sets || (set[h] & bits) == bits;
+                        return hub || !a.sets || (set[h] & bits) == bits;
                     };
                     auto hit = [&](int l2, int k) {
                         mine += push_entry<S>(a, wq, r0 + rl, chunk0, l2, k, cnt8, tile_tot);
@@ -789,14 +793,14 @@ __global__ __launch_bounds__(kBlock) void k_cycle_count(CycArgs a, int reps, uns
                             if (test(a.adj[k])) hit(0, k);
                     } else {
                         find_in_lists(a, c0, c1, min(n2, kSetLanes), test, hit);
-                        if (n2 > kSetLanes) {
+                        for (int l0 = kSetLanes; l0 < n2; l0 += kSetLanes) {
                             int g0 = 0, g1 = 0;
-                            if (kSetLanes + lane < n2) {
-                                const int z = a.adj[b2 + kSetLanes + lane];
+                            if (l0 + lane < n2) {
+                                const int z = a.adj[b2 + l0 + lane];
                                 g0 = a.off[z];
                                 g1 = a.off[z + 1];
                             }
-                            find_in_lists(a, g0, g1, n2 - kSetLanes, test, [&](int i, int k) { hit(kSetLanes + i, k); });
+                            find_in_lists(a, g0, g1, min(kSetLanes, n2 - l0), test, [&](int i, int k) { hit(l0 + i, k); });
                         }
                     }
                 }
@@ -1224,25 +1228,32 @@ static int count_reps(i64 R) {
     return (int)std::min<i64>(std::max<i64>((R + 2047) / 2048, kSetMinReps), kSetMaxReps);
 }
 
-// The queue of a 4- or 5-cycle count over R rep edges with X expansions; where
-// there is no memory for it, entries are resolved as they come.
+// The queue of a 4- or 5-cycle count over R rep edges with X expansions, and
+// the list of hubs' rep edges.  Both are dispensable: without memory for the
+// queue entries are resolved as they come, without the list hubs' rep edges
+// are treated as the others, unfiltered.
 struct CountQueue {
     DBuf<int3> entries;
     DBuf<int2> wide;
     DBuf<unsigned> count;
+    template <class T>
+    static DBuf<T> try_buf(Ctx& ctx, i64 n) {
+        try {
+            return ctx.buf<T>(n);
+        } catch (const Error& e) {
+            if (e.status != RAMA_ERR_OOM) throw;
+            return DBuf<T>();
+        }
+    }
     CountQueue(Ctx& ctx, int S, i64 R, i64 X, CycArgs& a) {
         count = ctx.buf<unsigned>((kQueueParts + 1) * 32);
         a.qcount = count.get();
-        wide = ctx.buf<int2>(R);
+        wide = try_buf<int2>(ctx, R);
         a.wide = wide.get();
         a.qcap = (int)std::min<i64>(X / (S == 4 ? 16 : 64) / kQueueParts + 1024, (i64)1 << 24);
-        try {
-            entries = ctx.buf<int3>((i64)kQueueParts * a.qcap);
-            a.queue = entries.get();
-        } catch (const Error& e) {
-            if (e.status != RAMA_ERR_OOM) throw;
-            a.qcap = 0;
-        }
+        entries = try_buf<int3>(ctx, (i64)kQueueParts * a.qcap);
+        a.queue = entries.get();
+        if (!a.queue) a.qcap = 0;
     }
 };
 // Counts blocks [a.blk0, a.blk0 + n) of `reps` rep edges.
@@ -1252,8 +1263,10 @@ static void count_blocks(Ctx& ctx, const CycArgs& a, unsigned n, int reps, unsig
     ctx.zero(a.qcount, (kQueueParts + 1) * 32);
     k_cycle_count<S><<<n, kBlock, 0, ctx.stream>>>(a, reps, cnt8, tile);
     RAMA_LAUNCHED();
-    k_cycle_count_wide<S><<<std::min(n, 1024u), kBlock, 0, ctx.stream>>>(a, r0, cnt8, tile);
-    RAMA_LAUNCHED();
+    if (a.wide) {
+        k_cycle_count_wide<S><<<std::min(n, 1024u), kBlock, 0, ctx.stream>>>(a, r0, cnt8, tile);
+        RAMA_LAUNCHED();
+    }
     const unsigned per_part = std::min<unsigned>(std::max<unsigned>(n * (unsigned)reps / 4096u, 1u), 64u);
     k_cycle_resolve<S><<<kQueueParts * per_part, kBlock, 0, ctx.stream>>>(a, r0, cnt8, tile);
     RAMA_LAUNCHED();

@@ -384,6 +384,90 @@ __global__ __launch_bounds__(kBlock) void k_cycle_count3(CycArgs a, unsigned cha
     if (threadIdx.x == 0) tile_tot[blk] = tot;
 }
 
+// The same for up to kFewReps rep edges, which one thread each does not fill
+// the chip with: a block of 1024 threads takes a count tile.  Pairs of short
+// lists are walked by a thread; the others are listed, and groups of 16 lanes
+// take one each and search the shorter list's entries in the longer, a wave
+// where both are long.  Contracted random graphs have lists of 20 to 100
+// entries, a chain of as many loads for one thread: 62 -> 23 us a launch on
+// 50021 nodes (up to 100k rep edges), 71^3 grid 16 -> 13.  Past about 400k rep
+// edges threads are enough and walk short lists faster: 1024x2048 grid, 250k
+// 44 -> 30 us, 380k 46 -> 42, 610k 47 -> 66; 192^3, 510k 6.6 -> 9.8.
+constexpr int kFewReps = 3 << 17;
+constexpr int kFewThreads = 1024;
+constexpr int kFewGroups = kFewThreads / 16;
+constexpr int kFewWalk = 32;    // entries of both lists that a thread walks
+constexpr int kFewGroup = 128;  // entries of the shorter list that a group takes
+
+// count_common by a group of 16 lanes, every lane returns it.
+__device__ __forceinline__ int group_count_common(const int* __restrict__ adj, int sb, int se, int lb, int le) {
+    int c = 0;
+    for (int i = sb + (int)(threadIdx.x & 15); i < se; i += 16) c += has_partner(adj, sb, i, adj[i], lb, le) ? 1 : 0;
+#pragma unroll
+    for (int d = 8; d >= 1; d >>= 1) c += __shfl_xor(c, d, 16);
+    return c;
+}
+
+__global__ __launch_bounds__(kFewThreads) void k_cycle_count3_few(CycArgs a, unsigned char* __restrict__ cnt8,
+                                                                  i64* __restrict__ tile_tot) {
+    __shared__ int cnt[kCycTile];
+    __shared__ unsigned char list[kCycTile];
+    __shared__ int nlist;
+    __shared__ i64 ws[kCycTile / 64];
+    const int tid = threadIdx.x, w = tid >> 6;
+    const i64 r0 = (i64)blockIdx.x * kCycTile, r = r0 + tid;
+    const bool on = tid < kCycTile && r < a.R;
+    int v1 = 0;
+    if (tid == 0) nlist = 0;
+    if (tid < kCycTile) cnt[tid] = 0;
+    __syncthreads();
+    if (on) {
+        v1 = a.rv1[r];
+        const int v2 = a.rv2[r];
+        const int n = a.off[v1 + 1] - a.off[v1] + a.off[v2 + 1] - a.off[v2];
+        if (n <= kFewWalk) cnt[tid] = count_common(a.off, a.adj, v1, v2);
+        else list[atomicAdd(&nlist, 1)] = (unsigned char)tid;
+    }
+    __syncthreads();
+    const int n = nlist;
+    for (int q = tid >> 4; q < n; q += kFewGroups) {
+        const int rl = list[q];
+        int sb, se, lb, le;
+        short_long(a.off, a.rv1[r0 + rl], a.rv2[r0 + rl], sb, se, lb, le);
+        if (se - sb > kFewGroup) {
+            if ((tid & 15) == 0) cnt[rl] = -1;
+            continue;
+        }
+        const int c = group_count_common(a.adj, sb, se, lb, le);
+        if ((tid & 15) == 0) cnt[rl] = c;
+    }
+    __syncthreads();
+    for (int q = w; q < n; q += kFewThreads / 64) {
+        const int rl = list[q];
+        if (cnt[rl] != -1) continue;  // uniform within the wave
+        const int c = wave_count_common(a.off, a.adj, __builtin_amdgcn_readfirstlane(a.rv1[r0 + rl]),
+                                        __builtin_amdgcn_readfirstlane(a.rv2[r0 + rl]));
+        if (lane_id() == 0) cnt[rl] = c;
+    }
+    __syncthreads();
+    if (w < kCycTile / 64) {
+        const int c = cnt[tid];
+        if (on) cnt8[r] = (unsigned char)(c < 255 ? c : 255);
+        if (a.nslot) wave_add_keyed(a.slot_total, on ? a.nslot[v1] : 0, (i64)c, on);
+        i64 t = c;
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) t += shfl_down64(t, d);
+        if (lane_id() == 0) ws[w] = t;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        i64 t = 0;
+#pragma unroll
+        for (int q = 0; q < kCycTile / 64; ++q) t += ws[q];
+        tile_tot[blockIdx.x] = t;
+    }
+}
+
 // 4- and 5-cycles.  Expansions of rep edge r = (v1, v2) are xoff[r] ..
 // xoff[r+1]-1: for 4-cycles the neighbours n1 of v1 (l1 = 0 .. d1-1), each
 // intersecting N(n1) with N(v2); for 5-cycles the pairs (n1, n2) at
@@ -1059,6 +1143,85 @@ __global__ __launch_bounds__(kBlock) void k_cycle_emit_dense(CycArgs a, const un
     emit_item<S>(a, c > 0, x, pos, budget, t1, t2, t3);
 }
 
+// Dense emit of 3-cycles for up to kFewReps rep edges: a block of 1024 threads
+// per count tile, groups of 16 lanes write one rep edge's triangles each, the
+// k-th entry of the shorter list that has a partner at the k-th place, a wave
+// where both lists are long.  (k_cycle_emit_dense<3> walks lists of up to 96
+// entries by one thread and longer ones one after another in the wave: 127 us a
+// launch on 50021 nodes, 43 here.)
+__global__ __launch_bounds__(kFewThreads) void k_cycle_emit3_few(CycArgs a, const unsigned char* __restrict__ cnt8,
+                                                                 const i64* __restrict__ tile_off, i64 base,
+                                                                 i64 budget, int* __restrict__ t1,
+                                                                 int* __restrict__ t2, int* __restrict__ t3) {
+    __shared__ int cnt[kCycTile];
+    __shared__ i64 pos[kCycTile];
+    __shared__ i64 wtot[kCycTile / 64];
+    const int tid = threadIdx.x, w = tid >> 6, gl = tid & 15;
+    const bool packed = a.nslot != nullptr;
+    if (tile_off[blockIdx.x + 1] == tile_off[blockIdx.x]) return;  // uniform: the tile writes nothing
+    const i64 tstart = (packed ? 0 : base) + tile_off[blockIdx.x];
+    if (!packed && tstart >= budget) return;  // uniform
+    const i64 r0 = (i64)blockIdx.x * kCycTile;
+    if (tid < kCycTile) cnt[tid] = r0 + tid < a.R ? (int)cnt8[r0 + tid] : 0;
+    __syncthreads();
+    for (int q = w; q < kCycTile; q += kFewThreads / 64) {
+        if (cnt[q] != 255) continue;  // uniform within the wave; else saturated: count again
+        const int c = wave_count_common(a.off, a.adj, __builtin_amdgcn_readfirstlane(a.rv1[r0 + q]),
+                                        __builtin_amdgcn_readfirstlane(a.rv2[r0 + q]));
+        if (lane_id() == 0) cnt[q] = c;
+    }
+    __syncthreads();
+    i64 before = 0, tot = 0;
+    if (w < kCycTile / 64) {
+        before = wave_excl_scan64((i64)cnt[tid], &tot);
+        if (lane_id() == 0) wtot[w] = tot;
+    }
+    __syncthreads();
+    if (w < kCycTile / 64) {
+        for (int q = 0; q < w; ++q) before += wtot[q];
+        pos[tid] = tstart + before;
+    }
+    __syncthreads();
+    // lanes sub, sub + width, ... of `width` share rep edge q
+    auto emit = [&](int q, int sub, int width, unsigned long long share) {
+        const int v1 = a.rv1[r0 + q], v2 = a.rv2[r0 + q];
+        i64 g = pos[q], last = budget;
+        int *u1 = t1, *u2 = t2, *u3 = t3;
+        if (packed) {
+            // the instance's own position, budget and region
+            const int z = a.nslot[v1];
+            g = a.slot_base[z] + (g - a.slot_first[z]);
+            last = a.slot_budget[z];
+            u1 += a.slot_out[z];
+            u2 += a.slot_out[z];
+            u3 += a.slot_out[z];
+        }
+        int sb, se, lb, le;
+        short_long(a.off, v1, v2, sb, se, lb, le);
+        const unsigned long long below = share & ((1ull << lane_id()) - 1ull);
+        for (int i0 = sb; i0 < se && g < last; i0 += width) {  // uniform among the sharing lanes
+            const int i = i0 + sub;
+            int mid = 0;
+            bool m = false;
+            if (i < se) {
+                mid = a.adj[i];
+                m = has_partner(a.adj, sb, i, mid, lb, le);
+            }
+            const unsigned long long bm = __ballot(m) & share;
+            if (m) put_tri(u1, u2, u3, g + __popcll(bm & below), last, v1, v2, mid);
+            g += __popcll(bm);
+        }
+    };
+    auto shorter = [&](int q) {
+        const int v1 = a.rv1[r0 + q], v2 = a.rv2[r0 + q];
+        return min(a.off[v1 + 1] - a.off[v1], a.off[v2 + 1] - a.off[v2]);
+    };
+    for (int q = tid >> 4; q < kCycTile; q += kFewGroups)
+        if (cnt[q] > 0 && shorter(q) <= kFewGroup) emit(q, gl, 16, 0xffffull << (lane_id() & 48));
+    for (int q = w; q < kCycTile; q += kFewThreads / 64)
+        if (cnt[q] > 0 && shorter(q) > kFewGroup) emit(q, lane_id(), 64, ~0ull);
+}
+
 // Sparse emit: one wave per block walks a contiguous range of count tiles in
 // order.  Each tile's 256 counts are read four per lane (expansion order is
 // lane-major), a wave scan turns them into write positions (tile start +
@@ -1155,13 +1318,25 @@ static void launch_emit(Ctx& ctx, const CycArgs& a, const unsigned char* cnt8, c
                         i64 W, i64 base, i64 budget, int* t1, int* t2, int* t3) {
     const int forced = emit_form_forced();
     if (forced == 1 || (forced == 0 && W * kEmitDenseShare >= (i64)(S - 2) * a.X)) {
-        k_cycle_emit_dense<S><<<(unsigned)ntiles, kBlock, 0, ctx.stream>>>(a, cnt8, tile_off, base, budget, t1, t2,
-                                                                           t3);
+        if (S == 3 && a.R <= kFewReps)
+            k_cycle_emit3_few<<<(unsigned)ntiles, kFewThreads, 0, ctx.stream>>>(a, cnt8, tile_off, base, budget, t1, t2,
+                                                                               t3);
+        else
+            k_cycle_emit_dense<S><<<(unsigned)ntiles, kBlock, 0, ctx.stream>>>(a, cnt8, tile_off, base, budget, t1, t2,
+                                                                               t3);
     } else {
         const i64 per = kEmitTilesPerWave;
         k_cycle_emit<S><<<(unsigned)((ntiles + per - 1) / per), 64, 0, ctx.stream>>>(a, cnt8, tile_off, ntiles, per,
                                                                                      base, budget, t1, t2, t3);
     }
+    RAMA_LAUNCHED();
+}
+
+static void launch_count3(Ctx& ctx, const CycArgs& a, unsigned ntiles, unsigned char* cnt8, i64* tile) {
+    if (a.R <= kFewReps)
+        k_cycle_count3_few<<<ntiles, kFewThreads, 0, ctx.stream>>>(a, cnt8, tile);
+    else
+        k_cycle_count3<<<ntiles, kBlock, 0, ctx.stream>>>(a, cnt8, tile);
     RAMA_LAUNCHED();
 }
 
@@ -1326,8 +1501,7 @@ static i64 run_stage(Ctx& ctx, const Csr& G, const int* rv1, const int* rv2, i64
     if (S == 3) {
         if (work_on) count_work<3>(ctx, G, rv1, rv2, nullptr, 0, R, wx, wy);
         prof::Scope ps(ctx, "cycles3_count", 4.0 * wy + 8.0 * wx, wx, wy);
-        k_cycle_count3<<<(unsigned)ntiles, kBlock, 0, ctx.stream>>>(a, cnt8.get(), tile.get());
-        RAMA_LAUNCHED();
+        launch_count3(ctx, a, (unsigned)ntiles, cnt8.get(), tile.get());
     }
     // Stages 4 and 5 count in chunks of blocks, each a prefix of the
     // expansion order, and stop once the attempted writes reach the budget
@@ -1452,8 +1626,7 @@ void run_stage_packed(Ctx& ctx, const Csr& G, const int* rv1, const int* rv2, i6
     DBuf<unsigned char> cnt8 = ctx.buf<unsigned char>(X + 3);  // counted up in whole words
     DBuf<i64> tile = ctx.buf<i64>(ntiles + 1);
     if constexpr (S == 3) {
-        k_cycle_count3<<<(unsigned)ntiles, kBlock, 0, ctx.stream>>>(a, cnt8.get(), tile.get());
-        RAMA_LAUNCHED();
+        launch_count3(ctx, a, (unsigned)ntiles, cnt8.get(), tile.get());
     } else {
         ctx.zero(tile.get(), ntiles);
         ctx.zero(cnt8.get(), X + 3);

@@ -121,3 +121,27 @@ def test_cycle_counts_of_hubs_equal_oracle(gpu, oracle, monkeypatch, repeats):
                 assert g[3] == o[3], (max_len, factor, tables)
                 for a, b in zip(g[:3], o[:3]):
                     assert np.array_equal(a, b), (max_len, factor, tables)
+
+
+@pytest.mark.parametrize("extra", [0, 20000])
+def test_triangles_of_few_and_many_rep_edges(gpu, oracle, monkeypatch, extra):
+    """3-cycles on both sides of the 393216 rep edges up to which groups of
+    lanes count and write them, with lists of a few, dozens and hundreds of
+    entries; rep edges without cycles fill up the count."""
+    i, j, c = _shared_hubs(7)
+    d, e, f = named("er800_dense")
+    n = int(max(i.max(), j.max())) + 1
+    m = n + int(max(d.max(), e.max())) + 1
+    k = 393216 - int((c < 0).sum()) - int((f < 0).sum()) + extra
+    a = np.arange(k, dtype=np.int32)
+    i, j = np.concatenate([i, d + n, m + a]), np.concatenate([j, e + n, m + a + 1])
+    c = np.concatenate([c, f, np.full(k, -1.0, np.float32)])
+    r, co, v, (rows, cols) = oracle.dcoo_init(i, j, c)
+    for factor in (2.0, 0.002):
+        o = oracle.conflicted_cycles(r, co, v, rows, cols, 3, factor)
+        for form in ("dense", "queue"):
+            monkeypatch.setenv("RAMA_EMIT_FORM", form)
+            g = gpu.conflicted_cycles(r, co, v, rows, cols, 3, factor)
+            assert g[3] == o[3], (factor, form)
+            for x, y in zip(g[:3], o[:3]):
+                assert np.array_equal(x, y), (factor, form)

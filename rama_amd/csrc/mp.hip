@@ -332,28 +332,41 @@ struct MPControl {
 };
 
 // Thread t's share of a fixed-order sum: p[t] + p[t + kBlock] + ... in
-// increasing index, with eight loads in flight at a time (the additions keep
+// increasing index, with kBatch loads in flight at a time (the additions keep
 // their order, so the result does not depend on the batching).
+template <int kBatch>
 __device__ __forceinline__ double strided_sum(const double* __restrict__ p, i64 n) {
     double s = 0.0;
     i64 k = threadIdx.x;
-    for (; k + 7 * kBlock < n; k += 8 * kBlock) {
-        double v[8];
+    for (; k + (kBatch - 1) * kBlock < n; k += kBatch * kBlock) {
+        double v[kBatch];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = p[k + (i64)u * kBlock];
+        for (int u = 0; u < kBatch; ++u) v[u] = p[k + (i64)u * kBlock];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) s += v[u];
+        for (int u = 0; u < kBatch; ++u) s += v[u];
+    }
+    if constexpr (kBatch > 8) {
+        for (; k + 7 * kBlock < n; k += 8 * kBlock) {
+            double v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] = p[k + (i64)u * kBlock];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) s += v[u];
+        }
     }
     for (; k < n; k += kBlock) s += p[k];
     return s;
 }
 
 // After an iteration on a large grid: sum the lower-bound partials in the
-// same fixed order as the fused path and apply the stall test.
+// same fixed order as the fused path and apply the stall test.  One block sums
+// up to 10^5 partials, bound by the latency of its loads: 58k partials 26 us
+// with 8 in flight per thread, 13 with 32.  (The edge sweep's fused sum keeps 8:
+// it is short, and the registers of 32 cost the sweep itself 15%.)
 __global__ __launch_bounds__(kBlock) void k_mp_finalize(const double* __restrict__ parts, i64 n, MPControl* ctl) {
     __shared__ double ws[kWaves];
     if (!ctl->active) return;
-    const double sum = block_reduce(strided_sum(parts, n), OpSum(), ws);
+    const double sum = block_reduce(strided_sum<32>(parts, n), OpSum(), ws);
     if (threadIdx.x == 0) {
         const double lb = sum + ctl->linact;
         ctl->prev = ctl->lb;
@@ -556,7 +569,7 @@ __global__ __launch_bounds__(kBlock) void k_mp_edges(i64 Ea, const int* __restri
     __syncthreads();
     if (!last) return;
     __threadfence();  // acquire: the other blocks' partials are visible to plain loads
-    const double sum = block_reduce(strided_sum(parts, nparts), OpSum(), ws);
+    const double sum = block_reduce(strided_sum<8>(parts, nparts), OpSum(), ws);
     if (threadIdx.x == 0) {
         const double tot = sum + ctl->linact;
         ctl->prev = ctl->lb;
@@ -672,7 +685,7 @@ __global__ __launch_bounds__(kBlock) void k_mp_finalize_packed(MPPack pk, const 
     MPControl* c = ctl + q;
     if (!c->active) return;
     const i64 n = (i64)(pk.tblk[q + 1] - pk.tblk[q]) + (pk.eblk[q + 1] - pk.eblk[q]);
-    const double sum = block_reduce(strided_sum(parts + pk.pbeg[q], n), OpSum(), ws);
+    const double sum = block_reduce(strided_sum<8>(parts + pk.pbeg[q], n), OpSum(), ws);
     if (threadIdx.x == 0) {
         const double lb = sum + c->linact;
         c->prev = c->lb;

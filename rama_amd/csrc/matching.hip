@@ -280,7 +280,7 @@ int matching_vertex_based(Ctx& ctx, const Csr& U, float mean_multiplier, DBuf<in
         }
         {
             // offsets + (neighbour, cost, neighbour's matched flag) per CSR entry + best per vertex
-            prof::Scope ps(ctx, "match_pick_best", 12.0 * U.nnz + 12.0 * n);
+            prof::Scope ps(ctx, "match_pick_best", 8.0 * U.nnz + 12.0 * n);
             k_pick_best<<<pick_grid, kBlock, 0, ctx.stream>>>(n, mean_multiplier, t, st, U.off.get(), U.adj.get(),
                                                               U.w.get(), matched.get(), best.get());
             RAMA_LAUNCHED();

@@ -1340,13 +1340,23 @@ static void launch_count3(Ctx& ctx, const CycArgs& a, unsigned ntiles, unsigned 
     RAMA_LAUNCHED();
 }
 
-// tile_rep[t] = rep edge containing the first expansion of tile t.
-__global__ void k_tile_rep(const i64* __restrict__ xoff, i64 R, int* __restrict__ tile_rep) {
-    const i64 r = (i64)blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= R) return;
-    const i64 b = xoff[r], e = xoff[r + 1];
-    if (e <= b) return;
-    for (i64 t = (b + kCycTile - 1) / kCycTile; t * kCycTile < e; ++t) tile_rep[t] = (int)r;
+// Before a 4- or 5-cycle count, in one launch (a memset each costs the host
+// more than this kernel): tile_rep[t] = rep edge containing the first expansion
+// of tile t; tile totals, count bytes (whole 16-byte words) and counters
+// cleared.
+__global__ __launch_bounds__(kBlock) void k_count_begin(const i64* __restrict__ xoff, i64 R, int* __restrict__ tile_rep,
+                                                        i64* __restrict__ tile, i64 ntiles, uint4* __restrict__ cnt8,
+                                                        i64 words, i64* __restrict__ counted, int ncounted,
+                                                        unsigned* __restrict__ qcount, int nqcount) {
+    const i64 i0 = (i64)blockIdx.x * kBlock + threadIdx.x, stride = (i64)gridDim.x * kBlock;
+    for (i64 r = i0; r < R; r += stride) {
+        const i64 b = xoff[r], e = xoff[r + 1];
+        for (i64 t = (b + kCycTile - 1) / kCycTile; t * kCycTile < e; ++t) tile_rep[t] = (int)r;
+    }
+    for (i64 i = i0; i < words; i += stride) cnt8[i] = make_uint4(0u, 0u, 0u, 0u);
+    for (i64 i = i0; i < ntiles; i += stride) tile[i] = 0;
+    if (i0 < ncounted) counted[i0] = 0;
+    for (i64 i = i0; i < nqcount; i += stride) qcount[i] = 0u;
 }
 
 // Work of one count launch for the profiler (only while it is on): the
@@ -1431,11 +1441,20 @@ struct CountQueue {
         if (!a.queue) a.qcap = 0;
     }
 };
+// k_count_begin for a stage of R rep edges and a.X expansions.
+static void count_begin(Ctx& ctx, const CycArgs& a, int* tile_rep, i64* tile, unsigned char* cnt8) {
+    const i64 ntiles = (a.X + kCycTile - 1) / kCycTile, words = (a.X + 15) / 16;
+    const i64 n = std::max<i64>(std::max<i64>(a.R, words), (kQueueParts + 1) * 32);
+    k_count_begin<<<(unsigned)std::min<i64>((n + kBlock - 1) / kBlock, 4096), kBlock, 0, ctx.stream>>>(
+        a.xoff, a.R, tile_rep, tile, ntiles, reinterpret_cast<uint4*>(cnt8), words, a.counted,
+        a.counted ? kCountedLines * 16 : 0, a.qcount, (kQueueParts + 1) * 32);
+    RAMA_LAUNCHED();
+}
 // Counts blocks [a.blk0, a.blk0 + n) of `reps` rep edges.
 template <int S>
 static void count_blocks(Ctx& ctx, const CycArgs& a, unsigned n, int reps, unsigned char* cnt8, i64* tile) {
     const i64 r0 = (i64)a.blk0 * reps;
-    ctx.zero(a.qcount, (kQueueParts + 1) * 32);
+    if (a.blk0 > 0) ctx.zero(a.qcount, (kQueueParts + 1) * 32);
     k_cycle_count<S><<<n, kBlock, 0, ctx.stream>>>(a, reps, cnt8, tile);
     RAMA_LAUNCHED();
     if (a.wide) {
@@ -1475,12 +1494,10 @@ static i64 run_stage(Ctx& ctx, const Csr& G, const int* rv1, const int* rv2, i64
     DBuf<int> tile_rep;
     if (S > 3) {
         tile_rep = ctx.buf<int>(ntiles);
-        k_tile_rep<<<grid_for(R), kBlock, 0, ctx.stream>>>(xoff.get(), R, tile_rep.get());
-        RAMA_LAUNCHED();
     }
     CycArgs a{OFF, G.adj.get(), rv1, rv2, S > 3 ? xoff.get() : nullptr, S > 3 ? tile_rep.get() : nullptr, R, X};
     a.sets = cycle_tables_on() ? 1 : 0;
-    DBuf<unsigned char> cnt8 = ctx.buf<unsigned char>(X + 3);  // counted up in whole words
+    DBuf<unsigned char> cnt8 = ctx.buf<unsigned char>((X + 15) / 16 * 16);  // cleared and counted up in whole words
     DBuf<i64> tile = ctx.buf<i64>(ntiles + 1);
     RAMA_REQUIRE(ntiles < ((i64)1 << 31), "too many cycle expansions");
     // profiling only: each count launch's expansions and list entries, and
@@ -1512,14 +1529,12 @@ static i64 run_stage(Ctx& ctx, const Csr& G, const int* rv1, const int* rv2, i64
     // they print it.
     i64 tiles_used = ntiles;
     if constexpr (S > 3) {
-        ctx.zero(tile.get(), ntiles);
-        ctx.zero(cnt8.get(), X + 3);
         DBuf<i64> cnt = ctx.buf<i64>(kCountedLines * 16);
-        ctx.zero(cnt.get(), kCountedLines * 16);
         a.counted = cnt.get();
         const int reps = count_reps(R);
         const unsigned nblk = (unsigned)((R + reps - 1) / reps);
         CountQueue queue(ctx, S, R, X, a);
+        count_begin(ctx, a, tile_rep.get(), tile.get(), cnt8.get());
         const bool early = !ctx.verbose && budget > base;
         const i64 need = budget - base;
         // the first chunk: a sixteenth of the blocks (a count that runs to
@@ -1609,8 +1624,6 @@ void run_stage_packed(Ctx& ctx, const Csr& G, const int* rv1, const int* rv2, i6
     DBuf<int> tile_rep;
     if (S > 3) {
         tile_rep = ctx.buf<int>(ntiles);
-        k_tile_rep<<<grid_for(R), kBlock, 0, ctx.stream>>>(xoff.get(), R, tile_rep.get());
-        RAMA_LAUNCHED();
     }
     DBuf<i64> slot = ctx.buf<i64>(2 * (i64)Q + 1);  // [0, Q) totals, [Q, 2Q] their exclusive scan
     i64* TOT = slot.get();
@@ -1623,15 +1636,14 @@ void run_stage_packed(Ctx& ctx, const Csr& G, const int* rv1, const int* rv2, i6
     a.slot_base = d_base;
     a.slot_budget = d_budget;
     a.slot_out = d_out;
-    DBuf<unsigned char> cnt8 = ctx.buf<unsigned char>(X + 3);  // counted up in whole words
+    DBuf<unsigned char> cnt8 = ctx.buf<unsigned char>((X + 15) / 16 * 16);  // cleared and counted up in whole words
     DBuf<i64> tile = ctx.buf<i64>(ntiles + 1);
     if constexpr (S == 3) {
         launch_count3(ctx, a, (unsigned)ntiles, cnt8.get(), tile.get());
     } else {
-        ctx.zero(tile.get(), ntiles);
-        ctx.zero(cnt8.get(), X + 3);
         const int reps = count_reps(R);
         CountQueue queue(ctx, S, R, X, a);
+        count_begin(ctx, a, tile_rep.get(), tile.get(), cnt8.get());
         count_blocks<S>(ctx, a, (unsigned)((R + reps - 1) / reps), reps, cnt8.get(), tile.get());
     }
     scan_exclusive_arr<i64>(ctx, tile.get(), tile.get(), ntiles);

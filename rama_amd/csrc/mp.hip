@@ -580,6 +580,72 @@ __global__ __launch_bounds__(kBlock) void k_mp_edges(i64 Ea, const int* __restri
     }
 }
 
+// All iterations of a small state in one launch, by one workgroup: its four
+// quarters of kBlock threads work as the blocks of k_mp_triangles and
+// k_mp_edges would, with barriers for the launches' order, and the partials are
+// added in the same order, so bounds and costs are those of the loop of
+// launches.  Ten iterations on about a thousand triangles, as contracted graphs
+// have them: 31 us against 78 us of kernels in twenty launches (and 70 us of the
+// host); 187x211 grid PD+ 11.1 -> 10.2 ms.  A second step of four blocks each is
+// where the launches' own parallelism begins to pay, hence the limit.
+constexpr int kMpSmallMax = 2048;  // triangles, and edges in a triangle, at most
+constexpr int kMpSmallThreads = 1024;
+__global__ __launch_bounds__(kMpSmallThreads) void k_mp_small(i64 T, i64 Ea, int steps, const int* c12, const int* c13,
+                                                              const int* c23, float* share, float* t12, float* t13,
+                                                              float* t23, const u32* pos, const int* hq, float* delta,
+                                                              float* eca, MPControl* ctl) {
+    constexpr int kQuarters = kMpSmallThreads / kBlock;
+    constexpr int kParts = 2 * kMpSmallMax / kBlock;
+    __shared__ double ws[kMpSmallThreads / 64];
+    __shared__ double parts[kParts];
+    __shared__ int active;
+    const int tid = threadIdx.x, quarter = tid / kBlock, lane = lane_id(), w = tid >> 6;
+    const int gt = (int)((T + kBlock - 1) / kBlock), ge = (int)((Ea + kMpEdgesPerBlock - 1) / kMpEdgesPerBlock);
+    if (tid == 0) active = ctl->active;
+    __syncthreads();
+    // block_reduce of each quarter, into parts[at]
+    auto reduce = [&](double x, int at, bool on) {
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) x = x + shfl_down64(x, d);
+        if (lane == 0) ws[w] = x;
+        __syncthreads();
+        if (on && tid % kBlock == 0) {
+            double r = ws[quarter * kWaves];
+#pragma unroll
+            for (int k = 1; k < kWaves; ++k) r = r + ws[quarter * kWaves + k];
+            parts[at] = r;
+        }
+        __syncthreads();
+    };
+    for (int it = 0; it < steps && active; ++it) {  // uniform
+        for (int b0 = 0; b0 < gt; b0 += kQuarters) {
+            const int b = b0 + quarter;
+            const i64 t = (i64)b * kBlock + tid % kBlock;
+            reduce(t < T ? mp_triangle<true>(t, c12, c13, c23, share, t12, t13, t23, pos, delta) : 0.0, b, b < gt);
+        }
+        for (int b0 = 0; b0 < ge; b0 += kQuarters) {
+            const int b = b0 + quarter;
+            const i64 k = (i64)b * kMpEdgesPerBlock + tid % kBlock;
+            reduce(mp_edge_pair<true>(k, Ea, hq, delta, eca, share), gt + b, b < ge);
+        }
+        double s = 0.0;
+        if (tid < gt + ge) s += parts[tid];
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) s = s + shfl_down64(s, d);
+        if (tid == 0) {
+            // the other waves hold no partial: their sums are zero
+            const double lb = s + ctl->linact;
+            ctl->prev = ctl->lb;
+            ctl->lb = lb;
+            ctl->iterations += 1;
+            if (lb - ctl->prev < 1e-3) active = 0;
+        }
+        __syncthreads();
+    }
+    if (tid == 0) ctl->active = active;
+}
+static_assert(2 * kMpSmallMax / kBlock <= 64, "one wave adds the partials");
+
 static double sum_parts(Ctx& ctx, MPState& S, i64 n) {
     double* P = S.lbparts.get();
     const i64 slot = S.lbparts.size() - 1;
@@ -835,7 +901,15 @@ double mp_run(Ctx& ctx, MPState& S, int steps) {
         C->linact = P[2];
     });
     ctx.reduce_ticket();  // created (and cleared) before any capture
-    ctx.repeat(steps, mp_graphs(), [&] { launch_round(ctx, S, true, C); });
+    if (S.T <= kMpSmallMax && S.Ea <= kMpSmallMax && !mp_graphs() && !prof::wants("mp_triangles") &&
+        !prof::wants("mp_edges")) {
+        k_mp_small<<<1, kMpSmallThreads, 0, ctx.stream>>>(S.T, S.Ea, steps, S.c12.get(), S.c13.get(), S.c23.get(),
+                                                          S.share.get(), S.t12.get(), S.t13.get(), S.t23.get(),
+                                                          S.pos.get(), S.hq.get(), S.delta.get(), S.eca.get(), C);
+        RAMA_LAUNCHED();
+    } else {
+        ctx.repeat(steps, mp_graphs(), [&] { launch_round(ctx, S, true, C); });
+    }
     MPControl h;
     ctx.read(C, &h, 1);
     S.max_col = h.max_col;

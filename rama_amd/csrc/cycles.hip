@@ -1230,7 +1230,12 @@ __global__ __launch_bounds__(kFewThreads) void k_cycle_emit3_few(CycArgs a, cons
 // Most expansions have no mid, so lanes stay busy instead of idling beside
 // the few that write.  Saturated counts (255) are counted again first.
 constexpr int kEmitQueue = 320;  // at most 63 waiting + 256 from one tile
-constexpr i64 kEmitTilesPerWave = 8;  // count tiles a queued-emit wave walks (latency-bound loop: keep it short)
+// Count tiles a queued-emit wave walks, one after another: at most
+// kEmitTilesPerWave, and several only once there are more than the waves that
+// the chip holds (71^3 grid, eight each -> one: 4-cycles 49 -> 24 us a launch,
+// 5-cycles 83 -> 47, 3-cycles 25 -> 10).
+constexpr i64 kEmitWaves = 8192;
+constexpr i64 kEmitTilesPerWave = 8;
 
 template <int S>
 __global__ __launch_bounds__(64) void k_cycle_emit(CycArgs a, const unsigned char* __restrict__ cnt8,
@@ -1325,7 +1330,7 @@ static void launch_emit(Ctx& ctx, const CycArgs& a, const unsigned char* cnt8, c
             k_cycle_emit_dense<S><<<(unsigned)ntiles, kBlock, 0, ctx.stream>>>(a, cnt8, tile_off, base, budget, t1, t2,
                                                                                t3);
     } else {
-        const i64 per = kEmitTilesPerWave;
+        const i64 per = std::min<i64>(std::max<i64>(ntiles / kEmitWaves, 1), kEmitTilesPerWave);
         k_cycle_emit<S><<<(unsigned)((ntiles + per - 1) / per), 64, 0, ctx.stream>>>(a, cnt8, tile_off, ntiles, per,
                                                                                      base, budget, t1, t2, t3);
     }

@@ -529,8 +529,8 @@ __device__ __forceinline__ void wave_lds_fence() {
 }
 
 // f(x) for the entries x of up to 16 lists, lane i of the group holding the
-// bounds [p0, p1) of list i (lists from cnt on are empty); the group's lanes share each list,
-// four lists are loaded at a time.
+// bounds [p0, p1) of list i (lists from cnt on are empty); the group's lanes
+// share each list, four lists are loaded at a time.
 template <class F>
 __device__ __forceinline__ void walk_lists(const CycArgs& a, int p0, int p1, int cnt, F f) {
     const int lane = threadIdx.x & (kSetLanes - 1);
@@ -554,42 +554,42 @@ __device__ __forceinline__ void walk_lists(const CycArgs& a, int p0, int p1, int
 template <class T, class F>
 __device__ __forceinline__ void find_in_lists(const CycArgs& a, int p0, int p1, int cnt, T test, F hit) {
     const int lane = threadIdx.x & (kSetLanes - 1);
-        for (int u0 = 0; u0 < cnt; u0 += 4) {  // uniform within the group
-            int s[4], e[4], x[4];
+    for (int u0 = 0; u0 < cnt; u0 += 4) {  // uniform within the group
+        int s[4], e[4], x[4];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                s[u] = __shfl(p0, u0 + u, kSetLanes);
-                e[u] = __shfl(p1, u0 + u, kSetLanes);
-                x[u] = s[u] + lane < e[u] ? a.adj[s[u] + lane] : -1;
-            }
-            unsigned hits = 0u, more = 0u;
+        for (int u = 0; u < 4; ++u) {
+            s[u] = __shfl(p0, u0 + u, kSetLanes);
+            e[u] = __shfl(p1, u0 + u, kSetLanes);
+            x[u] = s[u] + lane < e[u] ? a.adj[s[u] + lane] : -1;
+        }
+        unsigned hits = 0u, more = 0u;
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                hits |= x[u] >= 0 && test(x[u]) ? 1u << u : 0u;
-                more |= e[u] - s[u] > kSetLanes ? 1u << u : 0u;
-            }
-            auto pick = [](int v0, int v1, int v2, int v3, int u) {
-                const int lo = u & 1 ? v1 : v0, hi = u & 1 ? v3 : v2;
-                return u & 2 ? hi : lo;
-            };
-            for (; hits; hits &= hits - 1u) {
-                const int u = __builtin_ctz(hits);
-                hit(u0 + u, pick(s[0], s[1], s[2], s[3], u) + lane);
-            }
-            for (; more; more &= more - 1u) {
-                const int u = __builtin_ctz(more);
-                const int z = pick(e[0], e[1], e[2], e[3], u);
-                for (int k = pick(s[0], s[1], s[2], s[3], u) + kSetLanes + lane; k < z; k += 4 * kSetLanes) {
-                    int y[4];
+        for (int u = 0; u < 4; ++u) {
+            hits |= x[u] >= 0 && test(x[u]) ? 1u << u : 0u;
+            more |= e[u] - s[u] > kSetLanes ? 1u << u : 0u;
+        }
+        auto pick = [](int v0, int v1, int v2, int v3, int u) {
+            const int lo = u & 1 ? v1 : v0, hi = u & 1 ? v3 : v2;
+            return u & 2 ? hi : lo;
+        };
+        for (; hits; hits &= hits - 1u) {
+            const int u = __builtin_ctz(hits);
+            hit(u0 + u, pick(s[0], s[1], s[2], s[3], u) + lane);
+        }
+        for (; more; more &= more - 1u) {
+            const int u = __builtin_ctz(more);
+            const int z = pick(e[0], e[1], e[2], e[3], u);
+            for (int k = pick(s[0], s[1], s[2], s[3], u) + kSetLanes + lane; k < z; k += 4 * kSetLanes) {
+                int y[4];
 #pragma unroll
-                    for (int v = 0; v < 4; ++v) y[v] = k + v * kSetLanes < z ? a.adj[k + v * kSetLanes] : -1;
-                    unsigned far = 0u;
+                for (int v = 0; v < 4; ++v) y[v] = k + v * kSetLanes < z ? a.adj[k + v * kSetLanes] : -1;
+                unsigned far = 0u;
 #pragma unroll
-                    for (int v = 0; v < 4; ++v) far |= y[v] >= 0 && test(y[v]) ? 1u << v : 0u;
-                    for (; far; far &= far - 1u) hit(u0 + u, k + __builtin_ctz(far) * kSetLanes);
-                }
+                for (int v = 0; v < 4; ++v) far |= y[v] >= 0 && test(y[v]) ? 1u << v : 0u;
+                for (; far; far &= far - 1u) hit(u0 + u, k + __builtin_ctz(far) * kSetLanes);
             }
         }
+    }
 }
 
 // Adds c to the (saturating) count byte of expansion x, whose count is at

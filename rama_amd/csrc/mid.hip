@@ -8,9 +8,10 @@
 // more where matchings are long) whose sizes are read on the device: the host queues several rounds over buffers sized by the graph it
 // last saw, then reads one small state.  A round that the driver has to
 // handle itself (a conflicted cycle, a matching of more than six rounds, a
-// bucket too large for LDS, the switch to the spanning forest) raises the
-// state's stop word, and the launches queued behind it leave at once.  So does
-// the first matching of more than three rounds: from it on six are queued.
+// bucket too large for LDS, the switch to the spanning forest) raises an
+// outcome word of the state, and the launches queued behind it leave at once.
+// So does the first matching of more than three rounds: from it on six are
+// queued.
 //
 //   k_mid_begin    sums of the matching threshold, attractive neighbour lists
 //   k_mid_prune    (cycles of 4 and 5) the lists without their leaves
@@ -23,6 +24,13 @@
 //   k_mid_bucket   one block per bucket: stable LDS sort, runs of equal keys
 //                  summed
 //   k_mid_finish   compaction into the contracted graph, its CSR and state
+//
+// No launch stores an outcome word that it tests itself: its blocks start at
+// different times, and the waves of a late one could read the word differently
+// and part before a barrier.  `stop` is stored by the finish of the round before
+// (all of this round's launches test it), `found` by the cycle test, `ended` by
+// the keys and `skewed` by the scatter (only the launches behind test them); the
+// finish folds them into the next state's `stop`.
 //
 // The matching needs no matched flags: a vertex v is matched once
 // best[best[v]] == v, since matched vertices keep their best.  So a matching
@@ -440,7 +448,7 @@ __global__ __launch_bounds__(kMidThreads) void k_mid_keys(MidArgs a) {
     const int n = st->n, nf = st->nf, nblk = (n + kBlock - 1) / kBlock, found = st->found;
     if (st->stop) return;
     if (found) {
-        if (blockIdx.x == 0 && tid == 0) st->stop = kSmallCycles;
+        if (blockIdx.x == 0 && tid == 0) st->ended = kSmallCycles;
         return;
     }
     // the edges' ends and what the counts need are loaded together: a chain
@@ -488,9 +496,9 @@ __global__ __launch_bounds__(kMidThreads) void k_mid_keys(MidArgs a) {
         ended = nw == 0 || rel < 0.1f;
         matched = cur;
     }
-    const int stop = !ended ? kMidMatching : (matched == 0 ? kSmallDone : 0);
-    if (stop) {
-        if (blockIdx.x == 0 && tid == 0) st->stop = stop;
+    const int outcome = !ended ? kMidMatching : (matched == 0 ? kSmallDone : 0);
+    if (outcome) {
+        if (blockIdx.x == 0 && tid == 0) st->ended = outcome;
         return;
     }
     // first rank of every 256 vertices
@@ -586,7 +594,7 @@ __global__ __launch_bounds__(kMidThreads) void k_mid_scatter(MidArgs a) {
     __shared__ int ws[kMidWaves];
     __shared__ int over;
     MidState* st = a.st;
-    if (st->stop) return;
+    if (st->stop || st->ended) return;
     const int tid = threadIdx.x, lane = lane_id(), w = tid >> 6;
     const int nf = st->nf, kb = st->kb;
     const int ntiles = (nf + kMidTileEdges - 1) / kMidTileEdges;
@@ -631,7 +639,7 @@ __global__ __launch_bounds__(kMidThreads) void k_mid_scatter(MidArgs a) {
     }
     __syncthreads();
     if (over) {
-        if (blockIdx.x == 0 && tid == 0) st->stop = kMidSkew;
+        if (blockIdx.x == 0 && tid == 0) st->skewed = kMidSkew;
         return;
     }
     const int e0 = blockIdx.x * kMidTileEdges + w * 64 * kMidEdgeItems;
@@ -710,8 +718,8 @@ __global__ __launch_bounds__(kMidThreads) void k_mid_bucket(MidArgs a) {
     __shared__ int dstart[256];
     __shared__ int ws[kMidWaves];
     __shared__ int agg[8];
-    MidState* st = a.st;
-    if (st->stop) return;
+    const MidState* st = a.st;
+    if (st->stop || st->ended || st->skewed) return;
     const int tid = threadIdx.x, lane = lane_id(), w = tid >> 6, b = blockIdx.x;
     const int n = st->n, kb = st->kb;
     // labels of the nodes at entry, composed with this contraction
@@ -883,12 +891,14 @@ __global__ __launch_bounds__(kBlock) void k_mid_finish(MidArgs a) {
     __shared__ int ws[kWaves];
     __shared__ int base_s[2];
     __shared__ float wf[kWaves];
-    MidState* st = a.st;
+    const MidState* st = a.st;
     const int tid = threadIdx.x, b = blockIdx.x;
-    if (st->stop) {
+    if (st->stop || st->ended || st->skewed) {
         if (b == 0 && tid == 0) {
-            *a.nx = *st;
-            if (a.mirror) *a.mirror = *st;
+            MidState x = *st;
+            x.stop = x.stop ? x.stop : (x.ended ? x.ended : x.skewed);
+            *a.nx = x;
+            if (a.mirror) *a.mirror = x;
         }
         return;
     }
@@ -1046,7 +1056,13 @@ MidState mid_rounds(Ctx& ctx, DCoo& A, const Options& o, int iter, int first, in
     {
         MidState* s0 = states.get();
         const float* W = A.val.get();
-        const MidState init{0, iter, (int)nf0, n0, A.rows, A.cols, A.max_node, 0, 0, 0, 0, 0, 0.0f, 0.0f};
+        MidState init{};
+        init.iter = iter;
+        init.nf = (int)nf0;
+        init.n = n0;
+        init.rows = A.rows;
+        init.cols = A.cols;
+        init.max_node = A.max_node;
         int* L = lab.get();
         for_each(ctx, n0, [=] __device__(i64 v) {
             L[v] = (int)v;
@@ -1111,7 +1127,7 @@ MidState mid_rounds(Ctx& ctx, DCoo& A, const Options& o, int iter, int first, in
             MidState* s = states.get() + (queued & 1);
             for_each(ctx, 1, [=] __device__(i64) {
                 MidState x = *from;
-                x.stop = 0;
+                x.stop = x.ended = 0;
                 *s = x;
             });
             continue;

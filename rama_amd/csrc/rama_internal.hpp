@@ -234,10 +234,13 @@ enum MidReason : int {  // besides SmallReason's; 0: rounds still go on
     kMidSmall = 7,      // small enough for small_rounds
 };
 struct MidState {
-    int stop;
+    int stop;  // MidReason or SmallReason; set by the round before's finish
     int iter;  // the driver's round number after the rounds done
     int nf, n, rows, cols, max_node;
-    int found, any, matched, kb;
+    int found;   // this round's outcomes, each stored by one launch and tested by those behind it
+    int ended;
+    int skewed;
+    int any, matched, kb;
     int rounds;  // done since entry
     float thr, minw;
 };

@@ -17,6 +17,7 @@
 // triangle budget therefore keeps exactly the first `budget` writes.
 #include <cstdlib>
 #include <cstring>
+#include <optional>
 
 #include "rama_internal.hpp"
 #include "tuning.hpp"
@@ -50,8 +51,8 @@ struct CycArgs {
     // end of the expansions they covered ([1], a maximum).
     unsigned blk0 = 0;
     i64* counted = nullptr;
-    // 4- and 5-cycle counts: 1 if entries are looked up in the 2-hop sets, 0 if
-    // all are resolved; the queue of entries to resolve (kQueueParts parts of
+    // 4- and 5-cycle counts: 1 if they use their sets (lists and tables), 0 if
+    // every entry or expansion goes the general way; the queue of entries to resolve (kQueueParts parts of
     // qcap entries), its counters 128 bytes apart
     int sets = 1;
     int qcap = 0;
@@ -63,13 +64,24 @@ struct CycArgs {
 
 // Diagnostic switches (tests force each path on the same inputs; every
 // path gives the same counts and triangles):
-//   RAMA_CYCLE_TABLES=0   4- and 5-cycle counts without the 2-hop sets: every
-//                         list entry resolved against the lists
+//   RAMA_COUNT_FORM=sets | lists   the 4- and 5-cycle counts' form, instead of
+//                         the choice by what ends the count
+//   RAMA_CYCLE_TABLES=0   the same counts without their sets and tables: every
+//                         list entry resolved against the lists (sets form),
+//                         every expansion counted by its thread (lists form)
+//   RAMA_CYCLE_STATS=1    a line per 4- or 5-cycle count
 //   RAMA_EMIT_FORM=dense | queue   the emit form, instead of the choice by
 //                         the share of expansions with mids
 static bool cycle_tables_on() {
     const char* e = std::getenv("RAMA_CYCLE_TABLES");
     return !(e && e[0] == '0' && e[1] == 0);
+}
+static int count_form_forced() {  // 0: choose, 1: sets, 2: lists
+    const char* e = std::getenv("RAMA_COUNT_FORM");
+    if (!e) return 0;
+    if (std::strcmp(e, "sets") == 0) return 1;
+    if (std::strcmp(e, "lists") == 0) return 2;
+    return 0;
 }
 static int emit_form_forced() {  // 0: choose, 1: dense, 2: queue
     const char* e = std::getenv("RAMA_EMIT_FORM");
@@ -80,7 +92,8 @@ static int emit_form_forced() {  // 0: choose, 1: dense, 2: queue
 }
 
 // Adds the block's attempted writes to its counter line's [0] and raises
-// its [1] to the end of its expansions.  The counters are spread over
+// its [1] to the end of its expansions ([2]: entries the sets form resolved).
+// The counters are spread over
 // kCountedLines lines of 16 i64 (128 bytes): device atomics from every block
 // to one address serialise; the host sums the [0]s and takes the largest
 // [1].  Block-uniform call.
@@ -231,6 +244,23 @@ constexpr int kProbe = 16;
 __device__ __forceinline__ int probe_count(const int* __restrict__ adj, int sb, int se, int lb, int le) {
     int c = 0;
     for (int i = sb; i < se; ++i) c += has_partner(adj, sb, i, adj[i], lb, le) ? 1 : 0;
+    return c;
+}
+
+// count_common of the lists [ia, ie) and [ib, ib + nb) by one lane: from
+// the shorter list by binary searches when the pair is heavy and that list
+// is short, else the merge walk.
+__device__ __forceinline__ int lane_count_common(const int* __restrict__ adj, int ia, int ie, int ib, int nb) {
+    const int na = ie - ia;
+    if (na + nb > kHeavy && min(na, nb) <= kProbe)
+        return na <= nb ? probe_count(adj, ia, ie, ib, ib + nb) : probe_count(adj, ib, ib + nb, ia, ie);
+    int i = ia, j = ib, je = ib + nb, c = 0;
+    while (i < ie && j < je) {
+        const int x = adj[i], y = adj[j];
+        c += (x == y);
+        i += (x <= y);
+        j += (y <= x);
+    }
     return c;
 }
 
@@ -468,7 +498,510 @@ __global__ __launch_bounds__(kFewThreads) void k_cycle_count3_few(CycArgs a, uns
     }
 }
 
-// 4- and 5-cycles.  Expansions of rep edge r = (v1, v2) are xoff[r] ..
+// Adds `v` to the total of the tile holding expansion x, flushing the
+// running sum whenever the thread's expansions cross into the next tile.
+struct TileAcc {
+    i64 tile = -1;
+    i64 sum = 0;
+    __device__ __forceinline__ void add(i64* tot, i64 x, i64 v) {
+        const i64 t = x / kCycTile;
+        if (t != tile) {
+            flush(tot);
+            tile = t;
+        }
+        sum += v;
+    }
+    __device__ __forceinline__ void flush(i64* tot) {
+        if (tile >= 0 && sum != 0)
+            atomicAdd(reinterpret_cast<unsigned long long*>(tot + tile), (unsigned long long)sum);
+        sum = 0;
+    }
+};
+
+// 4- and 5-cycle counts, lists form (the sets form and the choice follow).
+//
+// 4-cycles: one thread per repulsive edge; its expansions n1 ∈ N(v1) are
+// xoff[r] .. xoff[r+1]-1 in order, each intersecting N(n1) with N(v2)
+// (held in registers).  tile_tot must be zero on entry.
+// Rep edges whose v1 has at least kWideRep neighbours, or whose v2 has more
+// than kRegList, are counted by the whole wave, one rep edge at a time: the
+// wave puts N(v2) in an LDS hash set (kSetSlots slots, lists of at most
+// kSetMax entries) and lane l takes expansions l, l + 64, ..., streaming
+// N(n1) and probing each entry.  After contraction supernodes have dozens
+// of neighbours: one lane per rep edge would walk long merge walks serially
+// while its wave waits.  A repeated value in either list (the min(a, b)
+// rule) or a longer N(v2) keeps the merge walk for that expansion.
+constexpr int kWideRep = 48;
+constexpr int kSetSlots = 256;
+constexpr int kSetMax = 128;
+
+__device__ __forceinline__ int set_hash(int m) { return (int)(((unsigned)m * 2654435761u) >> 24); }
+
+__global__ __launch_bounds__(kBlock) void k_cycle_count4(CycArgs a, unsigned char* __restrict__ cnt8,
+                                                         i64* __restrict__ tile_tot) {
+    __shared__ int wset[kWaves][4 * kSetSlots];
+    const int w = threadIdx.x >> 6;
+    const i64 r = (i64)(a.blk0 + xcd_block()) * kBlock + threadIdx.x;
+    const bool on = r < a.R;
+    i64 mine = 0, xend = 0;
+    int v1 = 0, v2 = 0, b1 = 0, d1 = 0, b2 = 0, n2 = 0;
+    i64 x0 = 0;
+    if (on) {
+        v1 = a.rv1[r];
+        v2 = a.rv2[r];
+        b1 = a.off[v1];
+        d1 = a.off[v1 + 1] - b1;
+        b2 = a.off[v2];
+        n2 = a.off[v2 + 1] - b2;
+        x0 = a.xoff[r];
+        xend = x0 + d1;
+    }
+    const bool wide = on && a.sets && (d1 >= kWideRep || n2 > kRegList);
+    if (on && !wide) {
+        int rb[kRegList];
+        const bool regs = n2 <= kRegList;
+        int rmax = -1, kw = kRegList;
+        bool rdup = false;
+        if (regs) {
+            load_reg_list(a.adj, b2, n2, rb);
+            reg_list_props(rb, n2, rmax, rdup);
+            kw = reg_width(n2);
+        }
+        TileAcc acc;
+        // the next n1's list bounds are loaded while this one is walked
+        int ia = 0, ie = 0;
+        if (d1 > 0) {
+            const int n1 = a.adj[b1];
+            ia = a.off[n1];
+            ie = a.off[n1 + 1];
+        }
+        for (int l = 0; l < d1; ++l) {
+            int na = 0, ne = 0;
+            if (l + 1 < d1) {
+                const int nn = a.adj[b1 + l + 1];
+                na = a.off[nn];
+                ne = a.off[nn + 1];
+            }
+            const int c = regs ? count_vs_regs_fast(a.adj, ia, ie, rb, rmax, rdup, kw)
+                               : lane_count_common(a.adj, ia, ie, b2, n2);
+            cnt8[x0 + l] = (unsigned char)(c < 255 ? c : 255);
+            acc.add(tile_tot, x0 + l, 2 * (i64)c);
+            mine += 2 * (i64)c;
+            ia = na;
+            ie = ne;
+        }
+        acc.flush(tile_tot);
+    }
+    // wide rep edges: the wave works as four groups of 16 lanes, group g
+    // taking the wide rep edges of lanes 16g .. 16g + 15 one after another
+    // (four rep edges in flight per wave); the attempted writes are credited
+    // to the rep's own lane (its instance, its block total)
+    const int lane = lane_id(), g = lane >> 4, gl = lane & 15;
+    const unsigned long long wm = __ballot(wide);
+    unsigned gm = (unsigned)((wm >> (16 * g)) & 0xffffull);  // this group's wide lanes
+    int niter = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) niter = max(niter, __popcll((wm >> (16 * q)) & 0xffffull));
+    int* gset = &wset[w][g * kSetSlots];
+    const unsigned long long gmask = 0xffffull << (16 * g);
+    for (int it = 0; it < niter; ++it) {
+        const bool gact = gm != 0u;  // uniform within the group
+        const int h = gact ? 16 * g + __builtin_ctz(gm) : lane;
+        if (gact) gm &= gm - 1u;
+        const int hb1 = __shfl(b1, h, 64), hd1 = gact ? __shfl(d1, h, 64) : 0;
+        const int hb2 = __shfl(b2, h, 64), hn2 = gact ? __shfl(n2, h, 64) : 0;
+        const i64 hx0 = __shfl(x0, h, 64);
+        // N(v2) into the group's set (a repeated value, or too long a list:
+        // merge walks instead)
+        bool use_set = gact && hn2 <= kSetMax;
+        int vmax = -1;
+        bool dup = false;
+        if (use_set) {
+            for (int k = gl; k < kSetSlots; k += 16) gset[k] = -1;
+        }
+        __builtin_amdgcn_wave_barrier();
+        if (use_set) {
+            for (int k = gl; k < hn2; k += 16) {
+                const int m = a.adj[hb2 + k];
+                dup |= k > 0 && a.adj[hb2 + k - 1] == m;
+                int hs = set_hash(m);
+                while (true) {
+                    const int old = atomicCAS(&gset[hs], -1, m);
+                    if (old == -1 || old == m) break;
+                    hs = (hs + 1) & (kSetSlots - 1);
+                }
+            }
+            vmax = hn2 > 0 ? a.adj[hb2 + hn2 - 1] : -1;
+        }
+        use_set = use_set && (__ballot(dup) & gmask) == 0ull;
+        __builtin_amdgcn_wave_barrier();
+        TileAcc acc;
+        i64 part = 0;
+        for (int l = gl; l < hd1; l += 16) {
+            const int n1 = a.adj[hb1 + l];
+            const int ia = a.off[n1], ie = a.off[n1 + 1];
+            int c = 0;
+            bool merge = !use_set;
+            if (use_set) {
+                // four entries per round of loads (past the end reads as
+                // above vmax), walked in order up to the first above vmax
+                int prev = -1;
+                bool stop = false;
+                for (int k = ia; k < ie && !stop; k += 4) {
+                    int xs[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) xs[u] = k + u < ie ? a.adj[k + u] : 0x7fffffff;
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        const int x = xs[u];
+                        if (stop || x > vmax) {
+                            stop = true;
+                            continue;
+                        }
+                        if (x == prev) {  // N(n1) repeats a value: the merge walk counts it
+                            merge = true;
+                            stop = true;
+                            continue;
+                        }
+                        prev = x;
+                        int hs = set_hash(x);
+                        while (true) {
+                            const int key = gset[hs];
+                            if (key == x) {
+                                ++c;
+                                break;
+                            }
+                            if (key == -1) break;
+                            hs = (hs + 1) & (kSetSlots - 1);
+                        }
+                    }
+                }
+            }
+            if (merge) c = lane_count_common(a.adj, ia, ie, hb2, hn2);
+            cnt8[hx0 + l] = (unsigned char)(c < 255 ? c : 255);
+            acc.add(tile_tot, hx0 + l, 2 * (i64)c);
+            part += 2 * (i64)c;
+        }
+        acc.flush(tile_tot);
+#pragma unroll
+        for (int d = 8; d >= 1; d >>= 1) part += __shfl_xor(part, d, 64);  // within the group
+        if (gact && lane == h) mine += part;
+        __builtin_amdgcn_wave_barrier();
+    }
+    if (a.nslot) wave_add_keyed(a.slot_total, on ? a.nslot[v1] : 0, mine, on);
+    if (a.counted) block_counted(a.counted, mine, xend);
+}
+
+// 5-cycles: one thread per (repulsive edge r, n2 = l2-th neighbour of v2);
+// its expansions (n1 = l1-th neighbour of v1, n2) are xoff[r] + l2*d1 + l1
+// for l1 = 0 .. d1-1, each intersecting N(n1) with N(n2); n1 == n2 is
+// skipped.  Threads of rep r are yoff[r] .. yoff[r+1]-1; ytile_rep gives
+// each block's first rep.  tile_tot must be zero on entry.
+//
+// Two ways to count one thread's d1 expansions, with identical counts:
+//  * 2-hop table (the common case): the block builds, for each distinct v1
+//    among its threads, an LDS hash table of v1's 2-hop neighbourhood,
+//    mid -> bitmask of the l1 whose list N(n1) holds mid.  The thread then
+//    walks N(n2) once, looks every mid up and adds its mask to bit-sliced
+//    per-l1 counters, instead of streaming every N(n1) against N(n2).  Valid
+//    when no list involved holds a value twice (then |N(n1) ∩ N(n2)| is the
+//    merge walk's min(a, b) count), d1 <= 32 and the 2-hop lists fit.
+//  * per expansion (otherwise): N(n2) in registers (or the merge walk /
+//    probes for long lists), each N(n1) streamed against it.
+constexpr int kT5Tables = 16;      // 2-hop tables (distinct v1 runs) per block
+constexpr int kT5SlotBits = 11;
+constexpr int kT5Slots = 1 << kT5SlotBits;  // slots of the block's shared hash table
+constexpr int kT5MaxFill = 1536;   // entries of all tables together at most this (load <= 3/4)
+constexpr int kT5MaxD1 = 32;       // d(v1) at most this (32-bit masks)
+constexpr int kT5RepWin = 256;     // rep edges a block locates its threads among in LDS
+constexpr int kT5MaxNode = 1 << 27;  // node ids below this: (mid, run) fits one key
+
+// The tables of a block share one open-addressing hash table of keys
+// mid * kT5Tables + run.
+__device__ __forceinline__ int t5_hash(int key) {
+    return (int)(((unsigned)key * 2654435761u) >> (32 - kT5SlotBits));
+}
+
+// The per-expansion form for one thread (see above).
+__device__ __forceinline__ void count5_direct(const CycArgs& a, int b1, int d1, int n2, int bq, int nq, i64 x0,
+                                              unsigned char* __restrict__ cnt8, i64* __restrict__ tile_tot,
+                                              i64& mine) {
+    int rb[kRegList];
+    const bool regs = nq <= kRegList;
+    int rmax = -1, kw = kRegList;
+    bool rdup = false;
+    if (regs) {
+        load_reg_list(a.adj, bq, nq, rb);
+        reg_list_props(rb, nq, rmax, rdup);
+        kw = reg_width(nq);
+    }
+    TileAcc acc;
+    // the next n1 and its list bounds are loaded while this one is walked
+    int n1 = d1 > 0 ? a.adj[b1] : 0;
+    int ia = d1 > 0 ? a.off[n1] : 0, ie = d1 > 0 ? a.off[n1 + 1] : 0;
+    for (int l = 0; l < d1; ++l) {
+        const int nn = l + 1 < d1 ? a.adj[b1 + l + 1] : 0;
+        const int na = l + 1 < d1 ? a.off[nn] : 0, ne = l + 1 < d1 ? a.off[nn + 1] : 0;
+        int c = 0;
+        if (n1 != n2)
+            c = regs ? count_vs_regs_fast(a.adj, ia, ie, rb, rmax, rdup, kw)
+                     : lane_count_common(a.adj, ia, ie, bq, nq);
+        cnt8[x0 + l] = (unsigned char)(c < 255 ? c : 255);
+        acc.add(tile_tot, x0 + l, 3 * (i64)c);
+        mine += 3 * (i64)c;
+        n1 = nn;
+        ia = na;
+        ie = ne;
+    }
+    acc.flush(tile_tot);
+}
+
+__global__ __launch_bounds__(kBlock) void k_cycle_count5(CycArgs a, const i64* __restrict__ yoff,
+                                                         const int* __restrict__ ytile_rep, i64 Y, int tables,
+                                                         unsigned char* __restrict__ cnt8,
+                                                         i64* __restrict__ tile_tot) {
+    __shared__ int tkey[kT5Slots];
+    __shared__ unsigned tmask[kT5Slots];
+    __shared__ int tv1[kT5Tables];
+    __shared__ int tok[kT5Tables];
+    __shared__ int tfill[kT5Tables];
+    __shared__ int sv1[kBlock];
+    __shared__ int wruns[kWaves];
+    const unsigned blk = a.blk0 + xcd_block();
+    const int tid = threadIdx.x, lane = lane_id(), w = tid >> 6;
+    const i64 y = (i64)blk * kCycTile + tid;
+    const bool on = y < Y;
+    i64 mine = 0, xend = 0;
+    int slot = 0;
+    int v1 = -1, b1 = 0, d1 = 0, n2 = 0, bq = 0, nq = 0;
+    i64 x0 = 0;
+    // rep owning each thread: the block's threads belong to reps r0, r0 + 1,
+    // ...; their thread offsets are loaded once (coalesced) and every thread
+    // marks where its rep starts, so a block max-scan (kept as a running max
+    // over the marks) hands each thread its rep.  Blocks whose threads span
+    // more than kT5RepWin reps fall back to a galloping search.
+    const i64 y0 = (i64)blk * kCycTile;
+    const i64 r0 = y0 < Y ? (i64)ytile_rep[blk] : 0;
+    sv1[tid] = -1;
+    __syncthreads();
+    bool wide = false;
+    for (int k = tid; k < kT5RepWin; k += kBlock) {
+        const i64 r = r0 + k;
+        if (r < a.R) {
+            const i64 ys = yoff[r];
+            if (ys >= y0 && ys < y0 + kCycTile && yoff[r + 1] > ys) sv1[ys - y0] = k;
+        }
+    }
+    if (y0 < Y) {
+        const i64 rl = r0 + kT5RepWin - 1;
+        wide = rl < a.R && yoff[rl + 1] < (y0 + kCycTile < Y ? y0 + kCycTile : Y);
+    }
+    __syncthreads();
+    int mark = sv1[tid];
+    // inclusive max-scan of the marks over the block (first thread: its rep
+    // r0 starts before the block, mark 0)
+    if (tid == 0 && mark < 0) mark = 0;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int t = __shfl_up(mark, d, 64);
+        if (lane >= d) mark = max(mark, t);
+    }
+    __shared__ int wmax[kWaves];
+    if (lane == 63) wmax[w] = mark;
+    __syncthreads();
+    for (int q = 0; q < w; ++q) mark = max(mark, wmax[q]);
+    __syncthreads();
+    if (on) {
+        i64 r = r0 + mark;
+        if (wide) {
+            // rep owning thread y (galloping from the block's first rep)
+            i64 lo = r0, hi = a.R - 1, step = 1;
+            while (lo + step <= hi && yoff[lo + step] <= y) {
+                lo += step;
+                step <<= 1;
+            }
+            hi = lo + step < a.R - 1 ? lo + step : a.R - 1;
+            while (lo < hi) {
+                const i64 mid = (lo + hi + 1) >> 1;
+                if (yoff[mid] <= y) lo = mid; else hi = mid - 1;
+            }
+            r = lo;
+        }
+        v1 = a.rv1[r];
+        const int v2 = a.rv2[r];
+        const int l2 = (int)(y - yoff[r]);
+        b1 = a.off[v1];
+        d1 = a.off[v1 + 1] - b1;
+        n2 = a.adj[a.off[v2] + l2];
+        bq = a.off[n2];
+        nq = a.off[n2 + 1] - bq;
+        x0 = a.xoff[r] + (i64)l2 * d1;
+        if (a.nslot) slot = a.nslot[v1];
+    }
+    // runs of equal v1 over the block's threads (rep edges are in row order,
+    // so a run is usually all threads of one v1); run k < kT5Tables gets
+    // table k
+    sv1[tid] = v1;
+    for (int k = tid; k < kT5Slots; k += kBlock) {
+        tkey[k] = -1;
+        tmask[k] = 0u;
+    }
+    __syncthreads();
+    const bool start = on && (tid == 0 || sv1[tid - 1] != v1);
+    const unsigned long long sm = __ballot(start);
+    if (lane == 0) wruns[w] = __popcll(sm);
+    __syncthreads();
+    int before = 0, runs = 0;
+    for (int q = 0; q < kWaves; ++q) {
+        before += q < w ? wruns[q] : 0;
+        runs += wruns[q];
+    }
+    // this thread's run index (its run starts at or before it)
+    const int run = before + __popcll(sm & ((2ull << lane) - 1ull)) - 1;
+    if (start && run < kT5Tables) {
+        tv1[run] = v1;
+        tok[run] = 1;
+    }
+    const int ntab = runs < kT5Tables ? runs : kT5Tables;
+    __syncthreads();
+    // build, in three steps: each wave sizes its tables (w, w + kWaves, ...:
+    // lane l holds the bounds of the list of v1's l-th neighbour n1); the
+    // tables that fit the shared capacity in run order are kept; each wave
+    // inserts its kept tables' (mid, l) pairs, flattened over its 64 lanes
+    constexpr int kPerWave = kT5Tables / kWaves;
+    int s0[kPerWave], s1[kPerWave];
+#pragma unroll
+    for (int i = 0; i < kPerWave; ++i) {
+        const int k = w + i * kWaves;
+        s0[i] = s1[i] = 0;
+        if (k >= ntab) continue;
+        const int v = tv1[k];
+        const int bv = a.off[v], dv = a.off[v + 1] - bv;
+        if (dv <= kT5MaxD1 && lane < dv) {
+            const int n1 = a.adj[bv + lane];
+            s0[i] = a.off[n1];
+            s1[i] = a.off[n1 + 1];
+        }
+        int fill = s1[i] - s0[i];
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) fill += __shfl_xor(fill, d, 64);
+        if (lane == 0) tfill[k] = dv <= kT5MaxD1 && tables ? fill : kT5MaxFill + 1;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        int used = 0;
+        for (int k = 0; k < ntab; ++k) {
+            const bool fits = used + tfill[k] <= kT5MaxFill;
+            tok[k] = fits ? 1 : 0;
+            used += fits ? tfill[k] : 0;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kPerWave; ++i) {
+        const int k = w + i * kWaves;
+        if (k >= ntab || !tok[k]) continue;  // wave-uniform
+        bool dup = false;
+        const int fill = tfill[k];
+        const int len = s1[i] - s0[i];
+        int excl = len;  // where list l starts among the table's pairs
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int t = __shfl_up(excl, d, 64);
+            if (lane >= d) excl += t;
+        }
+        excl -= len;
+        const int dv = a.off[tv1[k] + 1] - a.off[tv1[k]];
+        for (int f0 = 0; f0 < fill; f0 += 64) {  // wave-uniform: every lane takes part in the shuffles
+            const int f = f0 + lane;
+            int l = 0;
+            for (int j = 1; j < dv; ++j) l = __builtin_amdgcn_readlane(excl, j) <= f ? j : l;
+            const int q = __shfl(s0[i], l, 64) + (f - __shfl(excl, l, 64));
+            if (f >= fill) continue;
+            const int key = a.adj[q] * kT5Tables + k;
+            const unsigned bit = 1u << l;
+            int h = t5_hash(key);
+            while (true) {
+                const int old = atomicCAS(&tkey[h], -1, key);
+                if (old == -1 || old == key) {
+                    dup |= (atomicOr(&tmask[h], bit) & bit) != 0u;
+                    break;
+                }
+                h = (h + 1) & (kT5Slots - 1);
+            }
+        }
+        // a list that repeats a value disables its table
+        if (__ballot(dup) != 0ull && lane == 0) tok[k] = 0;
+    }
+    __syncthreads();
+    if (on) {
+        const bool table = run < ntab && tok[run] && nq <= 255;
+        bool direct = !table;
+        if (table) {
+            // per-l1 counts of N(n2)'s mids, bit-sliced over 8 planes
+            unsigned p[8] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
+            int prev = -1;
+            // four entries of N(n2) per round of loads
+            for (int q0 = bq; q0 < bq + nq && !direct; q0 += 4) {
+                int ms[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) ms[u] = q0 + u < bq + nq ? a.adj[q0 + u] : -1;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    if (direct || q0 + u >= bq + nq) continue;
+                    const int m = ms[u];
+                    if (m == prev) {  // N(n2) repeats a value: the min(a, b) rule needs the direct form
+                        direct = true;
+                        continue;
+                    }
+                    prev = m;
+                    const int want = m * kT5Tables + run;
+                    int h = t5_hash(want);
+                    unsigned mk = 0u;
+                    while (true) {
+                        const int key = tkey[h];
+                        if (key == want) {
+                            mk = tmask[h];
+                            break;
+                        }
+                        if (key == -1) break;
+                        h = (h + 1) & (kT5Slots - 1);
+                    }
+#pragma unroll
+                    for (int b = 0; b < 8; ++b) {
+                        const unsigned carry = p[b] & mk;
+                        p[b] ^= mk;
+                        mk = carry;
+                    }
+                }
+            }
+            if (!direct) {
+                unsigned nz = 0u;
+#pragma unroll
+                for (int b = 0; b < 8; ++b) nz |= p[b];
+                TileAcc acc;
+                for (int l = 0; l < d1; ++l) {
+                    int c = 0;
+                    if ((nz >> l) & 1u) {
+#pragma unroll
+                        for (int b = 0; b < 8; ++b) c |= (int)((p[b] >> l) & 1u) << b;
+                        if (a.adj[b1 + l] == n2) c = 0;
+                    }
+                    cnt8[x0 + l] = (unsigned char)(c < 255 ? c : 255);
+                    acc.add(tile_tot, x0 + l, 3 * (i64)c);
+                    mine += 3 * (i64)c;
+                }
+                acc.flush(tile_tot);
+            }
+        }
+        if (direct) count5_direct(a, b1, d1, n2, bq, nq, x0, cnt8, tile_tot, mine);
+        xend = x0 + d1;
+    }
+    if (a.nslot) wave_add_keyed(a.slot_total, slot, mine, on);
+    if (a.counted) block_counted(a.counted, mine, xend);
+}
+
+// 4- and 5-cycle counts, sets form.  Expansions of rep edge r = (v1, v2) are xoff[r] ..
 // xoff[r+1]-1: for 4-cycles the neighbours n1 of v1 (l1 = 0 .. d1-1), each
 // intersecting N(n1) with N(v2); for 5-cycles the pairs (n1, n2) at
 // l2 * d1 + l1, each intersecting N(n1) with N(n2), n1 == n2 left out.
@@ -492,11 +1025,9 @@ __global__ __launch_bounds__(kFewThreads) void k_cycle_count3_few(CycArgs a, uns
 // listed, and a launch of blocks takes a few of them each with a set of
 // kBigWords words.
 //
-// One thread per rep edge walking every N(n1) against N(v2) in registers, or
-// per (rep edge, n2) through per-block hash tables, took 9300 vector
-// instructions per wave and waited on the longest of its lanes' lists.  D mode
-// on the 12.47M-edge grid, all 4- and 5-cycle counts of a solve: 54.5 + 59.7 ms
-// so, 14 + 36 with the sets (a full pass: 9.3M rep edges and 100M expansions
+// The lists form takes 9300 vector instructions per wave there and waits on the
+// longest of its lanes' lists.  D mode on the 12.47M-edge grid, all 4- and 5-cycle
+// counts of a solve: 54.5 + 59.7 ms by lists, 14 + 36 with the sets (a full pass: 9.3M rep edges and 100M expansions
 // 5.0 -> 1.4 ms, 1.1G expansions 11 -> 8.2); the 192^3 grid's PD+ 14.0 + 8.1 ->
 // 11.0 + 7.7.  5-cycles are bound by the lists' load latency at 5 waves per SIMD
 // and by about 60 instructions per step of four lists.
@@ -680,7 +1211,11 @@ template <int S>
 __global__ __launch_bounds__(kBlock) void k_cycle_resolve(CycArgs a, i64 r0, unsigned char* __restrict__ cnt8,
                                                           i64* __restrict__ tile_tot) {
     const int part = blockIdx.x % kQueueParts, step = (int)(gridDim.x / kQueueParts) * kBlock;
-    const int n = (int)min(a.qcount[part * 32], (unsigned)a.qcap);
+    const unsigned passed = a.qcount[part * 32];  // those past the queue's end were resolved at once
+    const int n = (int)min(passed, (unsigned)a.qcap);
+    if (a.counted && blockIdx.x < kQueueParts && threadIdx.x == 0)
+        atomicAdd(reinterpret_cast<unsigned long long*>(a.counted + part % kCountedLines * 16 + 2),
+                  (unsigned long long)passed);
     i64 mine = 0;
     for (int q0 = (int)(blockIdx.x / kQueueParts) * kBlock; q0 < n; q0 += step) {  // uniform
         const int q = q0 + (int)threadIdx.x;
@@ -1345,6 +1880,29 @@ static void launch_count3(Ctx& ctx, const CycArgs& a, unsigned ntiles, unsigned 
     RAMA_LAUNCHED();
 }
 
+// Which form counts a single instance's 4- or 5-cycles.  The sets form pays
+// about 1.2 ns per entry that passes its filter (true mids, and the filter's own
+// errors where 2-hop neighbourhoods are large), the lists form 20 to 50 ps per
+// expansion of short lists (5-cycles, through the 2-hop tables) and 300 ps of
+// long ones.  So the count starts with the sets and goes over to the lists once
+// a chunk has passed on that many entries per expansion: full 5-cycle counts of
+// a random graph of degree 20 (5% and more pass) 14.4 ms by sets, 6.2 by lists,
+// of a 12-nearest-neighbour graph (two mids per expansion) 2.7 and 0.14, of a
+// random graph of degree 8 0.38 and 0.85.  A few thousand rep edges of short
+// lists start with the lists (a launch of 378 at a mid per expansion 17 ms by
+// sets, whose few groups resolve them in turn, and 0.27).  Where the count may go
+// on past kFewWrites writes per rep edge, as verbose ones do, the first chunk is
+// smaller, and long lists too are walked from the start.  A pack's counts run to
+// the end over all kinds of instances and take the lists (48 mixed instances,
+// PD+: 5.3 s by sets, 1.2 by lists).
+template <int S>
+constexpr i64 kShortLists = S == 4 ? 32 : 1024;  // expansions per rep edge, on average
+template <int S>
+constexpr double kDenseShare = S == 4 ? 0.25 : 0.03125;
+constexpr double kDenseLong = 0.25;
+constexpr i64 kFewReps45 = 8192;
+constexpr i64 kFewWrites = 4;
+
 // Before a 4- or 5-cycle count, in one launch (a memset each costs the host
 // more than this kernel): tile_rep[t] = rep edge containing the first expansion
 // of tile t; tile totals, count bytes (whole 16-byte words) and counters
@@ -1448,11 +2006,11 @@ struct CountQueue {
 };
 // k_count_begin for a stage of R rep edges and a.X expansions.
 static void count_begin(Ctx& ctx, const CycArgs& a, int* tile_rep, i64* tile, unsigned char* cnt8) {
-    const i64 ntiles = (a.X + kCycTile - 1) / kCycTile, words = (a.X + 15) / 16;
-    const i64 n = std::max<i64>(std::max<i64>(a.R, words), (kQueueParts + 1) * 32);
+    const i64 ntiles = (a.X + kCycTile - 1) / kCycTile, words = cnt8 ? (a.X + 15) / 16 : 0;
+    const i64 n = std::max<i64>(std::max<i64>(a.R, std::max(words, ntiles)), (kQueueParts + 1) * 32);
     k_count_begin<<<(unsigned)std::min<i64>((n + kBlock - 1) / kBlock, 4096), kBlock, 0, ctx.stream>>>(
         a.xoff, a.R, tile_rep, tile, ntiles, reinterpret_cast<uint4*>(cnt8), words, a.counted,
-        a.counted ? kCountedLines * 16 : 0, a.qcount, (kQueueParts + 1) * 32);
+        a.counted ? kCountedLines * 16 : 0, a.qcount, a.qcount ? (kQueueParts + 1) * 32 : 0);
     RAMA_LAUNCHED();
 }
 // Counts blocks [a.blk0, a.blk0 + n) of `reps` rep edges.
@@ -1470,6 +2028,55 @@ static void count_blocks(Ctx& ctx, const CycArgs& a, unsigned n, int reps, unsig
     k_cycle_resolve<S><<<kQueueParts * per_part, kBlock, 0, ctx.stream>>>(a, r0, cnt8, tile);
     RAMA_LAUNCHED();
 }
+
+// Counts rep edges [r0, a.R) by walking lists, after k_count_begin has cleared
+// the count bytes and tile totals, in launches of nblk blocks in all.
+template <int S>
+struct CountLists {
+    CycArgs a;  // of the rep edges from r0 on
+    DBuf<i64> yoff;
+    DBuf<int> ytile_rep;
+    i64 Y = 0;
+    unsigned nblk = 0;
+    int tables = 0;
+    CountLists(Ctx& ctx, const CycArgs& all, i64 r0, int n_nodes) : a(all) {
+        a.rv1 += r0;
+        a.rv2 += r0;
+        a.xoff += r0;
+        a.R -= r0;
+        if (S == 4) {
+            nblk = grid_for(a.R);
+            return;
+        }
+        // thread space: one thread per (rep edge, neighbour of v2)
+        tables = a.sets && n_nodes < kT5MaxNode ? 1 : 0;
+        yoff = ctx.buf<i64>(a.R + 1);
+        const int* OFF = a.off;
+        const int* rv2 = a.rv2;
+        i64* ym = ctx.mirror<i64>();
+        scan_exclusive<i64>(ctx, [=] __device__(i64 r) { const int u = rv2[r]; return (i64)(OFF[u + 1] - OFF[u]); },
+                            yoff.get(), a.R, ym);
+        ctx.read_mirror(yoff.get() + a.R, ym, &Y);
+        const i64 ytiles = (Y + kCycTile - 1) / kCycTile;
+        RAMA_REQUIRE(ytiles < ((i64)1 << 31), "too many cycle expansions");
+        nblk = (unsigned)ytiles;
+        if (Y == 0) return;
+        ytile_rep = ctx.buf<int>(ytiles);
+        k_count_begin<<<(unsigned)std::min<i64>((a.R + kBlock - 1) / kBlock, 4096), kBlock, 0, ctx.stream>>>(
+            yoff.get(), a.R, ytile_rep.get(), nullptr, 0, nullptr, 0, nullptr, 0, nullptr, 0);
+        RAMA_LAUNCHED();
+    }
+    // Blocks [first, first + n).
+    void run(Ctx& ctx, unsigned first, unsigned n, unsigned char* cnt8, i64* tile) {
+        if (n == 0) return;
+        a.blk0 = first;
+        if (S == 4)
+            k_cycle_count4<<<n, kBlock, 0, ctx.stream>>>(a, cnt8, tile);
+        else
+            k_cycle_count5<<<n, kBlock, 0, ctx.stream>>>(a, yoff.get(), ytile_rep.get(), Y, tables, cnt8, tile);
+        RAMA_LAUNCHED();
+    }
+};
 
 // Runs one stage over all expansions; returns the number of attempted writes.
 template <int S>
@@ -1532,52 +2139,101 @@ static i64 run_stage(Ctx& ctx, const Csr& G, const int* rv1, const int* rv2, i64
     // later decision are those of a full count.  Only the returned total is
     // then a lower bound of the full one; verbose runs count everything, as
     // they print it.
+    //
+    // The chunks take the sets form as long as few entries pass, the lists form
+    // from there on (kDenseShare).
     i64 tiles_used = ntiles;
     if constexpr (S > 3) {
         DBuf<i64> cnt = ctx.buf<i64>(kCountedLines * 16);
         a.counted = cnt.get();
-        const int reps = count_reps(R);
-        const unsigned nblk = (unsigned)((R + reps - 1) / reps);
-        CountQueue queue(ctx, S, R, X, a);
-        count_begin(ctx, a, tile_rep.get(), tile.get(), cnt8.get());
+        const int forced = count_form_forced();
         const bool early = !ctx.verbose && budget > base;
         const i64 need = budget - base;
-        // the first chunk: a sixteenth of the blocks (a count that runs to
-        // the end pays this launch's tail once; smaller first chunks cost D
-        // mode on the 2D grid 5 ms, larger ones overshoot budgets)
-        unsigned done = 0, chunk = early ? std::max<unsigned>(nblk / 16, 256u) : nblk;
-        i64 hc[2] = {0, X};
-        while (done < nblk) {
-            const unsigned n = std::min(chunk, nblk - done);
-            a.blk0 = done;
-            if (work_on) {
-                const i64 lo = (i64)done * reps, hi = std::min<i64>((i64)(done + n) * reps, R);
-                count_work<S>(ctx, G, rv1, rv2, nsum.get(), lo, hi, wx, wy);
+        const bool few = early && need <= kFewWrites * R, lengthy = X > kShortLists<S> * R;
+        const bool sets = forced ? forced == 1 : !(lengthy ? !few : R < kFewReps45);
+        std::optional<CountQueue> queue;  // of the sets form
+        if (sets) queue.emplace(ctx, S, R, X, a);
+        count_begin(ctx, a, tile_rep.get(), tile.get(), cnt8.get());
+        i64 hc[3] = {0, 0, 0};  // attempted writes, end of the expansions counted, entries resolved
+        auto totals = [&] {
+            i64 lines[kCountedLines * 16];
+            ctx.read(cnt.get(), lines, kCountedLines * 16);
+            hc[0] = hc[1] = hc[2] = 0;
+            for (int k = 0; k < kCountedLines; ++k) {
+                hc[0] += lines[k * 16];
+                hc[1] = std::max(hc[1], lines[k * 16 + 1]);
+                hc[2] += lines[k * 16 + 2];
             }
-            prof::Scope ps(ctx, S == 4 ? "cycles4_count" : "cycles5_count", 4.0 * wy + 8.0 * wx, wx, wy);
-            count_blocks<S>(ctx, a, n, reps, cnt8.get(), tile.get());
-            done += n;
-            if (!early || done >= nblk) break;
-            {
-                i64 lines[kCountedLines * 16];
-                ctx.read(cnt.get(), lines, kCountedLines * 16);
-                hc[0] = 0;
-                hc[1] = 0;
-                for (int k = 0; k < kCountedLines; ++k) {
-                    hc[0] += lines[k * 16];
-                    hc[1] = std::max(hc[1], lines[k * 16 + 1]);
-                }
-            }
-            if (hc[0] >= need) break;
-            // next chunk: cycle_chunk_pct percent (default 125) of the
-            // blocks that the rate so far says reach the budget (all the
-            // rest when it says they will not)
-            const double per_block = (double)hc[0] / (double)done;
+        };
+        // the chunk after `done` of n blocks: cycle_chunk_pct percent (default
+        // 125) of the blocks that the rate so far says reach the budget (all
+        // the rest when it says they will not)
+        auto next_chunk = [&](unsigned done, unsigned n, double per_block) {
             const double grow = 0.01 * (double)tune::get(tune::CycleChunkPct, X);
-            const double want = per_block > 0.0 ? grow * (double)(need - hc[0]) / per_block + 64.0 : 1e30;
-            chunk = want >= (double)(nblk - done) ? nblk - done : (unsigned)want;
+            const double want = early && per_block > 0.0 ? grow * (double)(need - hc[0]) / per_block + 64.0 : 1e30;
+            return want >= (double)(n - done) ? n - done : (unsigned)want;
+        };
+        i64 rdone = 0;
+        bool stopped = false;
+        if (sets) {
+            const int reps = count_reps(R);
+            const unsigned nblk = (unsigned)((R + reps - 1) / reps);
+            // the first chunk: a sixteenth of the blocks (a count that runs to
+            // the end pays this launch's tail once; smaller first chunks cost D
+            // mode on the 2D grid 5 ms, larger ones overshoot budgets), less
+            // where the count may go on past many mids per rep edge
+            unsigned done = 0, chunk = few ? std::max<unsigned>(nblk / 16, 256u) : std::max<unsigned>(nblk / 64, 32u);
+            if (forced == 1 && !early) chunk = nblk;
+            while (done < nblk) {
+                const unsigned n = std::min(chunk, nblk - done);
+                a.blk0 = done;
+                if (work_on)
+                    count_work<S>(ctx, G, rv1, rv2, nsum.get(), rdone, std::min<i64>((i64)(done + n) * reps, R), wx, wy);
+                {
+                    prof::Scope ps(ctx, S == 4 ? "cycles4_count" : "cycles5_count", 4.0 * wy + 8.0 * wx, wx, wy);
+                    count_blocks<S>(ctx, a, n, reps, cnt8.get(), tile.get());
+                }
+                done += n;
+                rdone = std::min<i64>((i64)done * reps, R);
+                if (done >= nblk) break;
+                totals();
+                stopped = early && hc[0] >= need;
+                if (stopped) break;
+                if (!forced && hc[2] >= (lengthy ? kDenseLong : kDenseShare<S>) * hc[1]) break;
+                chunk = next_chunk(done, nblk, (double)hc[0] / (double)done);
+            }
         }
-        if (done < nblk) {
+        queue.reset();
+        const i64 by_sets = rdone;
+        if (rdone < R && !stopped) {
+            CountLists<S> lists(ctx, a, rdone, G.n);
+            const i64 w0 = hc[0];
+            unsigned done = 0, chunk = early ? std::max<unsigned>(lists.nblk / 16, 256u) : lists.nblk;
+            while (done < lists.nblk) {
+                const unsigned n = std::min(chunk, lists.nblk - done);
+                if (work_on && done == 0) count_work<S>(ctx, G, rv1, rv2, nsum.get(), rdone, R, wx, wy);
+                {
+                    // profiling: the first chunk is booked with the work of all
+                    prof::Scope ps(ctx, S == 4 ? "cycles4_count" : "cycles5_count", 4.0 * wy + 8.0 * wx, wx, wy);
+                    lists.run(ctx, done, n, cnt8.get(), tile.get());
+                }
+                wx = wy = 0.0;
+                done += n;
+                if (done >= lists.nblk) break;
+                totals();
+                stopped = hc[0] >= need;
+                if (stopped) break;
+                chunk = next_chunk(done, lists.nblk, (double)(hc[0] - w0) / (double)done);
+            }
+        }
+        if (std::getenv("RAMA_CYCLE_STATS")) {
+            totals();
+            std::fprintf(stderr, "%d-cycle count: %lld rep edges (%lld by sets), %lld expansions, %lld counted, %lld mids, "
+                         "%lld entries resolved\n",
+                         S, (long long)R, (long long)by_sets, (long long)X, (long long)hc[1],
+                         (long long)(hc[0] / (S - 2)), (long long)hc[2]);
+        }
+        if (stopped) {
             // counted expansions [0, hc[1]): emit the tiles they touch; the
             // rest of the last tile contributes nothing
             tiles_used = (hc[1] + kCycTile - 1) / kCycTile;
@@ -1643,8 +2299,16 @@ void run_stage_packed(Ctx& ctx, const Csr& G, const int* rv1, const int* rv2, i6
     a.slot_out = d_out;
     DBuf<unsigned char> cnt8 = ctx.buf<unsigned char>((X + 15) / 16 * 16);  // cleared and counted up in whole words
     DBuf<i64> tile = ctx.buf<i64>(ntiles + 1);
+    if (S > 3 && std::getenv("RAMA_CYCLE_STATS"))
+        std::fprintf(stderr, "%d-cycle count of a pack: %lld rep edges (%lld by sets), %lld expansions\n", S, (long long)R,
+                     (long long)(count_form_forced() == 1 ? R : 0), (long long)X);
     if constexpr (S == 3) {
         launch_count3(ctx, a, (unsigned)ntiles, cnt8.get(), tile.get());
+    } else if (count_form_forced() != 1) {
+        // a pack's counts run to the end, past any number of mids
+        count_begin(ctx, a, tile_rep.get(), tile.get(), nullptr);
+        CountLists<S> lists(ctx, a, 0, G.n);
+        lists.run(ctx, 0, lists.nblk, cnt8.get(), tile.get());
     } else {
         const int reps = count_reps(R);
         CountQueue queue(ctx, S, R, X, a);

@@ -592,8 +592,7 @@ struct Handoff {
 // its initial dual on arrival), and every call of round() advances all
 // admitted instances by one contraction round.  Instances leave when they
 // finish; those that switch to the forest contraction, and those whose rounds
-// the single-instance solver runs without read-backs (kLeaveEdges), are
-// continued by `workers` threads with the single-instance rounds.
+// the single-instance solver runs in one launch (kLeavePack), are continued by `workers` threads with the single-instance rounds.
 class Lockstep {
    public:
     Lockstep(Ctx& ctx, const Options& o, int workers, LockstepSink& sink) : ctx_(ctx), o_(o), sink_(sink) {
@@ -604,15 +603,20 @@ class Lockstep {
     ~Lockstep() { finish(); }
 
     static constexpr int kMaxSlots = kLockstepMaxSlots;
-    // An instance of at most kLeaveEdges edges whose cycle searches find nothing
-    // any more leaves a pack of at most kLeavePack edges: its remaining rounds
-    // take a worker one launch (small_rounds), where the pack's rounds cost
-    // 0.4 ms however few instances are left (48 instances of up to 60k nodes:
-    // 49.8 -> 43.0 ms; a burst of 24 requests 45.6 -> 38.2).  In a larger pack
-    // the rounds are bound by their bytes and the small instances ride along
-    // (512 instances, 57.6M edges: 1% slower if they leave).
-    static constexpr i64 kLeaveEdges = kSmallMaxEdges;
+    // An instance that small_rounds takes and whose cycle searches find nothing
+    // any more leaves a pack of at most kLeavePack edges and kLeaveSlots slots
+    // per worker: its remaining rounds take a worker one launch, where the
+    // pack's rounds cost 0.4 ms however few instances are left (48 instances of
+    // up to 60k nodes: 49.8 -> 43.0 ms; a burst of 24 requests 45.6 -> 38.2).  In a
+    // larger pack the rounds are bound by their bytes and the small instances
+    // ride along (512 instances, 57.6M edges: 1% slower if they leave).  Of many
+    // slots that leave together each waits for a worker, about 0.3 ms an
+    // instance (512 instances of 2500 edges, P, 8 workers: 17 ms in the pack, 57 if
+    // they leave).  Cycles of 4 and 5 often turn up again once a few pairs are
+    // contracted, and then the worker's rounds are launches too (64 instances of
+    // 7000 edges, PD+, 8 workers: 39 ms in the pack, 50 if they leave; 16: 30 and 29).
     static constexpr i64 kLeavePack = (i64)1 << 22;
+    static constexpr int kLeaveSlots = 8, kLeaveSlotsLong = 2;
     int slots() const { return P_.Q(); }
     bool empty() const { return P_.Q() == 0; }
 
@@ -1211,7 +1215,8 @@ void Lockstep::round() {
     std::vector<int> done, hand;
     std::vector<char> keep((size_t)Qc, 1), mm;
     const bool duals = o_.max_cycle_length_primal >= 3 && o_.num_dual_itr_primal != 0;
-    const bool leave = nnz <= kLeavePack;
+    const int per_worker = duals && o_.max_cycle_length_primal > 3 ? kLeaveSlotsLong : kLeaveSlots;
+    const bool leave = nnz <= kLeavePack && Qc <= per_worker * (int)pool_.size();
     for (int c = 0; c < Qc; ++c) {
         if (hst[c].bad) {
             sink_.done(P_.s[c].id, RAMA_ERR_BAD_CONTRACTION, "Found bad contractions", nullptr, 0, P_.s[c].lb);
@@ -1219,7 +1224,9 @@ void Lockstep::round() {
         } else if (P_.s[c].nnz == 0) {
             done.push_back(c);  // A.nnz == 0 ends the rounds
             keep[c] = 0;
-        } else if (swc[c] || (leave && P_.s[c].nnz <= kLeaveEdges && (!duals || P_.s[c].quiet))) {
+        } else if (swc[c] || (leave && (!duals || P_.s[c].quiet) &&
+                              small_rounds_fit(P_.s[c].nnz, std::max(P_.s[c].rows, P_.s[c].cols), P_.s[c].max_node,
+                                               o_))) {
             hand.push_back(c);
             mm.push_back(swc[c] ? 0 : 1);
             keep[c] = 0;

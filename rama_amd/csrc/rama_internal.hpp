@@ -215,8 +215,9 @@ struct SmallState {
     int iter;  // the driver's round number after the rounds done
     int nnz, rows, cols, max_node;
 };
-// Whether A (the result of a contraction: no repeated pair, no self-loop)
-// can go to small_rounds under these options.
+// Whether a graph of these sizes (the result of a contraction: no repeated pair,
+// no self-loop) can go to small_rounds under these options.
+bool small_rounds_fit(i64 nnz, int max_dim, int max_node, const Options& o);
 bool small_rounds_fit(const DCoo& A, const Options& o);
 // Runs rounds from number `iter` on while matching picks the contractions and
 // no round's cycle search finds anything; A becomes the graph they leave and

@@ -623,15 +623,16 @@ __global__ __launch_bounds__(kSmThreads) void k_small_rounds(SmArgs a) {
     }
 }
 
-bool small_rounds_fit(const DCoo& A, const Options& o) {
-    const int n = A.max_node + 1;
-    if (A.nnz > kSmallMaxEdges || A.max_dim() > kSmallMaxNodes || n < 2) return false;
-    if (tune::get(tune::SmallRounds, A.nnz) == 0) return false;
+bool small_rounds_fit(i64 nnz, int max_dim, int max_node, const Options& o) {
+    const int n = max_node + 1;
+    if (nnz > kSmallMaxEdges || max_dim > kSmallMaxNodes || n < 2) return false;
+    if (tune::get(tune::SmallRounds, nnz) == 0) return false;
     const int len = o.num_dual_itr_primal == 0 ? 0 : o.max_cycle_length_primal;
     // cycles of 4 and 5 are looked for in a bit matrix
     if (len > 5 || (len > 3 && n * ((n + 31) / 32) > kSmallBitWords)) return false;
     return true;
 }
+bool small_rounds_fit(const DCoo& A, const Options& o) { return small_rounds_fit(A.nnz, A.max_dim(), A.max_node, o); }
 
 SmallState small_rounds(Ctx& ctx, DCoo& A, const Options& o, int iter, int* labels, i64 num_labels) {
     const int n0 = A.max_node + 1;

@@ -217,6 +217,17 @@ __device__ __forceinline__ bool mid_has(const int* __restrict__ p, int n, int x)
     return lo < n && p[lo] == x;
 }
 
+// Lanes of kLanes that share one of nu x nv pairs: eight where the pairs are
+// few, one where they fill the lanes.  Counts past kLanes are all the same here,
+// so they are cut before they are multiplied.
+constexpr __host__ __device__ int mid_pair_lanes(int nu, int nv, int lanes) {
+    const int pairs = (nu < lanes ? nu : lanes) * (nv < lanes ? nv : lanes);
+    return pairs * 2 > lanes ? 1 : (pairs * 4 > lanes ? 2 : (pairs * 8 > lanes ? 4 : 8));
+}
+static_assert(mid_pair_lanes(1, 1, 8) == 8 && mid_pair_lanes(2, 1, 64) == 8 && mid_pair_lanes(3, 3, 64) == 4 &&
+              mid_pair_lanes(5, 6, 64) == 2 && mid_pair_lanes(33, 1, 64) == 1, "shares of a pair");
+static_assert(mid_pair_lanes(kMidMaxNodes, kMidMaxNodes, 64) == 1, "two hubs (no overflow in a constant)");
+
 // Is there an attractive path of at most len - 1 edges between u and v, whose
 // lists of neighbours to pass through have nu and nv entries?  kLanes lanes
 // take the pairs of neighbours (x, y), one each or, of few pairs, a part of
@@ -226,7 +237,7 @@ __device__ __forceinline__ bool mid_joined(const MidArgs& a, const int* num, int
     const int* off = a.g.off;
     const int* pu = a.pos + off[u];
     const int* pv = a.pos + off[v];
-    const int pairs = nu * nv, lanes = pairs * 2 > kLanes ? 1 : (pairs * 4 > kLanes ? 2 : (pairs * 8 > kLanes ? 4 : 8));
+    const int lanes = mid_pair_lanes(nu, nv, kLanes);
     const int p0 = sub / lanes, step = kLanes / lanes, k0 = sub % lanes;
     int x = p0 / nv, y = p0 % nv;
     const int dx = step / nv, dy = step % nv;

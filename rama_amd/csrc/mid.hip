@@ -8,7 +8,8 @@
 // more where matchings are long) whose sizes are read on the device: the host queues several rounds over buffers sized by the graph it
 // last saw, then reads one small state.  A round that the driver has to
 // handle itself (a conflicted cycle, a matching of more than six rounds, a
-// bucket too large for LDS, the switch to the spanning forest) raises an
+// bucket too large for LDS, hubs whose cycle test takes too long, the switch to
+// the spanning forest) raises an
 // outcome word of the state, and the launches queued behind it leave at once.
 // So does the first matching of more than three rounds: from it on six are
 // queued.
@@ -64,6 +65,7 @@ constexpr int kMidPicks = 6;          // matching rounds queued per contraction 
 constexpr int kMidFewPicks = 3;       // and at first
 constexpr int kMidVertBlocks = kMidMaxNodes / kBlock;
 constexpr int kMidGrid = 1024;        // grid bound of the strided launches
+constexpr int kMidFound = 1, kMidTooMuch = 2;  // MidState::found
 
 struct MidGraph {
     int* row;    // forward edges, (row, col) order
@@ -228,12 +230,23 @@ static_assert(mid_pair_lanes(1, 1, 8) == 8 && mid_pair_lanes(2, 1, 64) == 8 && m
               mid_pair_lanes(5, 6, 64) == 2 && mid_pair_lanes(33, 1, 64) == 1, "shares of a pair");
 static_assert(mid_pair_lanes(kMidMaxNodes, kMidMaxNodes, 64) == 1, "two hubs (no overflow in a constant)");
 
+// What a lane of the cycle test may load one after another.  In the rounds it is
+// made for a lane loads some ten to fifty words; hubs joined by a repulsive edge
+// can ask for 10^8 pairs of one wave, and a queued round would take seconds.  A
+// lane that runs out hands the round to the driver, whose search spreads such
+// edges over the chip.  2048 loads are about 0.8 ms, a searched round's time.
+constexpr int kMidWork = 2048;
+// Loads of a search in n ascending entries.
+__device__ __forceinline__ int mid_search_loads(int n) { return 34 - __clz(n | 1); }
+
 // Is there an attractive path of at most len - 1 edges between u and v, whose
 // lists of neighbours to pass through have nu and nv entries?  kLanes lanes
 // take the pairs of neighbours (x, y), one each or, of few pairs, a part of
-// their lists, and ask for x = y, x next to y, a common neighbour.
+// their lists, and ask for x = y, x next to y, a common neighbour.  left: the
+// loads that the lane still has; below zero it gave up.
 template <int kLanes>
-__device__ __forceinline__ bool mid_joined(const MidArgs& a, const int* num, int u, int v, int nu, int nv, int sub) {
+__device__ __forceinline__ bool mid_joined(const MidArgs& a, const int* num, int u, int v, int nu, int nv, int sub,
+                                           int& left) {
     const int* off = a.g.off;
     const int* pu = a.pos + off[u];
     const int* pv = a.pos + off[v];
@@ -256,18 +269,36 @@ __device__ __forceinline__ bool mid_joined(const MidArgs& a, const int* num, int
             ny = k;
             z = vx;
         }
+        const int each = a.len > 4 ? 1 + mid_search_loads(ny) : 1;
+        left -= 4;
         bool hit = vx == vy;
-        for (int k = k0; k < nx; k += lanes) {
+        for (int k = k0; k < nx && left >= 0; k += lanes) {
             const int q = px[k];
             hit |= q == z || (a.len > 4 && mid_has(py, ny, q));
+            left -= each;
         }
         if (hit) return true;
+        if (left < 0) return false;
         x += dx;
         y += dy;
         if (y >= nv) {
             y -= nv;
             ++x;
         }
+    }
+    return false;
+}
+
+// The same for paths of two edges: the shorter list's entries, one per lane, in
+// the longer list.
+template <int kLanes>
+__device__ __forceinline__ bool mid_common(const MidArgs& a, int u, int v, int nu, int nv, int sub, int& left) {
+    const int* ps = a.pos + a.g.off[nu < nv ? u : v];
+    const int* pl = a.pos + a.g.off[nu < nv ? v : u];
+    const int ns = min(nu, nv), nl = max(nu, nv), each = 1 + mid_search_loads(nl);
+    for (int k = sub; k < ns && left >= 0; k += kLanes) {
+        if (mid_has(pl, nl, ps[k])) return true;
+        left -= each;
     }
     return false;
 }
@@ -284,13 +315,13 @@ __device__ __forceinline__ bool mid_joined(const MidArgs& a, const int* num, int
 __global__ __launch_bounds__(kBlock) void k_mid_cycles(MidArgs a) {
     MidState* st = a.st;
     if (st->stop) return;
-    constexpr int kMany = 4 * kMidGroup;  // pairs
+    constexpr int kMany = 4 * kMidGroup;  // pairs, or entries of the shorter list
     const int nf = st->nf, lane = lane_id(), sub = lane % kMidGroup;
     const float t = st->minw * a.tol;
-    const int* off = a.g.off;
     const int* num = a.len > 3 ? a.npath : a.npos;  // of the lists to walk
     const int stride = (int)gridDim.x * (kBlock / kMidGroup);
     bool hit = false;
+    int left = kMidWork;
     for (int e0 = ((int)xcd_block() * kWaves + (threadIdx.x >> 6)) * (64 / kMidGroup); e0 < nf; e0 += stride) {
         const int e = e0 + lane / kMidGroup;
         int u = 0, v = 0, nu = 0, nv = 0;
@@ -304,23 +335,20 @@ __global__ __launch_bounds__(kBlock) void k_mid_cycles(MidArgs a) {
             }
         }
         const bool on = nu > 0 && nv > 0;
-        const bool many = on && a.len > 3 && (float)nu * (float)nv > (float)kMany;
-        if (on && a.len == 3) {
-            // the shorter list's entries in the longer list
-            const int* ps = a.pos + off[nu < nv ? u : v];
-            const int* pl = a.pos + off[nu < nv ? v : u];
-            for (int k = sub; k < min(nu, nv); k += kMidGroup) hit |= mid_has(pl, max(nu, nv), ps[k]);
-        } else if (on && !many) {
-            hit = mid_joined<kMidGroup>(a, num, u, v, nu, nv, sub);
-        }
-        for (unsigned long long rest = __ballot(many && sub == 0); rest && !__any(hit); rest &= rest - 1ull) {
+        const bool many = on && (a.len == 3 ? min(nu, nv) > kMany : (float)nu * (float)nv > (float)kMany);
+        if (on && !many)
+            hit = a.len == 3 ? mid_common<kMidGroup>(a, u, v, nu, nv, sub, left)
+                             : mid_joined<kMidGroup>(a, num, u, v, nu, nv, sub, left);
+        for (unsigned long long rest = __ballot(many && sub == 0); rest && !__any(hit || left < 0); rest &= rest - 1ull) {
             const int src = __ffsll(rest) - 1;
-            hit = mid_joined<64>(a, num, __shfl(u, src, 64), __shfl(v, src, 64), __shfl(nu, src, 64),
-                                 __shfl(nv, src, 64), lane);
+            const int su = __shfl(u, src, 64), sv = __shfl(v, src, 64), mu = __shfl(nu, src, 64), mv = __shfl(nv, src, 64);
+            hit = a.len == 3 ? mid_common<64>(a, su, sv, mu, mv, lane, left)
+                             : mid_joined<64>(a, num, su, sv, mu, mv, lane, left);
         }
-        if (__any(hit) || __hip_atomic_load(&st->found, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) break;
+        if (__any(hit || left < 0) || __hip_atomic_load(&st->found, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) break;
     }
-    if (__any(hit) && lane == 0) __hip_atomic_store(&st->found, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int found = __any(hit) ? kMidFound : (__any(left < 0) ? kMidTooMuch : 0);
+    if (found && lane == 0) __hip_atomic_fetch_or(&st->found, found, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Matching round t's best neighbours (k_pick_best's choice: strongest
@@ -459,7 +487,7 @@ __global__ __launch_bounds__(kMidThreads) void k_mid_keys(MidArgs a) {
     const int n = st->n, nf = st->nf, nblk = (n + kBlock - 1) / kBlock, found = st->found;
     if (st->stop) return;
     if (found) {
-        if (blockIdx.x == 0 && tid == 0) st->ended = kSmallCycles;
+        if (blockIdx.x == 0 && tid == 0) st->ended = found & kMidFound ? kSmallCycles : kMidSkew;
         return;
     }
     // the edges' ends and what the counts need are loaded together: a chain

@@ -231,7 +231,7 @@ constexpr int kMidMaxEdges = 1 << 18;
 constexpr int kMidMaxNodes = 1 << 18;
 enum MidReason : int {  // besides SmallReason's; 0: rounds still go on
     kMidMatching = 5,   // this round's matching takes more rounds than are queued
-    kMidSkew = 6,       // a row bucket of the contraction does not fit in LDS
+    kMidSkew = 6,       // a row bucket of the contraction does not fit in LDS, or hubs make the cycle test too long
     kMidSmall = 7,      // small enough for small_rounds
 };
 struct MidState {

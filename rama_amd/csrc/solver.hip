@@ -111,7 +111,7 @@ void solve_rounds(Ctx& ctx, DCoo& A, SolveResult& out, const Options& o, int sta
                 reason = ms.stop;
                 next = ms.iter;
                 mid_first = next > iter ? 4 : 1;
-                // a row too long for its bucket: wait until the graph is half as large
+                // hubs too large for it: wait until the graph is half as large
                 if (reason == kMidSkew) mid_max = ms.nf / 2;
             }
             st.end(ctx, small ? "small_rounds" : "mid_rounds");

@@ -21,9 +21,9 @@ def _kernels():
 
 
 def _words(body):
-    stores = set(re.findall(r"\bst->(\w+)\s*=(?!=)", body)) | set(re.findall(r"_store\(&st->(\w+)", body))
+    stores = set(re.findall(r"\bst->(\w+)\s*=(?!=)", body)) | set(re.findall(r"_(?:store|fetch_or)\(&st->(\w+)", body))
     rest = re.sub(r"\bst->\w+\s*=(?!=)", "", body)
-    rest = re.sub(r"_store\(&st->\w+", "", rest)
+    rest = re.sub(r"_(?:store|fetch_or)\(&st->\w+", "", rest)
     return set(re.findall(r"\bst->(\w+)", rest)), stores
 
 

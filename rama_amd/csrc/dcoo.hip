@@ -720,7 +720,7 @@ void compress_matching(Ctx& ctx, const int* map, i64 n, int* out) {
 // Local ids are global - nbase[q].  Fields as the single-instance dCOO keeps
 // them: cols = max col + 1, rows = last row + 1, max_node = largest kept col.
 void slot_stats_clear(Ctx& ctx, SlotStats* st, int Q) {
-    for_each(ctx, Q, [=] __device__(i64 q) { st[q] = SlotStats{-1, -1, -1, 0, 0}; });
+    for_each(ctx, Q, [=] __device__(i64 q) { st[q] = SlotStats{-1, -1, -1, 0, 0, 0}; });
 }
 
 // rb[q] = first position of slot q in a sorted key array (q = 0..Q), the
@@ -771,7 +771,7 @@ struct ContractAcc {
     int mc = -1;    // largest col, diagonal included
     int mk = -1;    // largest col of a kept segment
     int kept = 0;   // kept segments
-    int bad = 0;    // negative self-loop
+    int bad = 0;    // bit 0: negative self-loop, bit 1: a kept cost that is not a number
 };
 struct ContractRed {
     __device__ ContractAcc operator()(ContractAcc a, ContractAcc b) const {
@@ -855,8 +855,9 @@ void contract_packed(Ctx& ctx, const DCoo& A, const int* node_map, int max_label
                 if (kp) {
                     a.mk = gc > a.mk ? gc : a.mk;
                     a.kept += 1;
+                    if (OV[s] != OV[s]) a.bad |= 2;
                 } else if (OV[s] < 0.0f) {
-                    a.bad = 1;
+                    a.bad |= 1;
                 }
             },
             ContractRed(),
@@ -864,7 +865,8 @@ void contract_packed(Ctx& ctx, const DCoo& A, const int* node_map, int max_label
                 atomicMax(&st[q].max_col, r.mc - NB[q]);
                 if (r.mk >= 0) atomicMax(&st[q].max_kept_col, r.mk - NB[q]);
                 atomicAdd(&st[q].kept, r.kept);
-                if (r.bad) st[q].bad = 1;
+                if (r.bad & 1) st[q].bad = 1;
+                if (r.bad & 2) st[q].nan = 1;
             });
         for_each(ctx, Q, [=] __device__(i64 q) {
             const i64 lo = RB[q], hi = RB[q + 1];

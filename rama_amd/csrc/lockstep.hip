@@ -603,13 +603,14 @@ class Lockstep {
     ~Lockstep() { finish(); }
 
     static constexpr int kMaxSlots = kLockstepMaxSlots;
-    // An instance that small_rounds takes and whose cycle searches find nothing
-    // any more leaves a pack of at most kLeavePack edges and kLeaveSlots slots
-    // per worker: its remaining rounds take a worker one launch, where the
-    // pack's rounds cost 0.4 ms however few instances are left (48 instances of
-    // up to 60k nodes: 49.8 -> 43.0 ms; a burst of 24 requests 45.6 -> 38.2).  In a
-    // larger pack the rounds are bound by their bytes and the small instances
-    // ride along (512 instances, 57.6M edges: 1% slower if they leave).  Of many
+    // An instance that small_rounds takes (no cost that is not a number, too: the
+    // single-instance launches pick otherwise from those) and whose cycle searches
+    // find nothing any more leaves a pack of at most kLeavePack edges and
+    // kLeaveSlots slots per worker: its remaining rounds take a worker one launch,
+    // where the pack's rounds cost 0.4 ms however few instances are left (48
+    // instances of up to 60k nodes: 49.8 -> 43.0 ms; a burst of 24 requests 45.6 ->
+    // 38.2).  In a larger pack the rounds are bound by their bytes and the small
+    // instances ride along (512 instances, 57.6M edges: 1% slower if they leave).  Of many
     // slots that leave together each waits for a worker, about 0.3 ms an
     // instance (512 instances of 2500 edges, P, 8 workers: 17 ms in the pack, 57 if
     // they leave).  Cycles of 4 and 5 often turn up again once a few pairs are
@@ -1224,7 +1225,7 @@ void Lockstep::round() {
         } else if (P_.s[c].nnz == 0) {
             done.push_back(c);  // A.nnz == 0 ends the rounds
             keep[c] = 0;
-        } else if (swc[c] || (leave && (!duals || P_.s[c].quiet) &&
+        } else if (swc[c] || (leave && (!duals || P_.s[c].quiet) && !hst[c].nan &&
                               small_rounds_fit(P_.s[c].nnz, std::max(P_.s[c].rows, P_.s[c].cols), P_.s[c].max_node,
                                                o_))) {
             hand.push_back(c);

@@ -29,7 +29,8 @@
 // No launch stores an outcome word that it tests itself: its blocks start at
 // different times, and the waves of a late one could read the word differently
 // and part before a barrier.  `stop` is stored by the finish of the round before
-// (all of this round's launches test it), `found` by the cycle test, `ended` by
+// (all of this round's launches test it), `found` by the cycle test, and by the
+// begin where a cost is not a number, `ended` by
 // the keys and `skewed` by the scatter (only the launches behind test them); the
 // finish folds them into the next state's `stop`.
 //
@@ -48,7 +49,8 @@
 // 31.8 -> 24.3; rounds of 7k to 2k edges of a 187x211 grid PD+ 1.85 -> 0.54.  Up
 // to 2^18 edges, the lists whose contraction leaves the symmetric CSR.
 //
-// Every sum and order is the stage-by-stage path's, so are the results.
+// Every sum and order is the stage-by-stage path's, so are the results.  (A round
+// with a cost that is not a number is the driver's.)
 #include "rama_internal.hpp"
 #include "tuning.hpp"
 
@@ -171,18 +173,23 @@ __device__ __forceinline__ void mid_compact(const MidArgs& a, int n, int* count,
 __global__ __launch_bounds__(kBlock) void k_mid_begin(MidArgs a) {
     __shared__ double ws[kWaves];
     __shared__ int wi[kWaves];
-    const MidState* st = a.st;
+    MidState* st = a.st;
     if (st->stop) return;
     const int nnz = 2 * st->nf, n = st->n;
     const int nb = min((nnz + kBlock - 1) / kBlock, (int)kReduceMaxBlocks);
     if ((int)blockIdx.x < nb) {  // uniform per block; the grid covers nb
         double s = 0.0;
         int c = 0;
+        bool nan = false;
         for (int i = blockIdx.x * kBlock + threadIdx.x; i < nnz; i += nb * kBlock) {
             const float x = a.g.w[i];
+            nan |= x != x;
             s += x >= 0.0f ? (double)x : 0.0;
             c += x >= 0.0f ? 1 : 0;
         }
+        // what the launches stage by stage pick from comparisons with a NaN hangs
+        // on their shape: the driver's round
+        if (nan) __hip_atomic_fetch_or(&st->found, kMidFound, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         const double r = block_reduce(s, OpSum(), ws);
         const int rc = block_reduce(c, OpSum(), wi);
         if (threadIdx.x == 0) {

@@ -94,6 +94,7 @@ struct SlotStats {
     int max_kept_col;  // largest local col of a kept edge, -1 if none
     int kept;          // kept edges
     int bad;           // a negative self-loop was contracted
+    int nan;           // the cost of a contraction's kept edge is not a number
 };
 void slot_stats_clear(Ctx& ctx, SlotStats* st, int Q);
 void slot_stats_edges(Ctx& ctx, const int* row, const int* col, i64 n, const int* nbase, int Q, SlotStats* st);
@@ -205,7 +206,8 @@ constexpr int kSmallMaxNodes = 4096;
 constexpr int kSmallBitWords = 20480;  // 32-bit words of the attractive adjacency's bit matrix
 enum SmallReason : int {
     kSmallMore = 0,    // the launch's rounds are used up
-    kSmallCycles = 1,  // the next round's cycle search finds something: its dual pass is due
+    kSmallCycles = 1,  // the next round is the driver's: its cycle search finds something and its dual pass is
+                       // due, or some cost is not a number
     kSmallDone = 2,    // nothing (left) to contract
     kSmallBad = 3,     // a negative self-loop was contracted
     kSmallForest = 4,  // the next round contracts by the spanning forest

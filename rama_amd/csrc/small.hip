@@ -22,7 +22,9 @@
 // Every decision follows the general path's arithmetic: the same thresholds
 // (matching.hip's sums in reduce_pair_to's order), the same stop rule, runs of
 // equal keys summed in double in input order.  So the rounds give the same
-// labels and costs, bit for bit, as the launches they replace.
+// labels and costs, bit for bit, as the launches they replace.  A round with a
+// cost that is not a number is left to the driver: what its launches pick from
+// such comparisons hangs on their shape.
 #include "rama_internal.hpp"
 #include "tuning.hpp"
 
@@ -78,6 +80,7 @@ struct SmShared {
     int found;     // conflicted cycle
     int st[4];     // contraction: largest row, col, kept col; negative self-loop
     int total;
+    int nan;
     int lastrow;
     float pos_sum, pos_cnt;
 };
@@ -93,7 +96,7 @@ struct SmArgs {
     int* label;   // out: label of each of the n0 nodes at entry
     int nf, n0, rows, cols;
     int iter;     // round number of the driver
-    int max_len, budget_on;  // primal cycle length (0: no dual pass)
+    int max_len;  // primal cycle length (0: no dual pass)
     float mult, ratio, tol;
     SmallState* out;
     SmallState* mirror;
@@ -193,24 +196,28 @@ __device__ __forceinline__ void sm_find_cycles(SmShared& s, int nf, int n, float
 
 // Sum and count of the non-negative costs of the nnz entries, added as
 // reduce_pair_to adds them: blocks of 256 consecutive entries, a wave tree,
-// the waves in order, then the blocks' partials by one more tree.
+// the waves in order, then the blocks' partials by one more tree.  s.nan: some
+// cost is not a number.
 __device__ __forceinline__ void sm_threshold(SmShared& s, int nnz) {
     const int lane = lane_id(), w = threadIdx.x >> 6;
     int cnt = 0;
+    bool nan = false;
     for (int vw = w; vw * 64 < nnz; vw += kSmWaves) {
         const int i = vw * 64 + lane;
         const float x = i < nnz ? s.g.w[i] : -1.0f;
+        nan |= x != x;
         double a = x >= 0.0f ? (double)x : 0.0;
         cnt += x >= 0.0f ? 1 : 0;
 #pragma unroll
         for (int d = 32; d >= 1; d >>= 1) a += shfl_down64(a, d);
         if (lane == 0) s.s.vws[vw] = a;
     }
-    if (threadIdx.x == 0) s.total = 0;
+    if (threadIdx.x == 0) s.total = s.nan = 0;
     __syncthreads();
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) cnt += __shfl_xor(cnt, d, 64);
     if (lane == 0) atomicAdd(&s.total, cnt);
+    if (nan) s.nan = 1;
     if (w == 0) {
         const int nvw = (nnz + 63) / 64, nb = (nnz + 255) / 256;
         double a = 0.0;
@@ -439,6 +446,10 @@ __global__ __launch_bounds__(kSmThreads) void k_small_rounds(SmArgs a) {
             }
         }
         sm_threshold(s, 2 * nf);
+        if (s.nan) {
+            reason = kSmallCycles;
+            break;
+        }
         const int matched = sm_matching(s, n, a.mult);
         if (matched == 0) {
             reason = kSmallDone;

@@ -241,7 +241,10 @@ static_assert(mid_pair_lanes(kMidMaxNodes, kMidMaxNodes, 64) == 1, "two hubs (no
 // made for a lane loads some ten to fifty words; hubs joined by a repulsive edge
 // can ask for 10^8 pairs of one wave, and a queued round would take seconds.  A
 // lane that runs out hands the round to the driver, whose search spreads such
-// edges over the chip.  2048 loads are about 0.8 ms, a searched round's time.
+// edges over the chip.  2048 loads are about 0.8 ms, a searched round's time:
+// 257x509 grid with long-range edges, PD+, 45.5 ms, 48 with 8192 loads, 61 without
+// a limit; 97x211 22.6, 24.7 and 34.9; grids without long-range edges and random
+// graphs the same.
 constexpr int kMidWork = 2048;
 // Loads of a search in n ascending entries.
 __device__ __forceinline__ int mid_search_loads(int n) { return 34 - __clz(n | 1); }
@@ -1180,6 +1183,7 @@ MidState mid_rounds(Ctx& ctx, DCoo& A, const Options& o, int iter, int first, in
         }
         if (h.stop) break;
     }
+    h.picks = a.picks;
     map_node_labels(ctx, lab.get(), n0, labels, num_labels);
     if (h.rounds & 1) {  // the graph ended up in the second set
         A.row = std::move(B.row);

@@ -246,6 +246,7 @@ struct MidState {
     int any, matched, kb;
     int rounds;  // done since entry
     float thr, minw;
+    int picks;   // host: matching rounds queued per round at the end
 };
 bool mid_rounds_fit(const DCoo& A, const Options& o);
 // As small_rounds; `first` rounds are queued before the first host wait.

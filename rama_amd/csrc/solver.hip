@@ -100,7 +100,7 @@ void solve_rounds(Ctx& ctx, DCoo& A, SolveResult& out, const Options& o, int sta
         // rounds' cycle searches still find something.
         if (use_mm && iter > 0 && (!duals || ctx.last_cycles_empty) && !observed) {
             const bool small = small_rounds_fit(A, o), mid = !small && A.nnz <= mid_max && mid_rounds_fit(A, o);
-            int reason = kSmallCycles, next = iter;
+            int reason = kSmallCycles, next = iter, picks = 0;
             st.begin(ctx);
             if (small) {
                 const SmallState ss = small_rounds(ctx, A, o, iter, out.labels.get(), N);
@@ -109,6 +109,7 @@ void solve_rounds(Ctx& ctx, DCoo& A, SolveResult& out, const Options& o, int sta
             } else if (mid) {
                 const MidState ms = mid_rounds(ctx, A, o, iter, mid_first, out.labels.get(), N);
                 reason = ms.stop;
+                picks = ms.picks;
                 next = ms.iter;
                 mid_first = next > iter ? 4 : 1;
                 // hubs too large for it: wait until the graph is half as large
@@ -116,8 +117,8 @@ void solve_rounds(Ctx& ctx, DCoo& A, SolveResult& out, const Options& o, int sta
             }
             st.end(ctx, small ? "small_rounds" : "mid_rounds");
             if (st.on && (small || mid))
-                std::fprintf(stderr, "rounds %d..%d: %lld edges, %s, reason %d, %.3f ms\n", iter, next - 1,
-                             (long long)e0, small ? "small" : "mid", reason,
+                std::fprintf(stderr, "rounds %d..%d: %lld edges, %s, reason %d, picks %d, %.3f ms\n", iter, next - 1,
+                             (long long)e0, small ? "small" : "mid", reason, picks,
                              std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - r0).count());
             if (reason == kSmallBad) throw Error(RAMA_ERR_BAD_CONTRACTION, "Found bad contractions");
             if (next > iter) out.iterations = next;

@@ -66,6 +66,9 @@ struct CycArgs {
 // path gives the same counts and triangles):
 //   RAMA_COUNT_FORM=sets | lists   the 4- and 5-cycle counts' form, instead of
 //                         the choice by what ends the count
+//   RAMA_COUNT_QUEUE=none | queue | list   the sets form without queue and list
+//                         of hubs, without the list, without the queue, as where
+//                         memory is short
 //   RAMA_CYCLE_TABLES=0   the same counts without their sets and tables: every
 //                         list entry resolved against the lists (sets form),
 //                         every expansion counted by its thread (lists form)
@@ -82,6 +85,10 @@ static int count_form_forced() {  // 0: choose, 1: sets, 2: lists
     if (std::strcmp(e, "sets") == 0) return 1;
     if (std::strcmp(e, "lists") == 0) return 2;
     return 0;
+}
+static bool count_queue_part(const char* part) {
+    const char* e = std::getenv("RAMA_COUNT_QUEUE");
+    return !e || e[0] == 0 || std::strcmp(e, part) == 0;
 }
 static int emit_form_forced() {  // 0: choose, 1: dense, 2: queue
     const char* e = std::getenv("RAMA_EMIT_FORM");
@@ -1996,10 +2003,10 @@ struct CountQueue {
     CountQueue(Ctx& ctx, int S, i64 R, i64 X, CycArgs& a) {
         count = ctx.buf<unsigned>((kQueueParts + 1) * 32);
         a.qcount = count.get();
-        wide = try_buf<int2>(ctx, R);
+        if (count_queue_part("list")) wide = try_buf<int2>(ctx, R);
         a.wide = wide.get();
         a.qcap = (int)std::min<i64>(X / (S == 4 ? 16 : 64) / kQueueParts + 1024, (i64)1 << 24);
-        entries = try_buf<int3>(ctx, (i64)kQueueParts * a.qcap);
+        if (count_queue_part("queue")) entries = try_buf<int3>(ctx, (i64)kQueueParts * a.qcap);
         a.queue = entries.get();
         if (!a.queue) a.qcap = 0;
     }

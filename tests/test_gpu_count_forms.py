@@ -49,6 +49,24 @@ def test_forms_equal_oracle(gpu, oracle, monkeypatch, name):
                     assert np.array_equal(x, y), (max_len, factor, form)
 
 
+@pytest.mark.parametrize("part", ["none", "queue", "list"])
+@pytest.mark.parametrize("name", ["ring_dup", "ring_wide", "hubs"])
+def test_sets_without_queue_or_list(gpu, oracle, monkeypatch, name, part):
+    """What the sets form does where memory for its queue or its list of hubs is
+    short: entries resolved as they come, hubs' rep edges unfiltered."""
+    i, j, c = _graph(name)
+    r, co, v, (rows, cols) = oracle.dcoo_init(i, j, c)
+    monkeypatch.setenv("RAMA_COUNT_FORM", "sets")
+    monkeypatch.setenv("RAMA_COUNT_QUEUE", part)
+    for max_len in (4, 5):
+        for factor in (0.5, 30.0):
+            o = oracle.conflicted_cycles(r, co, v, rows, cols, max_len, factor)
+            g = gpu.conflicted_cycles(r, co, v, rows, cols, max_len, factor)
+            assert g[3] == o[3], (max_len, factor)
+            for x, y in zip(g[:3], o[:3]):
+                assert np.array_equal(x, y), (max_len, factor)
+
+
 def _counts(capfd, length):
     err = capfd.readouterr().err
     return [(int(a), int(b)) for a, b in re.findall(r"%d-cycle count[^:]*: (\d+) rep edges \((\d+) by sets\)" % length, err)]

@@ -5,14 +5,13 @@
 // 4 host waits, about 0.25 ms whatever its size, most of it launch gaps and
 // 2 us kernels; with searches for cycles of up to five nodes 48 to 59 launches
 // and 18 waits, 0.45 to 0.6 ms.  Here a round is nine to eleven launches (three
-// more where matchings are long) whose sizes are read on the device: the host queues several rounds over buffers sized by the graph it
-// last saw, then reads one small state.  A round that the driver has to
-// handle itself (a conflicted cycle, a matching of more than six rounds, a
-// bucket too large for LDS, hubs whose cycle test takes too long, the switch to
-// the spanning forest) raises an
-// outcome word of the state, and the launches queued behind it leave at once.
-// So does the first matching of more than three rounds: from it on six are
-// queued.
+// more where matchings are long) whose sizes are read on the device: the host
+// queues several rounds over buffers sized by the graph it last saw, then reads one
+// small state.  A round that the driver has to handle itself (a conflicted cycle, a
+// matching of more than six rounds, a bucket too large for LDS, hubs whose cycle
+// test takes too long, the switch to the spanning forest) raises an outcome word of
+// the state, and the launches queued behind it leave at once.  So does the first
+// matching of more than three rounds: from it on six are queued.
 //
 //   k_mid_begin    sums of the matching threshold, attractive neighbour lists
 //   k_mid_prune    (cycles of 4 and 5) the lists without their leaves
@@ -30,9 +29,9 @@
 // different times, and the waves of a late one could read the word differently
 // and part before a barrier.  `stop` is stored by the finish of the round before
 // (all of this round's launches test it), `found` by the cycle test, and by the
-// begin where a cost is not a number, `ended` by
-// the keys and `skewed` by the scatter (only the launches behind test them); the
-// finish folds them into the next state's `stop`.
+// begin where a cost is not a number, `ended` by the keys and `skewed` by the
+// scatter (only the launches behind test them); the finish folds them into the next
+// state's `stop`.
 //
 // The matching needs no matched flags: a vertex v is matched once
 // best[best[v]] == v, since matched vertices keep their best.  So a matching
@@ -43,11 +42,11 @@
 // merged launches and the loads issued together.  Measured per round of
 // 20k to 200k edges: about 60 us on the device (picks 3 x 5.3, bucket 11,
 // keys 12, scatter 9, begin 7, finish 6, resolve and prune 4.6 each, cycles 4 to
-// 20, up to 90 where hubs are many) against 220 to 320 us stage by stage, 450 to
-// 600 with cycles of up to five nodes.  Solves: 1024x2048 grid with long-range
-// edges P 20.2 -> 15.6 ms, PD 55.2 -> 46.9; 257x509 PD 18.7 -> 14.3; 71^3 grid PD+
-// 31.8 -> 24.3; rounds of 7k to 2k edges of a 187x211 grid PD+ 1.85 -> 0.54.  Up
-// to 2^18 edges, the lists whose contraction leaves the symmetric CSR.
+// 20) against 220 to 320 us stage by stage, 450 to 600 with cycles of up to five
+// nodes.  Solves with and without this form (the other forms on): 1024x2048 grid
+// with long-range edges P 20.2 -> 15.6 ms, PD 55.2 -> 49.5; 257x509 PD 18.7 -> 15.2;
+// 71^3 grid PD+ 31.8 -> 24.3; rounds of 7k to 2k edges of a 187x211 grid PD+ 1.85 ->
+// 0.54.  Up to 2^18 edges, the lists whose contraction leaves the symmetric CSR.
 //
 // Every sum and order is the stage-by-stage path's, so are the results.  (A round
 // with a cost that is not a number is the driver's.)

@@ -211,7 +211,8 @@ __global__ __launch_bounds__(NT) void k_radix_scatter(const K* __restrict__ kin,
 // of equal key ranges leave most pairs of a graph's keys in a few of them: node
 // ids end below the next power of two, low ids hold the supernodes.  The
 // bucket sorts of a packed batch of 48 instances averaged 123 us with them, 23
-// with these; on uniform keys the sampling costs 3 to 8 us a sort.)
+// with these.  On uniform keys the samples, drawn by every block, cost a sort 4 us
+// at 40k pairs, 8 at 260k, 18 at 1M.)
 constexpr int kSplitBins = 4096;
 struct SplitMap {
     unsigned char bucket[kSplitBins];

@@ -24,7 +24,7 @@ enum Knob : int {
     SortPathU64 = 0,
     SortPathU32,
     // size = radix tiles; 1024 or 512 threads per 4096-pair tile in the
-    // scatter and onesweep passes
+    // scatter and onesweep passes (the bucket path's blocks have 1024)
     SortThreads,
     // size = items; blocks of the two-launch integer scan (64 .. 4096)
     ScanChunks,

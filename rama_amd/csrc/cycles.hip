@@ -1036,8 +1036,9 @@ __global__ __launch_bounds__(kBlock) void k_cycle_count5(CycArgs a, const i64* _
 // longest of its lanes' lists.  D mode on the 12.47M-edge grid, all 4- and 5-cycle
 // counts of a solve: 54.5 + 59.7 ms by lists, 14 + 36 with the sets (a full pass:
 // 9.3M rep edges and 100M expansions 5.0 -> 1.4 ms, 1.1G expansions 11 -> 8.2); the
-// 192^3 grid's PD+ 14.0 + 8.1 -> 11.0 + 7.7.  5-cycles are bound by the lists' load latency at 5 waves per SIMD
-// and by about 60 instructions per step of four lists.
+// 192^3 grid's PD+ 14.0 + 8.1 -> 11.0 + 7.7.  5-cycles are bound by the lists' load
+// latency (59% of the waves' time, 3.5 to 4 waves per SIMD) and by about 60
+// instructions per step of four lists.
 constexpr int kSetLanes = 16;                  // lanes per run
 constexpr int kSetGroups = kBlock / kSetLanes;
 constexpr int kSetWords = 64;                  // words of a group's set

@@ -31,7 +31,9 @@
 // (all of this round's launches test it), `found` by the cycle test, and by the
 // begin where a cost is not a number, `ended` by the keys and `skewed` by the
 // scatter (only the launches behind test them); the finish folds them into the next
-// state's `stop`.
+// state's `stop`.  They are loaded together, not one after another, and a state fills
+// a line of its own: every launch begins with them (1024x2048 grid P 15.3 ms otherwise,
+// 14.9 so).
 //
 // The matching needs no matched flags: a vertex v is matched once
 // best[best[v]] == v, since matched vertices keep their best.  So a matching
@@ -368,7 +370,7 @@ __global__ __launch_bounds__(kBlock) void k_mid_pick(MidArgs a, int t) {
     __shared__ double ws[kWaves];
     __shared__ int wi[kWaves];
     MidState* st = a.st;
-    if (st->stop || st->found) return;
+    if (st->stop | st->found) return;
     const int n = st->n;
     float thr;
     bool any;
@@ -433,7 +435,7 @@ __global__ __launch_bounds__(kBlock) void k_mid_pick(MidArgs a, int t) {
 __global__ __launch_bounds__(kBlock) void k_mid_resolve(MidArgs a) {
     __shared__ int wr[kMidPicks][kWaves], wm[kMidPicks][kWaves];
     const MidState* st = a.st;
-    if (st->stop || st->found) return;
+    if (st->stop | st->found) return;
     const int n = st->n;
     const int v = blockIdx.x * kBlock + threadIdx.x;
     if ((int)(blockIdx.x * kBlock) >= n) return;  // uniform per block
@@ -642,7 +644,7 @@ __global__ __launch_bounds__(kMidThreads) void k_mid_scatter(MidArgs a) {
     __shared__ int ws[kMidWaves];
     __shared__ int over;
     MidState* st = a.st;
-    if (st->stop || st->ended) return;
+    if (st->stop | st->ended) return;
     const int tid = threadIdx.x, lane = lane_id(), w = tid >> 6;
     const int nf = st->nf, kb = st->kb;
     const int ntiles = (nf + kMidTileEdges - 1) / kMidTileEdges;
@@ -767,7 +769,7 @@ __global__ __launch_bounds__(kMidThreads) void k_mid_bucket(MidArgs a) {
     __shared__ int ws[kMidWaves];
     __shared__ int agg[8];
     const MidState* st = a.st;
-    if (st->stop || st->ended || st->skewed) return;
+    if (st->stop | st->ended | st->skewed) return;
     const int tid = threadIdx.x, lane = lane_id(), w = tid >> 6, b = blockIdx.x;
     const int n = st->n, kb = st->kb;
     // labels of the nodes at entry, composed with this contraction
@@ -941,7 +943,7 @@ __global__ __launch_bounds__(kBlock) void k_mid_finish(MidArgs a) {
     __shared__ float wf[kWaves];
     const MidState* st = a.st;
     const int tid = threadIdx.x, b = blockIdx.x;
-    if (st->stop || st->ended || st->skewed) {
+    if (st->stop | st->ended | st->skewed) {
         if (b == 0 && tid == 0) {
             MidState x = *st;
             x.stop = x.stop ? x.stop : (x.ended ? x.ended : x.skewed);

@@ -236,13 +236,13 @@ enum MidReason : int {  // besides SmallReason's; 0: rounds still go on
     kMidSkew = 6,       // a row bucket of the contraction does not fit in LDS, or hubs make the cycle test too long
     kMidSmall = 7,      // small enough for small_rounds
 };
-struct MidState {
-    int stop;  // MidReason or SmallReason; set by the round before's finish
-    int iter;  // the driver's round number after the rounds done
-    int nf, n, rows, cols, max_node;
+struct alignas(128) MidState {  // a cache line: every launch begins by loading it
+    int stop;    // MidReason or SmallReason; set by the round before's finish
     int found;   // this round's outcomes, each stored by one launch and tested by those behind it
     int ended;
     int skewed;
+    int iter;  // the driver's round number after the rounds done
+    int nf, n, rows, cols, max_node;
     int any, matched, kb;
     int rounds;  // done since entry
     float thr, minw;
